@@ -115,7 +115,7 @@ def build_oracle() -> None:
     if shutil.which("make") is None:
         raise RuntimeError("make is required to build the oracle")
     _run(["make", "-s", "-C", str(ROOT / "oracle")])
-    if REFERENCE.is_dir():
+    if (REFERENCE / "include" / "maps.hpp").is_file():
         _run(["make", "-s", "-C", str(ROOT / "oracle"), "ref", f"REF={REFERENCE}"])
 
 
