@@ -36,6 +36,7 @@ SOURCES = [
     "amx_serve.cpp",
     "amx_gmsh.cpp",
     "amx_kernels.hip",
+    "amx_cong.hip",
     "amx_solver_kernels.hip",
     "amx_mrhs.hip",
     "amx_free.hip",

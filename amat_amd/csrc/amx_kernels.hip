@@ -17,6 +17,8 @@
 //                    reference's element order (node -> (element, row)
 //                    transposed lists), a block's list range staged in LDS,
 //                    with the BC rows fused.
+// Groups given as K_e = s_e K_ref run the kernels of amx_cong.hip instead (same
+// element rows, no stored matrices read).
 // The *_batched kernels run the same arithmetic for many operators (the jobs
 // of the solve server) in one launch.
 // Blocks are remapped so that each of the 8 XCDs walks a contiguous range of
@@ -1142,15 +1144,16 @@ __global__ void nsym_diag_kernel(const double* __restrict__ K, uint32_t N, uint6
 // stay in the null space of a Laplacian element); symmetric K stays symmetric.
 __global__ void bf16_diag_kernel(const double* __restrict__ src, const double* __restrict__ kref,
                                  const double* __restrict__ scale, const uint32_t* __restrict__ slot_elem,
-                                 uint32_t N, uint64_t n_rows, float* __restrict__ out)
+                                 uint32_t N, uint64_t n_rows, uint32_t rs, uint32_t ss, float* __restrict__ out)
 {
     const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;  // slot * N + r
     if (i >= n_rows) return;
     const uint64_t slot = i / N;
     const uint32_t r = (uint32_t)(i - slot * N);
     const uint32_t e = slot_elem[slot];
+    float& o = out[(uint64_t)r * rs + slot * ss];
     if (e == kPadSlot) {
-        out[i] = 0.0f;
+        o = 0.0f;
         return;
     }
     double d = 0.0;
@@ -1158,7 +1161,7 @@ __global__ void bf16_diag_kernel(const double* __restrict__ src, const double* _
         const double kv = src ? src[(uint64_t)e * N * N + (uint64_t)r * N + j] : scale[e] * kref[(uint64_t)r * N + j];
         d += (j == r) ? kv : kv - (double)bf16_to_f32(f64_to_bf16(kv));
     }
-    out[i] = (float)d;
+    o = (float)d;
 }
 
 __global__ void extract_diag_kernel(const double* __restrict__ K, TiledIndex ti, uint32_t sym_te, uint64_t n_rows,
@@ -1441,11 +1444,11 @@ void launch_relayout_scaled(const double* k_ref, const double* scale, const uint
 }
 
 void launch_bf16_diag(const double* src_rowmajor, const double* k_ref, const double* scale, const uint32_t* slot_elem,
-                      uint32_t n_slots, uint32_t n, float* out, hipStream_t s)
+                      uint32_t n_slots, uint32_t n, uint32_t rs, uint32_t ss, float* out, hipStream_t s)
 {
     const uint64_t rows = (uint64_t)n_slots * n;
     if (rows == 0) return;
-    bf16_diag_kernel<<<blocks_for(rows, 256), 256, 0, s>>>(src_rowmajor, k_ref, scale, slot_elem, n, rows, out);
+    bf16_diag_kernel<<<blocks_for(rows, 256), 256, 0, s>>>(src_rowmajor, k_ref, scale, slot_elem, n, rows, rs, ss, out);
     AMX_HIP(hipGetLastError());
 }
 

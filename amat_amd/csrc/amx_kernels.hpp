@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <vector>
 
 namespace amx {
 
@@ -62,10 +63,11 @@ void launch_relayout_from_rowmajor(const double* src, const uint32_t* slot_elem,
 // K_e = scale[elem] * k_ref (row-major n x n) -> tiled layout of kt.
 void launch_relayout_scaled(const double* k_ref, const double* scale, const uint32_t* slot_elem,
                             uint32_t n_slots, const Layout& L, KType kt, void* dst, hipStream_t s);
-// FP32 defect-corrected diagonal of the BF16 storage, [slot][r]; source either
-// row-major matrices (src_rowmajor) or k_ref + scale.
+// FP32 defect-corrected diagonal of the BF16 storage, entry (slot, r) at
+// out[r*rs + slot*ss]; source either row-major matrices (src_rowmajor) or
+// k_ref + scale.
 void launch_bf16_diag(const double* src_rowmajor, const double* k_ref, const double* scale, const uint32_t* slot_elem,
-                      uint32_t n_slots, uint32_t n, float* out, hipStream_t s);
+                      uint32_t n_slots, uint32_t n, uint32_t rs, uint32_t ss, float* out, hipStream_t s);
 // near-symmetric records: flags[r*n + c] (r > c) set to 1 where some matrix of
 // the group cannot code K[r][c] from K[c][r] (flags zeroed by the caller);
 // source either row-major matrices (src) or k_ref + scale
@@ -149,6 +151,38 @@ void launch_ebe_batched(uint32_t n, KType kt, bool vt_double, const EbeJob* jobs
                         bool masked);
 void launch_gather_batched(bool vt_double, const GatherJob* jobs, const uint32_t* prefix, uint32_t n_jobs,
                            uint32_t total_blocks, hipStream_t s);
+
+// ---- congruent groups (amx_cong.hip): K_e = scale[slot] * K_ref ----------
+struct CongArgs {
+    const double* kref;     // cong_pack of K_ref (BF16 storage: its diagonal zero)
+    const double* scale;    // [slot]
+    const uint32_t* map;    // [r][stride] local DoF ids, bit 31 as EbeArgs::map
+    const void* u;
+    void* out;              // ve (deterministic: row (slot, r) at ve_base + r*stride + slot) or v (atomic)
+    const float* kdiag;     // BF16 storage: FP32 diagonal [r][stride]
+    const uint32_t* skip;
+    uint64_t ve_base;
+    uint32_t stride;        // slots of the group
+    uint32_t slot_begin, n_slots;
+    uint32_t masked;        // identity BC form
+};
+bool cong_supported(uint32_t n);
+// blocks that share the rows of 64 elements in a launch over n_slots slots
+uint32_t cong_parts(uint32_t n, uint64_t n_slots);
+// blocks of a group's launch
+uint32_t cong_blocks(uint32_t n, uint32_t n_slots, uint32_t parts);
+// K_ref (row-major) in the order the kernel streams it (cong_pack_values: whole cache lines)
+uint64_t cong_pack_values(uint32_t n);
+std::vector<double> cong_pack(const std::vector<double>& kref, uint32_t n, bool zero_diag);
+void launch_cong(uint32_t n, KType kt, bool vt_double, bool atomic, const CongArgs& a, hipStream_t s);
+// many operators in one launch (deterministic scatter): work items are blocks,
+// cong_blocks per entry, prefix as for EbeJob
+struct CongJob {
+    CongArgs a;
+    uint32_t parts;
+};
+void launch_cong_batched(uint32_t n, KType kt, bool vt_double, const CongJob* jobs, const uint32_t* prefix,
+                         uint32_t n_jobs, uint32_t total_blocks, hipStream_t s);
 
 // ---- method 2 (FREE): element kernels from coordinates (amx_free.hip) ---
 struct FreeArgs {

@@ -180,6 +180,7 @@ void finalize_op(Op& op)
         g.nsym_xidx.release();
         g.nsym_colany = 0;
         for (auto& t : g.psx_tab) t.release();
+        g.cong_tab.release();
     }
     const bool free_m = op.is_free();
     if (free_m) {
@@ -209,6 +210,7 @@ void finalize_op(Op& op)
         g.L[1] = choose_layout(n, KType::F32);
         g.L[2] = choose_layout(n, KType::BF16);
         g.G = g.L[0].G;
+        g.cong = !free_m && op.scaled && op.sym_mode == 1 && cong_supported(n);
         // packed symmetric tiles when every stored matrix of the group is
         // bitwise symmetric (then K[r][c] and K[c][r] are the same value)
         if (!free_m && op.sym_mode == 1 && g.G > 1 && sym_supported(n)) {
@@ -245,21 +247,37 @@ void finalize_op(Op& op)
         // is known (near-symmetric records pad each element's rows to 64)
         auto assign_ve = [&](uint32_t pitch) {
             g.ve_base = ve_rows;
-            g.ve_rs = g.G > 1 ? g.n_slots : 1u;
-            g.ve_ss = g.G > 1 ? 1u : pitch;
-            ve_rows += (uint64_t)g.n_slots * (g.G > 1 ? n : pitch);
+            const bool by_row = g.G > 1 || g.cong;
+            g.ve_rs = by_row ? g.n_slots : 1u;
+            g.ve_ss = by_row ? 1u : pitch;
+            ve_rows += (uint64_t)g.n_slots * (by_row ? n : pitch);
         };
 
-        // map [slot][r]
+        // map [slot][r] (congruent groups: [r][slot], a wave reads row r of 64 slots)
         std::vector<uint32_t> hmap((size_t)g.n_slots * n, 0);
-        for (uint32_t sl = 0; sl < g.n_slots; sl++) {
+        auto entry = [&](uint32_t d) { return d | (zero_on_gather[d] ? kFlagBit : 0u); };
+        auto list_of = [&](uint32_t sl) {  // DoFs of the slot's element, NULL for padding
             const uint32_t i = g.slot_elem[sl];
-            if (i == kPadSlot) continue;
-            const uint32_t e = g.elems[i];
-            for (uint32_t r = 0; r < n; r++) {
-                const uint32_t d = op.local_map[op.eoff[e] + r];
-                hmap[(size_t)sl * n + r] = d | (zero_on_gather[d] ? kFlagBit : 0u);
+            return i == kPadSlot ? nullptr : &op.local_map[op.eoff[g.elems[i]]];
+        };
+        if (g.cong) {
+            // transposed in blocks of 64 slots, whose source rows stay in the cache
+            const int64_t nblk = ((int64_t)g.n_slots + 63) / 64;
+#pragma omp parallel for schedule(static) if (nblk > 1024)
+            for (int64_t b = 0; b < nblk; b++) {
+                const uint32_t first = (uint32_t)b * 64u, cnt = std::min(64u, g.n_slots - first);
+                const uint32_t* em[64];
+                for (uint32_t k = 0; k < cnt; k++) em[k] = list_of(first + k);
+                for (uint32_t r = 0; r < n; r++) {
+                    uint32_t* row = &hmap[(size_t)r * g.n_slots + first];
+                    for (uint32_t k = 0; k < cnt; k++)
+                        if (em[k]) row[k] = entry(em[k][r]);
+                }
             }
+        } else {
+            for (uint32_t sl = 0; sl < g.n_slots; sl++)
+                if (const uint32_t* em = list_of(sl))
+                    for (uint32_t r = 0; r < n; r++) hmap[(size_t)sl * n + r] = entry(em[r]);
         }
         upload(g.map, hmap, s, op.device_bytes);
         if (free_m) {
@@ -271,7 +289,24 @@ void finalize_op(Op& op)
         // element matrices: upload the source once, relayout on the device
         DevBuf src, src_scale, dslot;
         std::vector<uint32_t> slot_src(g.slot_elem);
-        if (op.scaled) {
+        std::vector<double> tab;
+        if (g.cong) {
+            // one table, kept: the packs of K_ref, the factors by slot (padding slots
+            // add exact zeros to rows that no list names), then K_ref as given and
+            // the factors by element for the layout kernels below
+            const uint64_t pack = cong_pack_values(n), nn = (uint64_t)n * n, ne = g.elems.size();
+            tab = cong_pack(op.kref, n, false);
+            tab.resize(2 * pack + g.n_slots + nn + ne, 0.0);
+            const std::vector<double> zero_diag = cong_pack(op.kref, n, true);
+            std::copy(zero_diag.begin(), zero_diag.end(), tab.begin() + pack);
+            double* cs = tab.data() + 2 * pack;
+            std::copy(op.kref.begin(), op.kref.end(), cs + g.n_slots);
+            for (uint64_t i = 0; i < ne; i++) {
+                cs[g.elem_slot[i]] = op.scale[g.elems[i]];
+                cs[g.n_slots + nn + i] = op.scale[g.elems[i]];
+            }
+            upload(g.cong_tab, tab, s, op.device_bytes);
+        } else if (op.scaled) {
             std::vector<double> sc(g.elems.size());
             for (uint32_t i = 0; i < g.elems.size(); i++) sc[i] = op.scale[g.elems[i]];
             uint64_t tmp = 0;
@@ -289,6 +324,10 @@ void finalize_op(Op& op)
         const double* src_rm = op.scaled ? nullptr : src.as<double>();
         const double* src_kref = op.scaled ? src.as<double>() : nullptr;
         const double* src_sc = op.scaled ? src_scale.as<double>() : nullptr;
+        if (g.cong) {
+            src_kref = g.cong_tab.as<double>() + 2 * cong_pack_values(n) + g.n_slots;
+            src_sc = src_kref + (uint64_t)n * n;
+        }
         // near-symmetric records for one-element FP64 tiles: find the lower
         // positions that some matrix cannot code from its transpose; few
         // enough of them -> records, else the whole layout
@@ -304,7 +343,7 @@ void finalize_op(Op& op)
         std::vector<uint32_t> xs, ptab[3];
         for (int kt = 0; kt < 3; kt++) {
             if (op.sym_mode != 1 || g.G != 1 || !nsym_supported(n) || g.n_slots == 0) break;
-            if (kt > 0 && !op.has(bits[kt])) continue;
+            if (kt > 0 && (!op.has(bits[kt]) || g.cong)) continue;
             DevBuf flags;
             flags.alloc((size_t)n * n * sizeof(uint32_t));
             AMX_HIP(hipMemsetAsync(flags.p, 0, flags.bytes, s));
@@ -335,7 +374,7 @@ void finalize_op(Op& op)
             if (kt == 0) {
                 g.nsym_colany = colany;
                 xs = first;
-                upload(g.nsym_xs, xs, s, op.device_bytes);
+                if (!g.cong) upload(g.nsym_xs, xs, s, op.device_bytes);
                 upload(g.nsym_xidx, xidx, s, op.device_bytes);
             } else {  // per lane (row min(l, n-1)): exception mask low, high, first X index
                 ptab[kt].assign(3 * 64, 0u);
@@ -354,17 +393,21 @@ void finalize_op(Op& op)
         assign_ve(g.L[0].nsym ? 64u : n);
         for (int kt = 0; kt < 3; kt++) {
             if (kt > 0 && !op.has(bits[kt])) continue;
-            const uint64_t bytes = (uint64_t)g.n_tiles * tile_values(g.L[kt], (KType)kt) * ktype_size((KType)kt);
-            g.K[kt].alloc(std::max<uint64_t>(bytes, 16));
-            op.device_bytes += g.K[kt].bytes;
-            if (kt == 0 && g.L[0].nsym)
+            if (kt == 0 || !g.cong) {
+                const uint64_t bytes = (uint64_t)g.n_tiles * tile_values(g.L[kt], (KType)kt) * ktype_size((KType)kt);
+                g.K[kt].alloc(std::max<uint64_t>(bytes, 16));
+                op.device_bytes += g.K[kt].bytes;
+            }
+            if (kt > 0 && g.cong)
+                ;  // rebuilt from K_ref in the kernel
+            else if (kt == 0 && g.L[0].nsym)
                 launch_relayout_nsym(src_rm, src_kref, src_sc, dslot.as<uint32_t>(), g.n_slots, g.L[0],
                                      dxrc[0].as<uint16_t>(), g.nsym_xidx.as<uint16_t>(), g.K[0].p, s);
             else if (g.L[kt].nsym)
                 launch_relayout_psx(src_rm, src_kref, src_sc, dslot.as<uint32_t>(), g.n_slots, g.L[kt], (KType)kt,
                                     dxrc[kt].as<uint16_t>(), g.K[kt].p, s);
             else if (op.scaled)
-                launch_relayout_scaled(src.as<double>(), src_scale.as<double>(), dslot.as<uint32_t>(), g.n_slots,
+                launch_relayout_scaled(src_kref, src_sc, dslot.as<uint32_t>(), g.n_slots,
                                        g.L[kt], (KType)kt, g.K[kt].p, s);
             else
                 launch_relayout_from_rowmajor(src.as<double>(), dslot.as<uint32_t>(), g.n_slots, g.L[kt], (KType)kt,
@@ -372,9 +415,8 @@ void finalize_op(Op& op)
             if (kt == (int)KType::BF16) {
                 g.kdiag16.alloc(std::max<uint64_t>((uint64_t)g.n_slots * n, 1) * sizeof(float));
                 op.device_bytes += g.kdiag16.bytes;
-                launch_bf16_diag(op.scaled ? nullptr : src.as<double>(), op.scaled ? src.as<double>() : nullptr,
-                                 op.scaled ? src_scale.as<double>() : nullptr, dslot.as<uint32_t>(), g.n_slots, n,
-                                 g.kdiag16.as<float>(), s);
+                launch_bf16_diag(src_rm, src_kref, src_sc, dslot.as<uint32_t>(), g.n_slots, n,
+                                 g.cong ? g.n_slots : 1u, g.cong ? 1u : n, g.kdiag16.as<float>(), s);
             }
         }
         AMX_HIP(hipStreamSynchronize(s));  // sources are freed at scope exit
@@ -570,6 +612,21 @@ void stage_block(Op& op, uint32_t eid, const double* m, int layout, uint32_t bi,
 
 }  // namespace
 
+CongArgs cong_args(const Group& g, KType kt, bool masked)
+{
+    CongArgs c{};
+    const uint64_t pack = cong_pack_values(g.n);
+    c.kref = g.cong_tab.as<double>() + (kt == KType::BF16 ? pack : 0);
+    c.scale = g.cong_tab.as<double>() + 2 * pack;
+    c.map = g.map.as<uint32_t>();
+    c.kdiag = kt == KType::BF16 ? g.kdiag16.as<float>() : nullptr;
+    c.ve_base = g.ve_base;
+    c.stride = g.n_slots;
+    c.n_slots = g.n_slots;
+    c.masked = masked ? 1u : 0u;
+    return c;
+}
+
 void ebe_launch(Op& op, KType kt, bool vt_double, bool masked, int phase, const void* u, void* v, hipStream_t s,
                 const uint32_t* skip, void* ve)
 {
@@ -591,6 +648,18 @@ void ebe_launch(Op& op, KType kt, bool vt_double, bool masked, int phase, const 
     }
     for (auto& g : op.groups) {
         const int k = (int)kt;
+        if (g.cong) {
+            AMX_REQUIRE(kt == KType::F64 || op.has(kt == KType::F32 ? AMX_PREC_FP32 : AMX_PREC_BF16),
+                        AMX_INVALID_STATE, "requested precision was not built at finalize");
+            CongArgs c = cong_args(g, kt, masked);
+            c.u = u;
+            c.out = atomic ? v : ve;
+            c.skip = skip;
+            if (phase == 0) c.n_slots = g.tiles_phase0 * g.G;
+            else if (phase == 1) { c.slot_begin = g.tiles_phase0 * g.G; c.n_slots = g.n_slots - c.slot_begin; }
+            launch_cong(g.n, kt, vt_double, atomic, c, s);
+            continue;
+        }
         AMX_REQUIRE(g.K[k].p != nullptr, AMX_INVALID_STATE, "requested precision was not built at finalize");
         EbeArgs a;
         a.K = g.K[k].p;
@@ -928,9 +997,10 @@ int amx_op_get_info(const amx_op* h, amx_op_info* info)
             // tiles; near-symmetric records (FP64 only) by their record size
             const uint64_t ns = g.L[0].sym ? (uint64_t)g.n * (g.n + 1) / 2 : nn;
             const uint64_t b64 = g.L[0].nsym ? amx::nsym_record_bytes(g.n, g.L[0].nx) : ns * 8;
-            // FP32 / BF16: the records as stored when built, else what they would hold
+            // FP32 / BF16: the records as stored when built, else what they would hold;
+            // congruent groups read a factor per element instead
             auto bytes_of = [&](int kt) {
-                return g.L[kt].nsym ? amx::tile_values(g.L[kt], (KType)kt) * amx::ktype_size((KType)kt)
+                return g.cong ? 8ull : g.L[kt].nsym ? amx::tile_values(g.L[kt], (KType)kt) * amx::ktype_size((KType)kt)
                                     : ns * amx::ktype_size((KType)kt);
             };
             if (g.L[0].sym) info->packed_symmetric++;
@@ -938,7 +1008,7 @@ int amx_op_get_info(const amx_op* h, amx_op_info* info)
             info->k_bytes_fp64 += ne * b64;
             info->k_bytes_fp32 += ne * bytes_of(1);
             info->k_bytes_bf16 += ne * bytes_of(2);
-            info->alg_bytes_fp64 += ne * (b64 + 4ull * g.n);
+            info->alg_bytes_fp64 += ne * ((g.cong ? 8ull : b64) + 4ull * g.n);
             info->flops += 2 * ne * nn;
         }
         info->alg_bytes_fp64 += 16ull * op.n_total;

@@ -40,6 +40,13 @@ struct Group {
     // FP32 / BF16 records (L[1] / L[2].nsym): per lane exception mask low,
     // high and first X index ([kt], kt = 1, 2)
     DevBuf psx_tab[3];
+    // congruent group (K_e = scale * K_ref, amx_cong.hip): the products read
+    // K_ref and a factor per slot instead of K; map and kdiag16 are [r][slot],
+    // the rows of ve likewise.  K[0] stays as the source of the multi-RHS
+    // layout and the diagonal; there is no K[1], K[2].
+    bool cong = false;
+    DevBuf cong_tab;                  // cong_pack of K_ref, the same with a zero diagonal, factor per slot;
+                                      // then K_ref and the factors as given (set-up)
 };
 
 struct Op {
@@ -166,6 +173,9 @@ struct DeviceGuard {
         if (prev >= 0 && hipGetDevice(&cur) == hipSuccess && cur != prev) (void)hipSetDevice(prev);
     }
 };
+
+// arguments of one application of a congruent group (u, out and skip unset)
+CongArgs cong_args(const Group& g, KType kt, bool masked);
 
 // launch pieces shared with the solvers
 // bc: 0 none, 1 identity, 2 penalty.  phase: 0 independent tiles, 1 dependent

@@ -95,6 +95,7 @@ struct amx_server {
     // batched element launches, key: n | kt << 16 | f64 << 24 | records << 25 |
     // (records) identity BC form << 26
     std::map<uint64_t, Table> ebe;
+    std::map<uint64_t, Table> cong;  // congruent groups, key: n | kt << 16 | f64 << 24; items are blocks
     Table gather[2], cg[2];         // [f64]
     std::vector<Job*> free_jobs;    // jobs on method-2 (FREE) operators: element kernels launched per job
     // the per-job FREE element kernels run on kAux side streams (default
@@ -156,6 +157,7 @@ void upload_table(Table& t, const std::vector<T>& rows, const std::vector<uint32
 void rebuild_tables(amx_server& S)
 {
     std::map<uint64_t, std::pair<std::vector<amx::EbeJob>, std::vector<uint32_t>>> ebe;
+    std::map<uint64_t, std::vector<amx::CongJob>> cong;
     std::vector<amx::GatherJob> g[2];
     std::vector<uint32_t> gp[2] = {{0}, {0}};
     std::vector<amx::CgJob> c[2];
@@ -170,6 +172,16 @@ void rebuild_tables(amx_server& S)
         if (op.is_free()) S.free_jobs.push_back(&j);
         for (auto& grp : op.groups) {
             if (op.is_free()) break;
+            if (grp.cong) {
+                amx::CongJob cj{};
+                cj.a = amx::cong_args(grp, j.kt, op.bc_operator == AMX_BCOP_IDENTITY);
+                cj.a.u = j.p.p;
+                cj.a.out = j.ve.p;
+                cj.a.skip = skip;
+                if (grp.n_slots)
+                    cong[(uint64_t)grp.n | ((uint64_t)j.kt << 16) | ((uint64_t)f << 24)].push_back(cj);
+                continue;
+            }
             // 60-DoF records: one-wave-block launches, one per BC form
             const bool rec = grp.L[(int)j.kt].nsym, masked = op.bc_operator == AMX_BCOP_IDENTITY;
             const uint64_t key = (uint64_t)grp.n | ((uint64_t)j.kt << 16) | ((uint64_t)f << 24) |
@@ -232,6 +244,18 @@ void rebuild_tables(amx_server& S)
         t.max_nx = 0;
         for (const auto& a : kv.second.first) t.max_nx = std::max(t.max_nx, a.nsym_nx);
     }
+    S.cong.clear();
+    for (auto& kv : cong) {
+        const uint32_t n = (uint32_t)(kv.first & 0xffff);
+        uint64_t slots = 0;
+        for (const auto& c : kv.second) slots += c.a.n_slots;
+        std::vector<uint32_t> prefix{0};
+        for (auto& c : kv.second) {
+            c.parts = amx::cong_parts(n, slots);
+            prefix.push_back(prefix.back() + amx::cong_blocks(n, c.a.n_slots, c.parts));
+        }
+        upload_table(S.cong[kv.first], kv.second, prefix);
+    }
     for (int f = 0; f < 2; f++) {
         upload_table(S.gather[f], g[f], gp[f]);
         upload_table(S.cg[f], c[f], cp[f]);
@@ -252,6 +276,12 @@ void launch_iteration(amx_server& S)
         Table& t = kv.second;
         amx::launch_ebe_batched(n, kt, f64, t.dev_jobs.as<amx::EbeJob>(), t.dev_prefix.as<uint32_t>(), t.n, t.total,
                                 s, rec, t.max_nx, masked);
+    }
+    for (auto& kv : S.cong) {
+        Table& t = kv.second;
+        amx::launch_cong_batched((uint32_t)(kv.first & 0xffff), (KType)((kv.first >> 16) & 0xff),
+                                 ((kv.first >> 24) & 1) != 0, t.dev_jobs.as<amx::CongJob>(),
+                                 t.dev_prefix.as<uint32_t>(), t.n, t.total, s);
     }
     if (!S.free_jobs.empty()) {  // element kernels from coordinates (FP64 or FP32) and the job's gather
         const int na = std::min<int>(amx_server::kAux, (int)S.free_jobs.size());

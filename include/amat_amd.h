@@ -207,9 +207,9 @@ typedef struct amx_op_info {
     double penalty;             /* value placed on constrained diagonals */
     uint64_t device_bytes;      /* device memory held by the handle */
     uint64_t k_bytes_fp64, k_bytes_fp32, k_bytes_bf16; /* element-matrix storage */
-    uint64_t alg_bytes_fp64;    /* E(b + 4n) + 16 N, b = FP64 bytes stored per element (8 n^2, 8 n(n+1)/2
-                                   packed, the record size of near-symmetric records): one FP64 matvec's
-                                   algorithmic HBM bytes */
+    uint64_t alg_bytes_fp64;    /* E(b + 4n) + 16 N, b = FP64 bytes read per element (8 n^2, 8 n(n+1)/2
+                                   packed, the record size of near-symmetric records, 8 for a factor): one
+                                   FP64 matvec's algorithmic HBM bytes */
     uint64_t flops;             /* 2 sum_e n_e^2 per matvec */
     uint32_t packed_symmetric;  /* element groups stored as packed symmetric tiles */
     uint32_t near_symmetric;    /* element groups stored as near-symmetric records (FP64) */
@@ -264,7 +264,9 @@ int amx_op_set_element_matrix(amx_op* op, uint32_t eid, const double* e_mat, int
 int amx_op_set_element_matrices(amx_op* op, uint32_t first_eid, uint32_t count,
                                 const double* e_mats, int layout);
 /* K_e = scale[e] * k_ref for every element (all elements share n): the
- * congruent structured meshes of the examples with per-element stiffness. */
+ * congruent structured meshes of the examples with per-element stiffness.
+ * With symmetric storage mode 1 and n = 8, 20, 24 or 60 the products read k_ref
+ * and the factors instead of stored matrices (the same results bit for bit). */
 int amx_op_set_element_matrices_scaled(amx_op* op, const double* k_ref, int layout,
                                        const double* scale);
 
