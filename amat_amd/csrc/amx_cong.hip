@@ -20,6 +20,7 @@
 #include <cstdint>
 #include <type_traits>
 
+#include "amx_device.hpp"
 #include "amx_internal.hpp"
 #include "amx_kernels.hpp"
 
@@ -31,13 +32,6 @@ constexpr uint32_t kFlagBit = 0x80000000u;
 constexpr uint32_t kIdxMask = 0x7fffffffu;
 constexpr int kWaveN = 8;  // largest n that cong_wave takes
 constexpr int kRows = 4;  // rows formed together: independent sums, one scalar load of 8 doubles per two columns
-
-__device__ __forceinline__ uint32_t xcd_block(uint32_t b, uint32_t nb)
-{
-    const uint32_t x = b & 7u, i = b >> 3;
-    const uint32_t q = nb >> 3, r = nb & 7u;
-    return x * q + (x < r ? x : r) + i;
-}
 
 __device__ __forceinline__ double madd(double acc, double k, double u)
 {
@@ -275,21 +269,16 @@ __global__ __launch_bounds__(256) void cong_kernel(CongArgs a, uint32_t parts)
     cong_group<N, KT, VT, ATOMIC>(a, b, parts);
 }
 
-// wave -> rows of 64 elements of entry owner (the largest j with prefix[j] <= w)
+// block -> block of the launch of entry job_of(prefix)
 template <int N, typename KT, typename VT>
 __global__ __launch_bounds__(256) void cong_batched_kernel(const CongJob* __restrict__ jobs,
                                                           const uint32_t* __restrict__ prefix, uint32_t n_jobs)
 {
     const uint32_t w = __builtin_amdgcn_readfirstlane(xcd_block(blockIdx.x, gridDim.x));
-    uint32_t lo = 0, hi = n_jobs;
-    while (hi - lo > 1) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (prefix[mid] <= w) lo = mid;
-        else hi = mid;
-    }
-    const CongArgs a = jobs[lo].a;
+    const uint32_t j = job_of(prefix, n_jobs, w);
+    const CongArgs a = jobs[j].a;
     if (a.skip && *a.skip) return;
-    cong_group<N, KT, VT, false>(a, w - prefix[lo], jobs[lo].parts);
+    cong_group<N, KT, VT, false>(a, w - prefix[j], jobs[j].parts);
 }
 
 template <int N, typename KT, typename VT> void launch_n(const CongArgs& a, bool atomic, hipStream_t s)

@@ -29,6 +29,7 @@
 #include <cstdint>
 #include <type_traits>
 
+#include "amx_device.hpp"
 #include "amx_internal.hpp"
 #include "amx_kernels.hpp"
 #include "amx_nsym.hpp"
@@ -40,16 +41,6 @@ namespace {
 constexpr uint32_t kFlagBit = 0x80000000u;
 constexpr uint32_t kIdxMask = 0x7fffffffu;
 constexpr uint32_t kPadSlot = 0xffffffffu;
-
-// Workgroups are dispatched round-robin over the 8 XCDs (block b runs on XCD
-// b % 8).  Return a logical block index such that XCD x gets the contiguous
-// logical range [x*q + min(x, r), ... + q + (x < r)), q = nb / 8, r = nb % 8.
-__device__ __forceinline__ uint32_t xcd_block(uint32_t b, uint32_t nb)
-{
-    const uint32_t x = b & 7u, i = b >> 3;
-    const uint32_t q = nb >> 3, r = nb & 7u;
-    return x * q + (x < r ? x : r) + i;
-}
 
 template <typename KT> struct KSize;
 template <> struct KSize<double> { static constexpr int v = 8; };
@@ -679,20 +670,7 @@ __global__ __launch_bounds__(64) void psx_kernel(const KT* __restrict__ K, uint3
     }
 }
 
-// index of the entry that owns work item x: the largest j < n with prefix[j] <= x
-// (x wave-uniform, so the search runs on the scalar unit)
-__device__ __forceinline__ uint32_t owner_of(const uint32_t* __restrict__ prefix, uint32_t n, uint32_t x)
-{
-    uint32_t lo = 0, hi = n;
-    while (hi - lo > 1) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (prefix[mid] <= x) lo = mid;
-        else hi = mid;
-    }
-    return lo;
-}
-
-// Many operators (jobs) in one launch: wave -> tile of entry owner_of(prefix).
+// Many operators (jobs) in one launch: wave -> tile of entry job_of(prefix).
 // Same per-tile arithmetic as ebe_tile_kernel (deterministic scatter only).
 // Jobs with near-symmetric records or packed records with exceptions run in
 // rec_batched_kernel instead.
@@ -704,7 +682,7 @@ __global__ __launch_bounds__(256) void ebe_tile_batched_kernel(const EbeJob* __r
     __shared__ __align__(16) KT ksh[SYM_OK ? 4u * sym_region_values<N, KT>() : 1u];
     const uint32_t gt = __builtin_amdgcn_readfirstlane(xcd_block(blockIdx.x, gridDim.x) * 4u + (threadIdx.x >> 6));
     if (gt >= prefix[n_jobs]) return;
-    const uint32_t j = owner_of(prefix, n_jobs, gt);
+    const uint32_t j = job_of(prefix, n_jobs, gt);
     const EbeJob& jb = jobs[j];
     if (jb.skip && *jb.skip) return;
     const uint32_t t = jb.tile_begin + (gt - prefix[j]);
@@ -733,7 +711,7 @@ __global__ __launch_bounds__(256) void ebe_tile_batched_kernel(const EbeJob* __r
 
 // Many jobs whose 60-DoF groups hold near-symmetric records (FP64) or packed
 // records with exceptions (FP32 / BF16), in one launch with the one-operator
-// kernels' shape: one-wave blocks, block -> element of entry owner_of(prefix),
+// kernels' shape: one-wave blocks, block -> element of entry job_of(prefix),
 // the dynamic LDS one region sized for the largest exception count of the
 // launch's jobs (so as many waves stay resident per CU as in a one-operator
 // launch).  Same arithmetic as ebe_nsym_kernel / psx_kernel.  MASKED: every
@@ -745,7 +723,7 @@ __global__ __launch_bounds__(64) void rec_batched_kernel(const EbeJob* __restric
     extern __shared__ __align__(16) char rec_lds[];
     const uint32_t gt = __builtin_amdgcn_readfirstlane(xcd_block(blockIdx.x, gridDim.x));
     if (gt >= prefix[n_jobs]) return;
-    const uint32_t j = owner_of(prefix, n_jobs, gt);
+    const uint32_t j = job_of(prefix, n_jobs, gt);
     const EbeJob& jb = jobs[j];
     if (jb.skip && *jb.skip) return;
     const uint32_t t = jb.tile_begin + (gt - prefix[j]), lane = threadIdx.x;
@@ -875,15 +853,14 @@ __global__ __launch_bounds__(256) void gather_kernel(const uint32_t* __restrict_
     gather_block<VT, BC>(off, pos, ve, u, flag, coef, v, n, d0, buf);
 }
 
-// many jobs in one launch: block -> 256 DoFs of entry owner_of(prefix)
+// many jobs in one launch: block -> 256 DoFs of entry job_of(prefix)
 template <typename VT>
 __global__ __launch_bounds__(256) void gather_batched_kernel(const GatherJob* __restrict__ jobs,
                                                             const uint32_t* __restrict__ prefix, uint32_t n_jobs)
 {
     __shared__ VT buf[kGatherWindow];
     const uint32_t gb = __builtin_amdgcn_readfirstlane(xcd_block(blockIdx.x, gridDim.x));
-    if (gb >= prefix[n_jobs]) return;
-    const uint32_t j = owner_of(prefix, n_jobs, gb);
+    const uint32_t j = job_of(prefix, n_jobs, gb);
     const GatherJob& jb = jobs[j];
     if (jb.skip && *jb.skip) return;
     const uint32_t d0 = (gb - prefix[j]) * 256u;
@@ -894,6 +871,111 @@ __global__ __launch_bounds__(256) void gather_batched_kernel(const GatherJob* __
     if (jb.bc == 1) gather_block<VT, 1>(jb.off, jb.pos, ve, u, jb.flag, jb.coef, v, jb.n, d0, buf);
     else if (jb.bc == 2) gather_block<VT, 2>(jb.off, jb.pos, ve, u, jb.flag, jb.coef, v, jb.n, d0, buf);
     else gather_block<VT, 0>(jb.off, jb.pos, ve, u, jb.flag, jb.coef, v, jb.n, d0, buf);
+}
+
+// The gather of a CG iteration with the sums of u . v of each reduction block:
+// block b of nblk = reduction_grid(n) owns DoFs b*256 + t + k*256*nblk, k < 4
+// (n <= kDotMaxDofs), the elements that thread t of reduction block b sums; its
+// 1,024 threads take the four runs side by side, then the first 256 add their
+// products in the order k = 0 .. 3 and the block's tree follows -- the sums of
+// a separate pass over u and v, bit for bit, without its launch and reads
+// (hex20 15^3 FP32, 47 k DoFs: gather 3.6 + dot product 7.4 us before, 6.0 us;
+// latency bounds it: list ranges, list entries, rows, then the block's tree).
+template <typename VT>
+__device__ __forceinline__ void gather_dot_block(const GatherJob& jb, uint32_t b, VT* buf)
+{
+    double* sh = reinterpret_cast<double*>(buf);  // once the windows are done: u, then v, of the block's 1,024 DoFs
+    static_assert(4u * kGatherWindow * sizeof(VT) >= 2304u * sizeof(double), "LDS overlay");
+    constexpr uint32_t PER = kGatherWindow / 256u;
+    const uint32_t tid = threadIdx.x & 255u, k = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+    const uint32_t n = jb.n, run = jb.nblk * 256u;
+    const uint32_t* __restrict__ off = jb.off;
+    const uint32_t* __restrict__ pos = jb.pos;
+    const VT* __restrict__ ve = static_cast<const VT*>(jb.ve);
+    const VT* __restrict__ u = static_cast<const VT*>(jb.u);
+    // list ranges of the four runs; every run loops as often as the longest
+    uint32_t e0 = 0, e1 = 0, span = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < 4u; j++) {
+        const uint32_t dj = b * 256u + j * run;
+        const uint32_t a = off[min(dj, n)], z = off[min(dj + 256u, n)];
+        span = max(span, z - a);
+        if (j == k) e0 = a, e1 = z;
+    }
+    const uint32_t d = b * 256u + k * run + tid;
+    const bool real = d < n;
+    uint32_t lb = 0, le = 0;
+    VT ud = VT(0);
+    bool flagged = false;
+    double co = 0.0;
+    if (real) {
+        lb = off[d], le = off[d + 1];
+        ud = u[d];
+        if (jb.bc) flagged = jb.flag[d] != 0;
+        if (jb.bc == 2) co = jb.coef[d];
+    }
+    VT* __restrict__ win = buf + k * kGatherWindow;
+    VT sum = VT(0);
+    for (uint32_t w0 = 0; w0 < span; w0 += kGatherWindow) {
+        const uint32_t w = e0 + w0, cnt = w < e1 ? min(kGatherWindow, e1 - w) : 0u;
+        if (cnt) {
+            uint32_t p[PER];
+            VT x[PER];
+#pragma unroll
+            for (uint32_t j = 0; j < PER; j++)
+                p[j] = __builtin_nontemporal_load(pos + w + min(tid + 256u * j, cnt - 1u));
+#pragma unroll
+            for (uint32_t j = 0; j < PER; j++) x[j] = ve[p[j]];
+#pragma unroll
+            for (uint32_t j = 0; j < PER; j++)
+                if (tid + 256u * j < cnt) win[tid + 256u * j] = x[j];
+        }
+        __syncthreads();
+        const uint32_t lo = max(lb, w), hi = min(le, w + cnt);
+        for (uint32_t q = lo; q < hi; q++) sum += win[q - w];
+        __syncthreads();
+    }
+    if (jb.bc == 1) {
+        if (flagged) sum = ud;
+    } else if (jb.bc == 2) {
+        if (flagged) sum = (VT)((double)sum + co * (double)ud);  // penalty row in FP64
+    }
+    if (real) static_cast<VT*>(jb.v)[d] = sum;
+    sh[threadIdx.x] = (double)ud;
+    sh[1024u + threadIdx.x] = (double)sum;
+    __syncthreads();
+    double acc = 0.0;
+    if (k == 0) {
+#pragma unroll
+        for (uint32_t j = 0; j < 4u; j++)
+            if (b * 256u + j * run + tid < n) acc = __builtin_fma(sh[j * 256u + tid], sh[1024u + j * 256u + tid], acc);
+    }
+    if (k == 0) sh[2048u + tid] = acc;
+    __syncthreads();
+    if (threadIdx.x < 64u) {
+        const double t = block_tree(sh + 2048);
+        if (threadIdx.x == 0) jb.dots[b] = t;
+    }
+}
+
+template <typename VT>
+__global__ __launch_bounds__(1024) void gather_dot_kernel(GatherJob jb)
+{
+    __shared__ __align__(16) VT buf[4u * kGatherWindow];
+    if (jb.skip && *jb.skip) return;
+    gather_dot_block<VT>(jb, __builtin_amdgcn_readfirstlane(xcd_block(blockIdx.x, gridDim.x)), buf);
+}
+
+template <typename VT>
+__global__ __launch_bounds__(1024) void gather_dot_batched_kernel(const GatherJob* __restrict__ jobs,
+                                                                 const uint32_t* __restrict__ prefix, uint32_t n_jobs)
+{
+    __shared__ __align__(16) VT buf[4u * kGatherWindow];
+    const uint32_t gb = __builtin_amdgcn_readfirstlane(xcd_block(blockIdx.x, gridDim.x));
+    const uint32_t j = job_of(prefix, n_jobs, gb);
+    const GatherJob jb = jobs[j];
+    if (jb.skip && *jb.skip) return;
+    gather_dot_block<VT>(jb, gb - prefix[j], buf);
 }
 
 template <typename VT, int BC>
@@ -1610,6 +1692,24 @@ void launch_ebe_batched(uint32_t n, KType kt, bool vt_double, const EbeJob* jobs
     }
 #undef AMX_EBE_N
 #undef AMX_EBE_B
+    AMX_HIP(hipGetLastError());
+}
+
+void launch_gather_dot(bool vt_double, const GatherJob& jb, hipStream_t s)
+{
+    if (jb.n == 0) return;
+    AMX_REQUIRE(jb.n <= kDotMaxDofs && jb.nblk == reduction_grid(jb.n), AMX_INVALID_STATE, "gather_dot: reduction grid");
+    if (vt_double) gather_dot_kernel<double><<<jb.nblk, 1024, 0, s>>>(jb);
+    else gather_dot_kernel<float><<<jb.nblk, 1024, 0, s>>>(jb);
+    AMX_HIP(hipGetLastError());
+}
+
+void launch_gather_dot_batched(bool vt_double, const GatherJob* jobs, const uint32_t* prefix, uint32_t n_jobs,
+                               uint32_t total_blocks, hipStream_t s)
+{
+    if (total_blocks == 0 || n_jobs == 0) return;
+    if (vt_double) gather_dot_batched_kernel<double><<<total_blocks, 1024, 0, s>>>(jobs, prefix, n_jobs);
+    else gather_dot_batched_kernel<float><<<total_blocks, 1024, 0, s>>>(jobs, prefix, n_jobs);
     AMX_HIP(hipGetLastError());
 }
 

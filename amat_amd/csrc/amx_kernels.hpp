@@ -140,8 +140,16 @@ struct GatherJob {
     void* v;
     uint32_t n, bc;
     const uint32_t* skip;
+    // launches with the dot product only: the sums of u . v per reduction block
+    // (dots[0 .. nblk - 1]), nblk = reduction_grid(n), n <= kDotMaxDofs
+    double* dots;
+    uint32_t nblk;
 };
 bool batched_n(uint32_t n);
+// the gather of a CG iteration with the sums of u . v of its reduction blocks
+void launch_gather_dot(bool vt_double, const GatherJob& jb, hipStream_t s);
+void launch_gather_dot_batched(bool vt_double, const GatherJob* jobs, const uint32_t* prefix, uint32_t n_jobs,
+                               uint32_t total_blocks, hipStream_t s);
 // records: every job's group holds near-symmetric records (FP64) or packed
 // records with exceptions (FP32 / BF16) of 60-DoF elements, at most max_nx
 // exception values each, and every job's masked flag equals `masked` (no job

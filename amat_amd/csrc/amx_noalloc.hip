@@ -16,7 +16,7 @@
 
 namespace {
 
-constexpr size_t kScalarsBytes = 256;  // two CgScalars, padded to keep the vectors aligned
+constexpr size_t kScalarsBytes = 512;  // two CgScalars, padded to keep the vectors aligned
 constexpr size_t kVecBytes = (size_t)AMX_NOALLOC_MAX_DOFS * sizeof(double);
 constexpr size_t kScratchBytes = amx::kPartialsBytes + kScalarsBytes + 5 * kVecBytes;
 static_assert(2 * sizeof(amx::CgScalars) <= kScalarsBytes, "scalar block");

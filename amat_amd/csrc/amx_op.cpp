@@ -687,6 +687,24 @@ void gather_launch(Op& op, bool vt_double, int bc, const void* u, void* v, hipSt
                   op.flag.as<uint8_t>(), op.coef64.as<double>(), v, op.n_total, s, skip);
 }
 
+GatherJob gather_job(const Op& op, const void* u, void* v, const void* ve, double* dots, const uint32_t* skip)
+{
+    GatherJob g{};
+    g.off = op.off.as<uint32_t>();
+    g.pos = op.pos.as<uint32_t>();
+    g.ve = ve ? ve : op.ve.p;
+    g.u = u;
+    g.flag = op.flag.as<uint8_t>();
+    g.coef = op.coef64.as<double>();
+    g.v = v;
+    g.n = op.n_total;
+    g.bc = (uint32_t)op.bc_operator;
+    g.skip = skip;
+    g.dots = dots;
+    g.nblk = reduction_grid(op.n_total);
+    return g;
+}
+
 void apply(Op& op, KType kt, bool vt_double, int bc, const void* u, void* v, hipStream_t s, const uint32_t* skip,
            void* ve)
 {

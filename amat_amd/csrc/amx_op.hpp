@@ -189,6 +189,12 @@ void ebe_launch(Op& op, KType kt, bool vt_double, bool masked, int phase, const 
                 const uint32_t* skip = nullptr, void* ve = nullptr);
 void gather_launch(Op& op, bool vt_double, int bc, const void* u, void* v, hipStream_t s,
                    const uint32_t* skip = nullptr, const void* ve = nullptr);
+// the handle's gather of ve (NULL: its own) with its BC form, v = A u; dots: where
+// launch_gather_dot leaves the block sums of u . v
+GatherJob gather_job(const Op& op, const void* u, void* v, const void* ve, double* dots, const uint32_t* skip);
+// q = A p and the block sums of p . q (partials + kDotOff) of a CG iteration
+void apply_dot(Op& op, KType kt, bool f64, const void* p, void* q, double* partials, CgScalars* dsc, hipStream_t s,
+               void* ve = nullptr);
 // complete one-rank operator application: v = A u with BC form bc
 void apply(Op& op, KType kt, bool vt_double, int bc, const void* u, void* v, hipStream_t s,
            const uint32_t* skip = nullptr, void* ve = nullptr);

@@ -96,7 +96,9 @@ struct amx_server {
     // (records) identity BC form << 26
     std::map<uint64_t, Table> ebe;
     std::map<uint64_t, Table> cong;  // congruent groups, key: n | kt << 16 | f64 << 24; items are blocks
-    Table gather[2], cg[2];         // [f64]
+    // [f64]: the gathers that also form p . q (jobs of up to kDotMaxDofs DoFs), the
+    // gathers and dot products of larger jobs, the vector updates of all
+    Table gather_dot[2], gather[2], pq[2], cg[2];
     std::vector<Job*> free_jobs;    // jobs on method-2 (FREE) operators: element kernels launched per job
     // the per-job FREE element kernels run on kAux side streams (default
     // priority) forked from and joined back into `stream` every iteration, so
@@ -158,10 +160,10 @@ void rebuild_tables(amx_server& S)
 {
     std::map<uint64_t, std::pair<std::vector<amx::EbeJob>, std::vector<uint32_t>>> ebe;
     std::map<uint64_t, std::vector<amx::CongJob>> cong;
-    std::vector<amx::GatherJob> g[2];
-    std::vector<uint32_t> gp[2] = {{0}, {0}};
-    std::vector<amx::CgJob> c[2];
-    std::vector<uint32_t> cp[2] = {{0}, {0}};
+    std::vector<amx::GatherJob> g[2], gd[2];
+    std::vector<uint32_t> gp[2] = {{0}, {0}}, gdp[2] = {{0}, {0}};
+    std::vector<amx::CgJob> c[2], pq[2];
+    std::vector<uint32_t> cp[2] = {{0}, {0}}, pqp[2] = {{0}, {0}};
     S.free_jobs.clear();
     for (auto& kv : S.jobs) {
         Job& j = *kv.second;
@@ -208,20 +210,17 @@ void rebuild_tables(amx_server& S)
             e.first.push_back(a);
             e.second.push_back(e.second.back() + grp.n_tiles);
         }
+        const bool dot = j.n <= amx::kDotMaxDofs;
         if (!op.is_free()) {  // method-2 jobs gather on their side stream (launch_iteration)
-            amx::GatherJob ga{};
-            ga.off = op.off.as<uint32_t>();
-            ga.pos = op.pos.as<uint32_t>();
-            ga.ve = j.ve.p;
-            ga.u = j.p.p;
-            ga.flag = op.flag.as<uint8_t>();
-            ga.coef = op.coef64.as<double>();
-            ga.v = j.q.p;
-            ga.n = j.n;
-            ga.bc = (uint32_t)op.bc_operator;
-            ga.skip = skip;
-            g[f].push_back(ga);
-            gp[f].push_back(gp[f].back() + (j.n + 255) / 256);
+            const amx::GatherJob ga =
+                amx::gather_job(op, j.p.p, j.q.p, j.ve.p, j.partials.as<double>() + amx::kDotOff, skip);
+            if (dot) {
+                gd[f].push_back(ga);
+                gdp[f].push_back(gdp[f].back() + ga.nblk);
+            } else {
+                g[f].push_back(ga);
+                gp[f].push_back(gp[f].back() + (j.n + 255) / 256);
+            }
         }
         amx::CgJob cj{};
         cj.x = j.xi;
@@ -236,6 +235,10 @@ void rebuild_tables(amx_server& S)
         cj.nblk = amx::reduction_grid(j.n);
         c[f].push_back(cj);
         cp[f].push_back(cp[f].back() + cj.nblk);
+        if (!dot) {
+            pq[f].push_back(cj);
+            pqp[f].push_back(pqp[f].back() + cj.nblk);
+        }
     }
     S.ebe.clear();
     for (auto& kv : ebe) {
@@ -257,14 +260,16 @@ void rebuild_tables(amx_server& S)
         upload_table(S.cong[kv.first], kv.second, prefix);
     }
     for (int f = 0; f < 2; f++) {
+        upload_table(S.gather_dot[f], gd[f], gdp[f]);
         upload_table(S.gather[f], g[f], gp[f]);
+        upload_table(S.pq[f], pq[f], pqp[f]);
         upload_table(S.cg[f], c[f], cp[f]);
     }
     S.tables_dirty = false;
 }
 
 // one CG iteration of every unfinished job: the order of the single-solve
-// loop (apply = element kernels + gather, then p.q, update, p)
+// loop (element kernels, gather and p.q, update, decision and p)
 void launch_iteration(amx_server& S)
 {
     hipStream_t s = S.stream;
@@ -295,7 +300,13 @@ void launch_iteration(amx_server& S)
                             S.aux[i % na], skip, jp->ve.p);
             // the job's gather follows on the same stream (the arithmetic of the
             // batched gather), so it overlaps the other jobs' element kernels
-            amx::gather_launch(op, jp->f64iter, op.bc_operator, jp->p.p, jp->q.p, S.aux[i % na], skip, jp->ve.p);
+            if (jp->n <= amx::kDotMaxDofs)
+                amx::launch_gather_dot(jp->f64iter,
+                                       amx::gather_job(op, jp->p.p, jp->q.p, jp->ve.p,
+                                                       jp->partials.as<double>() + amx::kDotOff, skip),
+                                       S.aux[i % na]);
+            else
+                amx::gather_launch(op, jp->f64iter, op.bc_operator, jp->p.p, jp->q.p, S.aux[i % na], skip, jp->ve.p);
         }
         for (int k = 0; k < na; k++) {
             AMX_HIP(hipEventRecord(S.join[k], S.aux[k]));
@@ -303,12 +314,15 @@ void launch_iteration(amx_server& S)
         }
     }
     for (int f = 0; f < 2; f++) {
+        Table& d = S.gather_dot[f];
+        amx::launch_gather_dot_batched(f == 1, d.dev_jobs.as<amx::GatherJob>(), d.dev_prefix.as<uint32_t>(), d.n,
+                                       d.total, s);
         Table& t = S.gather[f];
         amx::launch_gather_batched(f == 1, t.dev_jobs.as<amx::GatherJob>(), t.dev_prefix.as<uint32_t>(), t.n,
                                    t.total, s);
     }
     for (int f = 0; f < 2; f++) {
-        Table& t = S.cg[f];
+        Table& t = S.pq[f];
         amx::cg_pq_batched(f == 1, t.dev_jobs.as<amx::CgJob>(), t.dev_prefix.as<uint32_t>(), t.n, t.total, s);
     }
     for (int f = 0; f < 2; f++) {
@@ -317,7 +331,7 @@ void launch_iteration(amx_server& S)
     }
     for (int f = 0; f < 2; f++) {
         Table& t = S.cg[f];
-        amx::cg_p_batched(f == 1, t.dev_jobs.as<amx::CgJob>(), t.dev_prefix.as<uint32_t>(), t.n, t.total, s);
+        amx::cg_next_batched(f == 1, t.dev_jobs.as<amx::CgJob>(), t.dev_prefix.as<uint32_t>(), t.n, t.total, s);
     }
 }
 

@@ -33,6 +33,20 @@ void build_dinv(Op& op, double* dinv, double* d, hipStream_t s)
     invert(d, dinv, op.n_total, s);
 }
 
+// q = A p (a no-op once the solve has stopped) and the block sums of p . q
+void apply_dot(Op& op, KType kt, bool f64, const void* p, void* q, double* partials, CgScalars* dsc, hipStream_t s,
+               void* ve)
+{
+    const uint32_t* skip = &dsc->done;
+    if (op.scatter == AMX_SCATTER_DETERMINISTIC && op.n_total <= kDotAloneDofs && op.n_total > 0) {
+        ebe_launch(op, kt, f64, op.bc_operator == AMX_BCOP_IDENTITY, 2, p, q, s, skip, ve);
+        launch_gather_dot(f64, gather_job(op, p, q, ve, partials + kDotOff, skip), s);
+        return;
+    }
+    apply(op, kt, f64, op.bc_operator, p, q, s, skip, ve);
+    cg_pq(f64, p, q, op.n_total, partials, dsc, s);
+}
+
 namespace {
 
 void ensure(DevBuf& b, size_t bytes)
@@ -103,13 +117,11 @@ CgScalars cg_loop_ws(Op& op, KType kt, bool f64, void* x, void* r, void* z, void
     // poll every `chunk` iterations: about 1/8 of the iterations of a small
     // solve, every other one of a large solve
     const uint32_t chunk = n > (1u << 21) ? 2 : (n > (1u << 17) ? 4 : 8);
-    const uint32_t* skip = &dsc->done;
     for (int launched = 0;;) {
         for (uint32_t k = 0; k < chunk; k++) {
-            apply(op, kt, f64, op.bc_operator, p, q, s, skip);
-            cg_pq(f64, p, q, n, partials, dsc, s);
+            apply_dot(op, kt, f64, p, q, partials, dsc, s);
             cg_update(f64, x, r, z, p, q, dinv, n, partials, dsc, s);
-            cg_p(f64, p, z, n, dsc, s);
+            cg_next(f64, p, z, n, partials, dsc, s);
         }
         launched += (int)chunk;
         const CgScalars sc = read_scalars_via(host, dsc, s);
@@ -167,13 +179,11 @@ CgScalars ru_pcg(Op& op, KType kt, bool f64v, const double* b, double* x, void* 
     true_rr = true;
     if (sc.done) return sc;
     const uint32_t chunk = n > (1u << 21) ? 2 : (n > (1u << 17) ? 4 : 8);
-    const uint32_t* skip = &dsc->done;
     for (;;) {
         for (uint32_t k = 0; k < chunk; k++) {
-            apply(op, kt, f64v, op.bc_operator, ps, qs, s, skip);
-            cg_pq(f64v, ps, qs, n, partials, dsc, s);
+            apply_dot(op, kt, f64v, ps, qs, partials, dsc, s);
             cg_update(f64v, xs, rs, zs, ps, qs, dinv, n, partials, dsc, s);
-            cg_p(f64v, ps, zs, n, dsc, s);
+            cg_next(f64v, ps, zs, n, partials, dsc, s);
         }
         sc = read_scalars(op, dsc, s);
         if (!sc.done) continue;

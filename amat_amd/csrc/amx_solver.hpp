@@ -17,9 +17,15 @@ namespace amx {
 // limit reached).
 struct CgScalars {
     double rz, pq, rr, bb, alpha, beta, tol2, rmax2, d2, rr_prev;  // rr_prev: true ||r||^2 at the last replacement
+    // rz, rmax2 and iter as cg_update found them, and whether cg_next is to do
+    // nothing (the solve had stopped, or broke down): the blocks of cg_next read
+    // these while its first block writes rz, rmax2, iter and done.  No launch
+    // reads a scalar that one of its own blocks writes.
+    double rz_was, rmax2_was;
     uint32_t done, iter, max_it, breakdown, counter, state;
     uint32_t n_upd, max_upd;      // replacements done / allowed (reliable updates)
     uint32_t upd_iter, phase_len; // iteration of the last replacement; iterations of the phase before it
+    uint32_t iter_was, halt;
 };
 
 // one job of a batched CG launch (vectors of the launch's type)
@@ -38,16 +44,33 @@ struct CgJob {
 // Reductions: at most kMaxRedBlocks blocks; their partial sums, group sums and
 // counters live in a per-solve buffer of kPartialsBytes, zeroed when allocated.
 constexpr uint32_t kMaxRedBlocks = 1024;
+// A CG iteration leaves the block sums of p . q at kDotOff, of r . z and r . r
+// at kRzOff (strides of kMaxRedBlocks).
 constexpr size_t kPartialsBytes = 4096 * sizeof(double);
+constexpr size_t kDotOff = 0, kRzOff = kMaxRedBlocks;
+// largest n whose reduction blocks own four runs of 256 elements (the gather
+// of an iteration then forms the sums of p . q as well)
+constexpr uint32_t kDotMaxDofs = kMaxRedBlocks * 1024u;
+// A solve alone lets the gather form p . q up to this n: the launch saved counts
+// for more than the CUs that one block per 1,024 DoFs leaves idle (per
+// iteration, fused / separate: hex20 15^3, 47 k DoFs, 23.4 / 24.7 us FP64 and
+// 23.6 / 25.5 FP32; hex8 48^3, 118 k, 26.3 / 23.8; tet10 36^3, 389 k, 65.6 /
+// 63.4).  Served jobs fill the chip together and are always fused.
+constexpr uint32_t kDotAloneDofs = 65536u;
 // FP64 CG: residual replacements allowed after the recurrence stops (the
 // first one measures the true residual; more run only when it misses rtol)
 constexpr uint32_t kCgReplacements = 4;
 uint32_t reduction_grid(uint32_t n);
 void cg_init(bool f64, const void* b, const double* dinv, void* x, void* r, void* z, void* p, uint32_t n,
              double* partials, CgScalars* sc, hipStream_t s);
-void cg_pq(bool f64, const void* p, const void* q, uint32_t n, double* partials, CgScalars* sc, hipStream_t s);
+// One iteration after q = A p, three launches: the block sums of p . q (skipped
+// where the gather formed them), x += alpha p, r -= alpha q, z = r / diag with
+// the block sums of r . z and r . r, then the decision and p = z + beta p.
+void cg_pq(bool f64, const void* p, const void* q, uint32_t n, double* partials, const CgScalars* sc, hipStream_t s);
 void cg_update(bool f64, void* x, void* r, void* z, const void* p, const void* q, const double* dinv, uint32_t n,
                double* partials, CgScalars* sc, hipStream_t s);
+void cg_next(bool f64, void* p, const void* z, uint32_t n, double* partials, CgScalars* sc, hipStream_t s);
+// p = z + beta p with the scalars' beta (after a residual replacement)
 void cg_p(bool f64, void* p, const void* z, uint32_t n, const CgScalars* sc, hipStream_t s);
 void residual(const double* b, const double* ax, double* r, uint32_t n, double* partials, CgScalars* sc, hipStream_t s);
 void scale_to_f32(const double* r, float* r32, uint32_t n, const CgScalars* sc, hipStream_t s);
@@ -64,7 +87,7 @@ void cg_pq_batched(bool f64, const CgJob* jobs, const uint32_t* prefix, uint32_t
                    hipStream_t s);
 void cg_update_batched(bool f64, const CgJob* jobs, const uint32_t* prefix, uint32_t n_jobs, uint32_t total_blocks,
                        hipStream_t s);
-void cg_p_batched(bool f64, const CgJob* jobs, const uint32_t* prefix, uint32_t n_jobs, uint32_t total_blocks,
+void cg_next_batched(bool f64, const CgJob* jobs, const uint32_t* prefix, uint32_t n_jobs, uint32_t total_blocks,
                   hipStream_t s);
 void cg_reset(CgScalars* sc, double rtol, uint32_t max_it, hipStream_t s, double delta = 0.0,
               uint32_t max_upd = 0);

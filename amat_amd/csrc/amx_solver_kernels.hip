@@ -2,12 +2,14 @@
 //
 // All inner products accumulate in FP64 whatever the vector type.  Reductions
 // are deterministic: a fixed grid, a fixed element-to-thread assignment, an
-// LDS tree per block, and the partials summed in a fixed tree order by the
-// blocks that finish last (per group, then overall).  The scalars
+// LDS tree per block, and the block sums summed in a fixed tree order -- by
+// every block of the next launch inside an iteration, by the blocks that
+// finish last (per group, then overall) where no launch follows.  The scalars
 // (alpha, beta, residual norms, the converged flag) never leave the device;
 // every kernel becomes a no-op once `done` is set.
 #include <hip/hip_runtime.h>
 
+#include "amx_device.hpp"
 #include "amx_internal.hpp"
 #include "amx_solver.hpp"
 
@@ -125,35 +127,55 @@ __device__ bool reduce_partials(const double (&v)[NV], double* partials, uint32_
     return reduce_partials_n<NV>(v, partials, counter, tot, sh, blockIdx.x, gridDim.x);
 }
 
-// end of a CG update (one thread): plain runs stop on convergence or the
-// iteration limit; reliable-update runs (d2 > 0) stop there too, or when ||r||
-// has fallen below sqrt(d2) of its largest value since the last replacement,
-// or when the phase has run twice as long as the previous one (64 iterations
-// at least: a recurrence stalled by the operator's error), and leave the
-// decision to the replacement (state 1).  A stopped run keeps
-// rz and beta of the previous iteration.
-__device__ __forceinline__ void cg_update_finish(CgScalars* sc, double rz_new, double rr)
+// Decision after an iteration, from the new r . z and r . r: plain runs stop on
+// convergence or the iteration limit; reliable-update runs (d2 > 0) stop there
+// too, or when ||r|| has fallen below sqrt(d2) of its largest value since the
+// last replacement, or when the phase has run twice as long as the previous
+// one (64 iterations at least: a recurrence stalled by the operator's error),
+// and leave the decision to the replacement (state 1).  A stopped run keeps rz
+// and beta of the previous iteration.  Every block decides for itself, from
+// scalars that no block of the launch writes; `first` writes the outcome.
+__device__ __forceinline__ bool cg_decide(CgScalars* sc, double rz_new, double rr, bool first, double& beta)
 {
-    sc->iter += 1;
-    sc->rr = rr;
+    const uint32_t iter = sc->iter_was + 1u;
     const bool reliable = sc->d2 > 0.0;
-    if (rr <= sc->tol2 * sc->bb || sc->iter >= sc->max_it) {
-        sc->done = 1u;
-        if (reliable) sc->state = 1u;
-        return;
+    bool stop = rr <= sc->tol2 * sc->bb || iter >= sc->max_it;
+    double m = sc->rmax2_was;
+    if (!stop && reliable) {
+        m = rr > m ? rr : m;
+        const uint32_t len = iter - sc->upd_iter, cap = 2u * sc->phase_len;
+        if (rr < sc->d2 * m || len >= (cap > 64u ? cap : 64u)) stop = true;
     }
-    if (reliable) {
-        const double m = rr > sc->rmax2 ? rr : sc->rmax2;
+    beta = rz_new / sc->rz_was;
+    if (first) {
+        sc->iter = iter;
+        sc->rr = rr;
         sc->rmax2 = m;
-        const uint32_t len = sc->iter - sc->upd_iter, cap = 2u * sc->phase_len;
-        if (rr < sc->d2 * m || len >= (cap > 64u ? cap : 64u)) {
+        if (stop) {
+            if (reliable) sc->state = 1u;
             sc->done = 1u;
-            sc->state = 1u;
-            return;
+        } else {
+            sc->beta = beta;
+            sc->rz = rz_new;
         }
     }
-    sc->beta = rz_new / sc->rz;
-    sc->rz = rz_new;
+    return stop;
+}
+
+// block sums of NV values per thread -> part[k * kMaxRedBlocks + blk]
+template <int NV>
+__device__ __forceinline__ void leave_sums(const double (&v)[NV], double* part, uint32_t blk, double* sh)
+{
+#pragma unroll
+    for (int k = 0; k < NV; k++) sh[k * kBlock + threadIdx.x] = v[k];
+    __syncthreads();
+    if (threadIdx.x < 64u) {
+#pragma unroll
+        for (int k = 0; k < NV; k++) {
+            const double t = block_tree(sh + k * kBlock);
+            if (threadIdx.x == 0) part[k * kMaxRedBlocks + blk] = t;
+        }
+    }
 }
 
 template <typename VT>
@@ -186,51 +208,138 @@ __global__ __launch_bounds__(kBlock) void cg_init_kernel(const VT* __restrict__ 
     }
 }
 
+// The iteration's launches, for reduction block blk of nblk.  A thread's
+// elements i = blk*256 + t + k*256*nblk are loaded four at a time, the first
+// four before the totals of the launch before are summed.
+// Each launch is bound by latency until the vectors outgrow the caches: hex8
+// 48^3 (118 k DoFs) update 11.2 -> 4.8 us, decision and p 3.5 -> 4.7 us (it now
+// sums two totals), p . q 7.6 -> 3.2 us; a CG iteration 38.8 -> 23.8 us.
+constexpr int kAhead = 4;
+
 template <typename VT>
-__global__ __launch_bounds__(kBlock) void cg_pq_kernel(const VT* __restrict__ p, const VT* __restrict__ q, uint32_t n,
-                                                      double* partials, CgScalars* sc)
+__device__ __forceinline__ void cg_pq_block(const VT* __restrict__ p, const VT* __restrict__ q, uint32_t n,
+                                            double* partials, uint32_t blk, uint32_t nblk, double* sh)
 {
-    if (sc->done) return;
-    __shared__ double sh[kBlock];
     double acc[1] = {0.0};
-    for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock)
-        acc[0] += (double)p[i] * (double)q[i];
-    double tot[1];
-    if (!reduce_partials<1>(acc, partials, &sc->counter, tot, sh)) return;
-    if (threadIdx.x == 0) {
-        sc->pq = tot[0];
-        if (!(tot[0] > 0.0)) {  // operator not SPD on this direction
-            sc->breakdown = 1u;
-            sc->done = 1u;
-        } else {
-            sc->alpha = sc->rz / tot[0];
+    for (uint32_t i = blk * kBlock + threadIdx.x; i < n; i += nblk * kBlock) acc[0] += (double)p[i] * (double)q[i];
+    leave_sums<1>(acc, partials + kDotOff, blk, sh);
+}
+
+template <typename VT>
+__device__ __forceinline__ void cg_update_block(VT* __restrict__ x, VT* __restrict__ r, VT* __restrict__ z,
+                                                const VT* __restrict__ p, const VT* __restrict__ q,
+                                                const double* __restrict__ dinv, uint32_t n, double* partials,
+                                                CgScalars* sc, uint32_t blk, uint32_t nblk, double* sh)
+{
+    if (sc->done) {
+        if (blk == 0 && threadIdx.x == 0) sc->halt = 1u;
+        return;
+    }
+    const uint32_t step = nblk * kBlock;
+    VT xv[kAhead], rv[kAhead], pv[kAhead], qv[kAhead];
+    double dv[kAhead];
+    auto load = [&](uint32_t i0) {
+#pragma unroll
+        for (int k = 0; k < kAhead; k++) {
+            const uint32_t i = min(i0 + k * step, n - 1u);
+            xv[k] = x[i], rv[k] = r[i], pv[k] = p[i], qv[k] = q[i], dv[k] = dinv[i];
         }
+    };
+    uint32_t i0 = blk * kBlock + threadIdx.x;
+    load(i0);
+    double pq[1];
+    block_totals<1>(partials + kDotOff, nblk, sh, pq);
+    __syncthreads();  // sh is used again below
+    const double rz = sc->rz, alpha = rz / pq[0];
+    const bool bad = !(pq[0] > 0.0);  // operator not SPD on this direction
+    if (blk == 0 && threadIdx.x == 0) {
+        sc->pq = pq[0];
+        sc->rz_was = rz;
+        sc->rmax2_was = sc->rmax2;
+        sc->iter_was = sc->iter;
+        sc->halt = bad ? 1u : 0u;
+        if (bad) sc->breakdown = 1u;
+        else sc->alpha = alpha;
+    }
+    if (bad) return;
+    double acc[2] = {0.0, 0.0};
+    for (; i0 < n;) {
+#pragma unroll
+        for (int k = 0; k < kAhead; k++) {
+            const uint32_t i = i0 + k * step;
+            if (i < n) {
+                x[i] = (VT)((double)xv[k] + alpha * (double)pv[k]);
+                const double ri = (double)rv[k] - alpha * (double)qv[k];
+                const VT rn = (VT)ri;
+                const VT zn = (VT)(dv[k] * (double)rn);
+                r[i] = rn;
+                z[i] = zn;
+                acc[0] += (double)rn * (double)zn;
+                acc[1] += (double)rn * (double)rn;
+            }
+        }
+        i0 += kAhead * step;
+        if (i0 < n) load(i0);
+    }
+    leave_sums<2>(acc, partials + kRzOff, blk, sh);
+}
+
+template <typename VT>
+__device__ __forceinline__ void cg_next_block(VT* __restrict__ p, const VT* __restrict__ z, uint32_t n,
+                                              const double* partials, CgScalars* sc, uint32_t blk, uint32_t nblk,
+                                              double* sh)
+{
+    if (sc->halt) {  // stopped before this iteration, or a breakdown in it
+        if (blk == 0 && threadIdx.x == 0 && sc->breakdown) sc->done = 1u;
+        return;
+    }
+    const uint32_t step = nblk * kBlock;
+    VT zv[kAhead], pv[kAhead];
+    auto load = [&](uint32_t i0) {
+#pragma unroll
+        for (int k = 0; k < kAhead; k++) {
+            const uint32_t i = min(i0 + k * step, n - 1u);
+            zv[k] = z[i], pv[k] = p[i];
+        }
+    };
+    uint32_t i0 = blk * kBlock + threadIdx.x;
+    load(i0);
+    double tot[2], beta;
+    block_totals<2>(partials + kRzOff, nblk, sh, tot);
+    if (cg_decide(sc, tot[0], tot[1], blk == 0 && threadIdx.x == 0, beta)) return;
+    for (; i0 < n;) {
+#pragma unroll
+        for (int k = 0; k < kAhead; k++)
+            if (i0 + k * step < n) p[i0 + k * step] = (VT)((double)zv[k] + beta * (double)pv[k]);
+        i0 += kAhead * step;
+        if (i0 < n) load(i0);
     }
 }
 
 template <typename VT>
-__global__ __launch_bounds__(kBlock) void cg_update_kernel(VT* __restrict__ x, VT* __restrict__ r, VT* __restrict__ z,
-                                                          const VT* __restrict__ p, const VT* __restrict__ q,
-                                                          const double* __restrict__ dinv, uint32_t n,
-                                                          double* partials, CgScalars* sc)
+__global__ __launch_bounds__(kBlock) void cg_pq_kernel(const VT* p, const VT* q, uint32_t n, double* partials,
+                                                      const CgScalars* sc)
 {
-    if (sc->done) return;
     __shared__ double sh[kBlock];
-    const double alpha = sc->alpha;
-    double acc[2] = {0.0, 0.0};
-    for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
-        x[i] = (VT)((double)x[i] + alpha * (double)p[i]);
-        const double ri = (double)r[i] - alpha * (double)q[i];
-        const VT rv = (VT)ri;
-        const VT zv = (VT)(dinv[i] * (double)rv);
-        r[i] = rv;
-        z[i] = zv;
-        acc[0] += (double)rv * (double)zv;
-        acc[1] += (double)rv * (double)rv;
-    }
-    double tot[2];
-    if (!reduce_partials<2>(acc, partials, &sc->counter, tot, sh)) return;
-    if (threadIdx.x == 0) cg_update_finish(sc, tot[0], tot[1]);
+    if (sc->done) return;
+    cg_pq_block<VT>(p, q, n, partials, blockIdx.x, gridDim.x, sh);
+}
+
+template <typename VT>
+__global__ __launch_bounds__(kBlock) void cg_update_kernel(VT* x, VT* r, VT* z, const VT* p, const VT* q,
+                                                          const double* dinv, uint32_t n, double* partials,
+                                                          CgScalars* sc)
+{
+    __shared__ double sh[2 * kBlock];
+    cg_update_block<VT>(x, r, z, p, q, dinv, n, partials, sc, blockIdx.x, gridDim.x, sh);
+}
+
+template <typename VT>
+__global__ __launch_bounds__(kBlock) void cg_next_kernel(VT* p, const VT* z, uint32_t n, const double* partials,
+                                                        CgScalars* sc)
+{
+    __shared__ double sh[2 * kBlock];
+    cg_next_block<VT>(p, z, n, partials, sc, blockIdx.x, gridDim.x, sh);
 }
 
 template <typename VT>
@@ -310,93 +419,39 @@ __global__ void invert_kernel(const double* __restrict__ d, double* __restrict__
 // Block -> (job j, local block lb) through the block prefix; every job keeps
 // the grid of its single-job launch (reduction_grid(n) blocks, same stride),
 // so its sums are bit-identical to a solve of that job alone.
-__device__ __forceinline__ uint32_t job_of(const uint32_t* __restrict__ prefix, uint32_t n, uint32_t x)
-{
-    uint32_t lo = 0, hi = n;
-    while (hi - lo > 1) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (prefix[mid] <= x) lo = mid;
-        else hi = mid;
-    }
-    return lo;
-}
-
 template <typename VT>
 __global__ __launch_bounds__(kBlock) void cg_pq_batched_kernel(const CgJob* __restrict__ jobs,
                                                               const uint32_t* __restrict__ prefix, uint32_t n_jobs)
 {
-    const uint32_t gb = __builtin_amdgcn_readfirstlane(blockIdx.x);
-    const uint32_t j = job_of(prefix, n_jobs, gb);
-    const CgJob& jb = jobs[j];
-    CgScalars* sc = jb.sc;
-    if (sc->done) return;
     __shared__ double sh[kBlock];
-    const uint32_t lb = gb - prefix[j], nblk = jb.nblk, n = jb.n;
-    const VT* p = static_cast<const VT*>(jb.p);
-    const VT* q = static_cast<const VT*>(jb.q);
-    double acc[1] = {0.0};
-    for (uint32_t i = lb * kBlock + threadIdx.x; i < n; i += nblk * kBlock) acc[0] += (double)p[i] * (double)q[i];
-    double tot[1];
-    if (!reduce_partials_n<1>(acc, jb.partials, &sc->counter, tot, sh, lb, nblk)) return;
-    if (threadIdx.x == 0) {
-        sc->pq = tot[0];
-        if (!(tot[0] > 0.0)) {
-            sc->breakdown = 1u;
-            sc->done = 1u;
-        } else {
-            sc->alpha = sc->rz / tot[0];
-        }
-    }
+    const uint32_t j = job_of(prefix, n_jobs, blockIdx.x);
+    const CgJob jb = jobs[j];
+    if (jb.sc->done) return;
+    cg_pq_block<VT>(static_cast<const VT*>(jb.p), static_cast<const VT*>(jb.q), jb.n, jb.partials,
+                    blockIdx.x - prefix[j], jb.nblk, sh);
 }
 
 template <typename VT>
 __global__ __launch_bounds__(kBlock) void cg_update_batched_kernel(const CgJob* __restrict__ jobs,
                                                                   const uint32_t* __restrict__ prefix, uint32_t n_jobs)
 {
-    const uint32_t gb = __builtin_amdgcn_readfirstlane(blockIdx.x);
-    const uint32_t j = job_of(prefix, n_jobs, gb);
-    const CgJob& jb = jobs[j];
-    CgScalars* sc = jb.sc;
-    if (sc->done) return;
-    __shared__ double sh[kBlock];
-    const uint32_t lb = gb - prefix[j], nblk = jb.nblk, n = jb.n;
-    VT* x = static_cast<VT*>(jb.x);
-    VT* r = static_cast<VT*>(jb.r);
-    VT* z = static_cast<VT*>(jb.z);
-    const VT* p = static_cast<const VT*>(jb.p);
-    const VT* q = static_cast<const VT*>(jb.q);
-    const double* dinv = jb.dinv;
-    const double alpha = sc->alpha;
-    double acc[2] = {0.0, 0.0};
-    for (uint32_t i = lb * kBlock + threadIdx.x; i < n; i += nblk * kBlock) {
-        x[i] = (VT)((double)x[i] + alpha * (double)p[i]);
-        const double ri = (double)r[i] - alpha * (double)q[i];
-        const VT rv = (VT)ri;
-        const VT zv = (VT)(dinv[i] * (double)rv);
-        r[i] = rv;
-        z[i] = zv;
-        acc[0] += (double)rv * (double)zv;
-        acc[1] += (double)rv * (double)rv;
-    }
-    double tot[2];
-    if (!reduce_partials_n<2>(acc, jb.partials, &sc->counter, tot, sh, lb, nblk)) return;
-    if (threadIdx.x == 0) cg_update_finish(sc, tot[0], tot[1]);
+    __shared__ double sh[2 * kBlock];
+    const uint32_t j = job_of(prefix, n_jobs, blockIdx.x);
+    const CgJob jb = jobs[j];
+    cg_update_block<VT>(static_cast<VT*>(jb.x), static_cast<VT*>(jb.r), static_cast<VT*>(jb.z),
+                        static_cast<const VT*>(jb.p), static_cast<const VT*>(jb.q), jb.dinv, jb.n, jb.partials, jb.sc,
+                        blockIdx.x - prefix[j], jb.nblk, sh);
 }
 
 template <typename VT>
-__global__ __launch_bounds__(kBlock) void cg_p_batched_kernel(const CgJob* __restrict__ jobs,
-                                                             const uint32_t* __restrict__ prefix, uint32_t n_jobs)
+__global__ __launch_bounds__(kBlock) void cg_next_batched_kernel(const CgJob* __restrict__ jobs,
+                                                                const uint32_t* __restrict__ prefix, uint32_t n_jobs)
 {
-    const uint32_t gb = __builtin_amdgcn_readfirstlane(blockIdx.x);
-    const uint32_t j = job_of(prefix, n_jobs, gb);
-    const CgJob& jb = jobs[j];
-    const CgScalars* sc = jb.sc;
-    if (sc->done) return;
-    const uint32_t lb = gb - prefix[j], nblk = jb.nblk, n = jb.n;
-    VT* p = static_cast<VT*>(jb.p);
-    const VT* z = static_cast<const VT*>(jb.z);
-    const double beta = sc->beta;
-    for (uint32_t i = lb * kBlock + threadIdx.x; i < n; i += nblk * kBlock) p[i] = (VT)((double)z[i] + beta * (double)p[i]);
+    __shared__ double sh[2 * kBlock];
+    const uint32_t j = job_of(prefix, n_jobs, blockIdx.x);
+    const CgJob jb = jobs[j];
+    cg_next_block<VT>(static_cast<VT*>(jb.p), static_cast<const VT*>(jb.z), jb.n, jb.partials, jb.sc,
+                      blockIdx.x - prefix[j], jb.nblk, sh);
 }
 
 // ---- reliable updates (mixed-precision CG with residual replacement) ----
@@ -498,7 +553,7 @@ void cg_init(bool f64, const void* b, const double* dinv, void* x, void* r, void
     AMX_HIP(hipGetLastError());
 }
 
-void cg_pq(bool f64, const void* p, const void* q, uint32_t n, double* partials, CgScalars* sc, hipStream_t s)
+void cg_pq(bool f64, const void* p, const void* q, uint32_t n, double* partials, const CgScalars* sc, hipStream_t s)
 {
     const uint32_t g = reduction_grid(n);
     if (f64) cg_pq_kernel<double><<<g, kBlock, 0, s>>>((const double*)p, (const double*)q, n, partials, sc);
@@ -512,6 +567,14 @@ void cg_update(bool f64, void* x, void* r, void* z, const void* p, const void* q
     const uint32_t g = reduction_grid(n);
     if (f64) cg_update_kernel<double><<<g, kBlock, 0, s>>>((double*)x, (double*)r, (double*)z, (const double*)p, (const double*)q, dinv, n, partials, sc);
     else cg_update_kernel<float><<<g, kBlock, 0, s>>>((float*)x, (float*)r, (float*)z, (const float*)p, (const float*)q, dinv, n, partials, sc);
+    AMX_HIP(hipGetLastError());
+}
+
+void cg_next(bool f64, void* p, const void* z, uint32_t n, double* partials, CgScalars* sc, hipStream_t s)
+{
+    const uint32_t g = reduction_grid(n);
+    if (f64) cg_next_kernel<double><<<g, kBlock, 0, s>>>((double*)p, (const double*)z, n, partials, sc);
+    else cg_next_kernel<float><<<g, kBlock, 0, s>>>((float*)p, (const float*)z, n, partials, sc);
     AMX_HIP(hipGetLastError());
 }
 
@@ -571,12 +634,12 @@ void cg_update_batched(bool f64, const CgJob* jobs, const uint32_t* prefix, uint
     AMX_HIP(hipGetLastError());
 }
 
-void cg_p_batched(bool f64, const CgJob* jobs, const uint32_t* prefix, uint32_t n_jobs, uint32_t total_blocks,
+void cg_next_batched(bool f64, const CgJob* jobs, const uint32_t* prefix, uint32_t n_jobs, uint32_t total_blocks,
                   hipStream_t s)
 {
     if (!total_blocks) return;
-    if (f64) cg_p_batched_kernel<double><<<total_blocks, kBlock, 0, s>>>(jobs, prefix, n_jobs);
-    else cg_p_batched_kernel<float><<<total_blocks, kBlock, 0, s>>>(jobs, prefix, n_jobs);
+    if (f64) cg_next_batched_kernel<double><<<total_blocks, kBlock, 0, s>>>(jobs, prefix, n_jobs);
+    else cg_next_batched_kernel<float><<<total_blocks, kBlock, 0, s>>>(jobs, prefix, n_jobs);
     AMX_HIP(hipGetLastError());
 }
 
