@@ -315,6 +315,16 @@ std::vector<double> free_quadrature(int kind, uint32_t ngt, uint32_t& nq, uint32
     return t;
 }
 
+std::vector<double> gauss_rule(uint32_t ngt)
+{
+    check_ngt(ngt);
+    double pw[2 * 16];
+    gauss_legendre(ngt, pw);
+    std::vector<double> r(2 * ngt);
+    for (uint32_t i = 0; i < ngt; i++) r[i] = pw[2 * i], r[ngt + i] = pw[2 * i + 1];
+    return r;
+}
+
 }  // namespace amx
 
 extern "C" {

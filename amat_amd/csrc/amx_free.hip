@@ -28,6 +28,7 @@
 #include <atomic>
 #include <type_traits>
 
+#include "amx_device.hpp"
 #include "amx_internal.hpp"
 #include "amx_kernels.hpp"
 
@@ -44,17 +45,6 @@ __device__ __forceinline__ void lds_sync_wave()
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
-
-// two-value LDS accesses of the compute type RT (FP64 or FP32)
-template <typename RT> struct Vec2;
-template <> struct Vec2<double> {
-    using type = double2;
-    __device__ static type make(double a, double b) { return make_double2(a, b); }
-};
-template <> struct Vec2<float> {
-    using type = float2;
-    __device__ static type make(float a, float b) { return make_float2(a, b); }
-};
 
 // det J and inv[d][k] = cofactor(J)[k][d] / det (cofactors as in the host
 // element routines, amx_fem.cpp jacobian; one division)
@@ -157,254 +147,404 @@ __global__ __launch_bounds__(256) void free_laplace_kernel(const RT* __restrict_
 }
 
 // ---- hex20 isotropic elasticity -----------------------------------------
-// A wave takes EW = 64/QP element slots at a time; in phase 1 lane
-// l = e*QP + q holds element e at quadrature point q (QP: the point count
-// padded to 8, 32 or 64; padding points carry weight 0) and writes P (or inv
-// and w for DIAG) to an LDS slot; in phase 2 lane o = 3a+i < 60 sums the
-// output o of each element over the points.  xe: [slot][60], qp: [QP][61].
-// The grid is persistent: a block loads the dN table into LDS once and its
-// waves loop over element groups.  LDS strides avoid bank conflicts of the
-// 16-byte reads: dN rows [q][a][4] at kTabRow doubles (2*kTabRow = 4 * odd
-// dwords, so 8 rows hit 8 distinct bank groups), node values [e][a][x y z
-// u_x u_y u_z] at kElemRow doubles per element (likewise); the P slots
-// overlay the node values once phase 1 has read them.
-constexpr int kH20Slot = 12;   // S[4i+d] = P_di (DIAG: S[4k+d] = inv[d][k]), S[3] = w
-// LDS strides per compute type: FP64 reads two values per 16-byte access
-// (dN rows of 82, node values x y z u_x u_y u_z at 6 per node, 122 per
-// element); FP32 reads a whole dN row quadruple, a P row or a node's
-// x y z u_x in one 16-byte access (rows of 84, 8 values per node: x y z u_x
-// u_y u_z and 2 pad, 164 per element)
-template <typename RT> struct H20Lds;
-template <> struct H20Lds<double> { static constexpr int tab_row = 82, elem_row = 122, node = 6; };
-template <> struct H20Lds<float> { static constexpr int tab_row = 84, elem_row = 164, node = 8; };
+// The serendipity interpolant is a polynomial with few terms per direction, so
+// its derivatives need not be summed node by node at every point.  With a the
+// direction of the derivative and b, c the other two (cyclic), signs s_b, s_c
+// of the four node lines along a (end values f-, f+, middle f0), and
+//   D = f+ - f-,  S = f+ + f- - 2 f0  of a line, D00 = sum D, D10 = sum s_b D,
+//   D01 = sum s_c D, D11 = sum s_b s_c D (S alike), E_b0, E_b1 the sum and
+//   difference over s_c of f+ - f- of the b-edge middles, E_c0, E_c1 alike:
+//   df/da = A(b, c) + a B(b, c)
+//   A = al + be b^2 + ga c^2 + de bc + ep c + ze b^2 c + et b + th bc^2
+//   B = s00 + s10 b + s01 c + s11 bc
+//   al = (E_b0 + E_c0)/4 - D00/8, be = D00/8 - E_b0/4, ga = D00/8 - E_c0/4,
+//   de = D11/8, ep = E_b1/4, ze = D01/8 - E_b1/4, et = E_c1/4,
+//   th = D10/8 - E_c1/4, sxx = Sxx/4.
+// At the ngt^3 points of a tensor rule that is about 5 operations per value
+// instead of 20, and the transposed sums of the output likewise.
+//
+// A wave takes EW elements at a time, the values passed through its LDS region
+// between the stages:
+//   1  lane (element, coordinate, direction), 9 per element: 20 node values ->
+//      12 coefficients -> the derivative at all points;
+//   2  lane (element, point): J -> inverse and weight, kept in registers;
+//   3  stage 1 on u in place of the coordinates;
+//   4  lane (element, point): H -> stress -> P, 9 values in place of H;
+//   5  lane (element, component, direction): the points' P -> 12 coefficients
+//      -> 20 node contributions; then the sum over directions.
+// EW = 7 fills 63 lanes in stages 1, 3 and 5 (and 189 = 2.95 waves of points at
+// ngt = 3).  Coordinates and u in turn, so that a region holds the derivatives
+// of three fields and not of six (both at once: 27 KB per wave at ngt = 3, 5
+// waves per CU, 126 us on 48^3).  LDS rows have odd strides: lanes of stages
+// 1, 3 and 5 hit distinct banks.
+//
+// What bounds it: the chain of stages with 8 (FP64, ngt = 3) to 16 waves per CU
+// in flight (VGPRs; 4 waves per SIMD asked for in FP64 spill, 132 us).  Against
+// node-by-node sums (60 per point and direction, 440 LDS values per lane),
+// element kernel FP64 / matvec FP64 / matvec FP32:
+//   48^3, ngt = 3   176 -> 78 us   217 -> 110 us   147 -> 71 us
+//   48^3, ngt = 2    59 -> 53 us    86 ->  83 us    62 -> 55 us
+//   24^3, ngt = 3                   36 ->  20 us    27 -> 15 us
+//   24^3, ngt = 4                   75 ->  42 us    56 -> 27 us
+// Relative L2 error of the FP64 product (12^3): ngt = 2 2.5e-15 -> 4.5e-16,
+// ngt = 3 and 4 as before (9e-15, 2.1e-14: the digits of the rule).
+constexpr uint32_t kH20Node[3][5] = {  // byte j: 8 * node of entry j (per line f-, f+, f0; then the edge pairs)
+    {0x18400800u, 0x28205010u, 0x70303860u, 0x68784858u, 0x90988880u},
+    {0x20581800u, 0x10087838u, 0x68302848u, 0x90889880u, 0x70605040u},
+    {0x08802000u, 0x38188828u, 0x90301098u, 0x70506040u, 0x68487858u}};
 
-template <int QP, typename RT> constexpr int h20_wave_values()
+template <int NG> struct H20 {
+    static constexpr int EW = NG == 4 ? 3 : 7;      // elements per wave
+    static constexpr int PTS = NG * NG * NG;
+    static constexpr int TS = PTS | 1;              // values of one (field, direction), odd
+    static constexpr int GS = 9 * TS;               // derivatives of one element's three fields
+    static constexpr int CS = 181, IS = 61;         // node contributions [direction][60], node values [field][20]
+    static constexpr int WAVE = EW * (GS > CS ? GS : CS);
+    static constexpr int P2 = (EW * PTS + 63) / 64; // passes over the points
+};
+
+// 12 coefficients of a (field, direction) from its 20 node values
+template <typename RT> struct H20Coef {
+    RT al, be, ga, de, ep, ze, et, th, s00, s10, s01, s11;
+
+    static __device__ __forceinline__ void fly(const RT x[4], RT& q00, RT& q10, RT& q01, RT& q11)
+    {
+        const RT a0 = x[0] + x[1], a1 = x[1] - x[0], b0 = x[2] + x[3], b1 = x[3] - x[2];
+        q00 = a0 + b0, q01 = b0 - a0, q10 = a1 + b1, q11 = b1 - a1;
+    }
+    __device__ __forceinline__ void from_nodes(const RT (&v)[20])
+    {
+        RT D[4], S[4], d00, d10, d01, d11;
+#pragma unroll
+        for (int l = 0; l < 4; l++) {
+            D[l] = v[3 * l + 1] - v[3 * l];
+            S[l] = (v[3 * l + 1] - v[3 * l + 2]) + (v[3 * l] - v[3 * l + 2]);
+        }
+        fly(D, d00, d10, d01, d11);
+        fly(S, s00, s10, s01, s11);
+        s00 *= RT(0.25), s10 *= RT(0.25), s01 *= RT(0.25), s11 *= RT(0.25);
+        const RT e0 = v[13] - v[12], e1 = v[15] - v[14], g0 = v[17] - v[16], g1 = v[19] - v[18];
+        const RT eb0 = RT(0.25) * (e0 + e1), eb1 = RT(0.25) * (e1 - e0);
+        const RT ec0 = RT(0.25) * (g0 + g1), ec1 = RT(0.25) * (g1 - g0);
+        be = RT(0.125) * d00 - eb0, ga = RT(0.125) * d00 - ec0, al = eb0 - ga;
+        de = RT(0.125) * d11;
+        ep = eb1, ze = RT(0.125) * d01 - eb1;
+        et = ec1, th = RT(0.125) * d10 - ec1;
+    }
+    // derivative at the points (b, c, a), a fastest
+    template <int NG> __device__ __forceinline__ void evaluate(const RT (&x)[NG], RT* g) const
+    {
+#pragma unroll
+        for (int b = 0; b < NG; b++) {
+            const RT xb = x[b];
+            const RT a0 = al + xb * (et + xb * be), a1 = ep + xb * (de + xb * ze), a2 = ga + xb * th;
+            const RT b0 = s00 + xb * s10, b1 = s01 + xb * s11;
+#pragma unroll
+            for (int c = 0; c < NG; c++) {
+                const RT A = a0 + x[c] * (a1 + x[c] * a2), B = b0 + x[c] * b1;
+#pragma unroll
+                for (int a = 0; a < NG; a++) g[(b * NG + c) * NG + a] = A + x[a] * B;
+            }
+        }
+    }
+    // the transposed sums: coefficients of the points' values p
+    template <int NG> __device__ __forceinline__ void collect(const RT (&x)[NG], const RT* p)
+    {
+        al = be = ga = de = ep = ze = et = th = s00 = s10 = s01 = s11 = RT(0);
+#pragma unroll
+        for (int b = 0; b < NG; b++) {
+            RT r0 = RT(0), r1 = RT(0), r2 = RT(0), t0 = RT(0), t1 = RT(0);
+#pragma unroll
+            for (int c = 0; c < NG; c++) {
+                RT q0 = RT(0), q1 = RT(0);
+#pragma unroll
+                for (int a = 0; a < NG; a++) {
+                    const RT v = p[(b * NG + c) * NG + a];
+                    q0 += v;
+                    q1 += x[a] * v;
+                }
+                const RT cq = x[c] * q0;
+                r0 += q0, r1 += cq, r2 += x[c] * cq;
+                t0 += q1, t1 += x[c] * q1;
+            }
+            const RT xb = x[b], br0 = xb * r0, br1 = xb * r1;
+            al += r0, et += br0, be += xb * br0;
+            ep += r1, de += br1, ze += xb * br1;
+            ga += r2, th += xb * r2;
+            s00 += t0, s10 += xb * t0, s01 += t1, s11 += xb * t1;
+        }
+    }
+    // node contributions (the order of from_nodes)
+    __device__ __forceinline__ void to_nodes(RT (&v)[20]) const
+    {
+        const RT d00 = RT(0.125) * (be + ga - al), d11 = RT(0.125) * de, d01 = RT(0.125) * ze, d10 = RT(0.125) * th;
+        const RT q00 = RT(0.25) * s00, q10 = RT(0.25) * s10, q01 = RT(0.25) * s01, q11 = RT(0.25) * s11;
+#pragma unroll
+        for (int l = 0; l < 4; l++) {
+            const RT sb = (l & 1) ? RT(1) : RT(-1), sc = (l & 2) ? RT(1) : RT(-1);
+            const RT D = (d00 + sb * d10) + sc * (d01 + sb * d11), S = (q00 + sb * q10) + sc * (q01 + sb * q11);
+            v[3 * l] = S - D;
+            v[3 * l + 1] = S + D;
+            v[3 * l + 2] = RT(-2) * S;
+        }
+        const RT eb0 = RT(0.25) * (al - be), eb1 = RT(0.25) * (ep - ze);
+        const RT ec0 = RT(0.25) * (al - ga), ec1 = RT(0.25) * (et - th);
+        v[13] = eb0 - eb1, v[15] = eb0 + eb1, v[17] = ec0 - ec1, v[19] = ec0 + ec1;
+        v[12] = -v[13], v[14] = -v[15], v[16] = -v[17], v[18] = -v[19];
+    }
+};
+
+// P = inv . sigma at a point (w: |J|, weight and factor): H becomes P, [i][d]
+template <typename RT>
+__device__ __forceinline__ void h20_point(const RT (&inv)[3][3], RT w, RT (&H)[3][3], RT k1, RT k2, RT k3)
 {
-    return (64 / QP) * H20Lds<RT>::elem_row > 64 * kH20Slot ? (64 / QP) * H20Lds<RT>::elem_row : 64 * kH20Slot;
+    RT g[3][3], sg[3][3];
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int k = 0; k < 3; k++) g[i][k] = H[i][0] * inv[0][k] + H[i][1] * inv[1][k] + H[i][2] * inv[2][k];
+    const RT exx = g[0][0] * w, eyy = g[1][1] * w, ezz = g[2][2] * w;
+    sg[0][0] = k1 * exx + k2 * eyy + k2 * ezz;
+    sg[1][1] = k2 * exx + k1 * eyy + k2 * ezz;
+    sg[2][2] = k2 * exx + k2 * eyy + k1 * ezz;
+    sg[0][1] = sg[1][0] = (k3 * w) * (g[0][1] + g[1][0]);
+    sg[1][2] = sg[2][1] = (k3 * w) * (g[1][2] + g[2][1]);
+    sg[0][2] = sg[2][0] = (k3 * w) * (g[0][2] + g[2][0]);
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int d = 0; d < 3; d++) H[i][d] = inv[d][0] * sg[i][0] + inv[d][1] * sg[i][1] + inv[d][2] * sg[i][2];
 }
 
-template <int QP, typename RT, bool MASKED, bool ATOMIC, bool DIAG>
-__global__ __launch_bounds__(256) void free_hex20_kernel(const RT* __restrict__ xe, const double* __restrict__ scale,
-                                                        const uint32_t* __restrict__ map, const RT* __restrict__ u,
-                                                        RT* __restrict__ out, uint64_t ve_base, uint32_t rs,
-                                                        uint32_t ss, uint32_t slot_begin, uint32_t n_slots,
-                                                        const double* __restrict__ qp, uint32_t nq,
-                                                        double c1, double c2, double c3,
-                                                        const uint32_t* __restrict__ skip)
+// the derivatives of an element group's three fields at the points, from the
+// node values in W (overlaid)
+template <int NG, typename RT>
+__device__ __forceinline__ void h20_derivatives(RT* W, uint32_t lane, const RT (&x)[NG])
 {
-    using RT2 = typename Vec2<RT>::type;
-    constexpr int EW = 64 / QP, WD = h20_wave_values<QP, RT>();
-    constexpr int kTabRow = H20Lds<RT>::tab_row, kElemRow = H20Lds<RT>::elem_row, NS = H20Lds<RT>::node;
-    constexpr bool F32 = std::is_same<RT, float>::value;
-    __shared__ __align__(16) RT tab[QP * kTabRow];
-    __shared__ RT wq[QP];
-    __shared__ __align__(16) RT work[4][WD];
-    const RT k1 = (RT)c1, k2 = (RT)c2, k3 = (RT)c3;
-    if (skip && *skip) return;
-    for (uint32_t i = threadIdx.x; i < QP * 80u; i += blockDim.x) {
-        const uint32_t q = i / 80u, r = i - q * 80u, a = r >> 2, d = r & 3u;
-        tab[q * kTabRow + r] = d < 3 ? (RT)qp[q * 61u + 3u * a + d] : RT(0);
+    using T = H20<NG>;
+    const uint32_t t = min(lane, 9u * T::EW - 1u), e = t / 9u, r = t - 9u * e, f = r / 3u, d = r - 3u * f;
+    const char* in = reinterpret_cast<const char*>(W + e * T::IS + f * 20u);
+    RT v[20];
+#pragma unroll
+    for (int w = 0; w < 5; w++) {
+        const uint32_t pk = d == 0 ? kH20Node[0][w] : d == 1 ? kH20Node[1][w] : kH20Node[2][w];
+#pragma unroll
+        for (int b = 0; b < 4; b++)
+            v[4 * w + b] = *reinterpret_cast<const RT*>(in + ((pk >> (8 * b)) & 0xffu) * sizeof(RT) / 8u);
     }
-    for (uint32_t q = threadIdx.x; q < QP; q += blockDim.x) wq[q] = (RT)qp[q * 61u + 60u];
-    __syncthreads();
+    H20Coef<RT> co;
+    co.from_nodes(v);
+    lds_sync_wave();  // every lane's node values are read before the derivatives overlay them
+    if (lane < 9u * T::EW) co.template evaluate<NG>(x, W + t * T::TS);
+    lds_sync_wave();
+}
 
-    const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
-    RT* W = work[wv];
+// where point t of a group finds the derivatives of a field in direction d
+template <int NG> struct H20At {
+    uint32_t base, at[3];
+    __device__ __forceinline__ explicit H20At(uint32_t t)
+    {
+        const uint32_t e = t / H20<NG>::PTS, q = t - e * H20<NG>::PTS;
+        const uint32_t ix = q / (NG * NG), iy = q / NG % NG, iz = q % NG;
+        base = e * H20<NG>::GS;
+        at[0] = base + (iy * NG + iz) * NG + ix;
+        at[1] = base + (iz * NG + ix) * NG + iy;
+        at[2] = base + (ix * NG + iy) * NG + iz;
+    }
+};
+
+// rule: the NG points, then the NG weights, of the one-dimensional rule
+template <int NG, typename RT, bool MASKED, bool ATOMIC>
+__global__ __launch_bounds__(64, sizeof(RT) == 4 && NG <= 3 ? 4 : 1) void free_hex20_kernel(const RT* __restrict__ xe, const double* __restrict__ scale,
+                                                       const uint32_t* __restrict__ map, const RT* __restrict__ u,
+                                                       RT* __restrict__ out, uint64_t ve_base, uint32_t rs,
+                                                       uint32_t ss, uint32_t slot_begin, uint32_t n_slots,
+                                                       const double* __restrict__ rule, double c1, double c2,
+                                                       double c3, const uint32_t* __restrict__ skip)
+{
+    using T = H20<NG>;
+    constexpr int EW = T::EW, PTS = T::PTS, TS = T::TS;
+    __shared__ RT W[T::WAVE];
+    if (skip && *skip) return;
+    const RT k1 = (RT)c1, k2 = (RT)c2, k3 = (RT)c3;
+    RT x[NG], wq[T::P2];
+#pragma unroll
+    for (int i = 0; i < NG; i++) x[i] = (RT)rule[i];
+#pragma unroll
+    for (int j = 0; j < T::P2; j++) {
+        const uint32_t q = (threadIdx.x + 64u * j) % PTS;
+        wq[j] = (RT)(rule[NG + q % NG] * rule[NG + q / NG % NG] * rule[NG + q / (NG * NG)]);
+    }
     const uint32_t n_groups = (n_slots + EW - 1) / EW;
-    const uint32_t pa = lane < 60 ? lane / 3u : 19u, pi = lane < 60 ? lane - 3u * pa : 0u;
 
-    // the next group's coordinates, map entries, element values and factor are
+    // the next group's coordinates, map entries, node values and factors are
     // loaded into registers while the current group is computed: lane value j
     // is entry idx = lane + 64 j of the group's EW x 60 block
     constexpr int NL = (EW * 60 + 63) / 64;
-    RT px[NL], pu[NL], ps = RT(0);
+    RT px[NL], pu[NL], ps[T::P2];
     uint32_t pm[NL];
     auto issue = [&](uint32_t grp) {
-        const uint32_t first = grp * EW, n_here = min((uint32_t)EW, n_slots - first);
-        const uint64_t slot0 = (uint64_t)slot_begin + first;
+        const uint32_t lane = threadIdx.x, first = grp * EW, n_here = min((uint32_t)EW, n_slots - first);
+        const uint64_t src0 = ((uint64_t)slot_begin + first) * 60u;
+        // branch-free: entries past the group's elements repeat its last entry
+        const uint32_t last = n_here * 60u - 1u;
 #pragma unroll
         for (int j = 0; j < NL; j++) {
-            const uint32_t idx = lane + 64u * j, e = idx / 60u;
-            const bool ok = idx < EW * 60u && e < n_here;
-            // branch-free: entries outside the group load the group's first entry
-            const uint64_t src = (slot0 + (ok ? e : 0u)) * 60u + (ok ? idx - 60u * e : 0u);
-            const RT xv = (RT)xe[src];
-            const uint32_t mv = DIAG ? 0u : map[src];
-            px[j] = ok ? xv : RT(0);
-            pm[j] = ok ? mv : 0u;
+            const uint64_t src = src0 + min(lane + 64u * j, last);
+            px[j] = xe[src];
+            pm[j] = map[src];
         }
-        const uint32_t e = lane / QP;
-        const RT sv = (RT)scale[slot0 + min(e, n_here - 1u)];
-        ps = e < n_here ? sv : RT(0);
+#pragma unroll
+        for (int j = 0; j < T::P2; j++)
+            ps[j] = (RT)scale[(uint64_t)slot_begin + first + min((lane + 64u * j) / PTS, n_here - 1u)];
     };
     auto gather = [&]() {
 #pragma unroll
         for (int j = 0; j < NL; j++) {
-            RT v = RT(0);
-            if constexpr (!DIAG) {
-                v = u[pm[j] & kMask];  // entries outside the group read u[0]; their elements are not stored
-                if (MASKED && (pm[j] & kFlag)) v = RT(0);
-            }
+            RT v = u[pm[j] & kMask];
+            if (MASKED && (pm[j] & kFlag)) v = RT(0);
             pu[j] = v;
         }
     };
-
-    uint32_t grp = blockIdx.x * 4u + wv;  // uniform per wave
-    if (grp < n_groups) {
-        issue(grp);
-        gather();
-    }
-    for (; grp < n_groups; grp += gridDim.x * 4u) {
-        const uint32_t first = grp * EW;
-        const uint32_t n_here = min((uint32_t)EW, n_slots - first);
-        const uint64_t slot0 = (uint64_t)slot_begin + first;
-        const uint32_t next = grp + gridDim.x * 4u;
-
-        // element e's node a at W[e*kElemRow + NS a]: x y z, then u
+    // node values of the three fields, [element][field][node]
+    auto put = [&](uint32_t lane, const RT (&v)[NL]) {
 #pragma unroll
         for (int j = 0; j < NL; j++) {
             const uint32_t idx = lane + 64u * j;
             if (idx < EW * 60u) {
                 const uint32_t e = idx / 60u, r = idx - e * 60u, a = r / 3u, k = r - 3u * a;
-                W[e * kElemRow + NS * a + k] = px[j];
-                W[e * kElemRow + NS * a + 3u + k] = pu[j];
+                W[e * T::IS + k * 20u + a] = v[j];
             }
         }
-        const RT sc_here = ps;
         lds_sync_wave();
-        if (next < n_groups) issue(next);
+    };
 
-        // phase 1
-        {
-            const uint32_t e = lane / QP, q = lane % QP;
-            const RT* XU = W + e * kElemRow;
-            const RT* T = tab + q * kTabRow;
-            RT J[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}}, H[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
-#pragma unroll 4
-            for (int a = 0; a < 20; a++) {
-                RT dn[3], xs[3], us[3];
-                if constexpr (F32) {
-                    const float4 t4 = *reinterpret_cast<const float4*>(T + 4 * a);
-                    const float4 x4 = *reinterpret_cast<const float4*>(XU + 8 * a);
-                    dn[0] = t4.x, dn[1] = t4.y, dn[2] = t4.z;
-                    xs[0] = x4.x, xs[1] = x4.y, xs[2] = x4.z;
-                    us[0] = x4.w;
-                    if constexpr (!DIAG) {
-                        const float2 u2 = *reinterpret_cast<const float2*>(XU + 8 * a + 4);
-                        us[1] = u2.x, us[2] = u2.y;
-                    }
-                } else {
-                    const RT2 t01 = *reinterpret_cast<const RT2*>(T + 4 * a);
-                    const RT2 p0 = *reinterpret_cast<const RT2*>(XU + 6 * a);
-                    const RT2 p1 = *reinterpret_cast<const RT2*>(XU + 6 * a + 2);
-                    dn[0] = t01.x, dn[1] = t01.y, dn[2] = T[4 * a + 2];
-                    xs[0] = p0.x, xs[1] = p0.y, xs[2] = p1.x;
-                    us[0] = p1.y;
-                    if constexpr (!DIAG) {
-                        const RT2 p2 = *reinterpret_cast<const RT2*>(XU + 6 * a + 4);
-                        us[1] = p2.x, us[2] = p2.y;
-                    }
-                }
+    uint32_t base = 0, grp = xcd_block(blockIdx.x, gridDim.x);  // consecutive groups on one XCD
+    if (grp < n_groups) {
+        issue(grp);
+        gather();
+    }
+    for (; grp < n_groups; base += gridDim.x, grp = base + xcd_block(blockIdx.x, gridDim.x)) {
+        const uint32_t first = grp * EW, n_here = min((uint32_t)EW, n_slots - first);
+        const uint32_t next = base + gridDim.x + xcd_block(blockIdx.x, gridDim.x);
+        // the lane's LDS addresses are formed anew for every group: kept over the
+        // loop they take 80 registers, and with them a third of the waves
+        uint32_t lane = threadIdx.x;
+        asm volatile("" : "+v"(lane));
+        put(lane, px);
+        h20_derivatives<NG, RT>(W, lane, x);
+        RT inv[T::P2][3][3], w[T::P2];
 #pragma unroll
-                for (int k = 0; k < 3; k++)
+        for (int j = 0; j < T::P2; j++) {
+            const H20At<NG> g(min(lane + 64u * j, (uint32_t)EW * PTS - 1u));
+            RT J[3][3];
 #pragma unroll
-                    for (int d = 0; d < 3; d++) J[k][d] += xs[k] * dn[d];
-                if constexpr (!DIAG) {
+            for (int k = 0; k < 3; k++)
 #pragma unroll
-                    for (int k = 0; k < 3; k++)
+                for (int d = 0; d < 3; d++) J[k][d] = W[g.at[d] + (3 * k + d) * TS];
+            w[j] = jac_inv_r(J, inv[j]) * wq[j] * ps[j];
+        }
+        lds_sync_wave();
+        put(lane, pu);
+        if (next < n_groups) issue(next);
+        h20_derivatives<NG, RT>(W, lane, x);
 #pragma unroll
-                        for (int d = 0; d < 3; d++) H[k][d] += us[k] * dn[d];
-                }
-            }
-            RT inv[3][3];
-            const RT det = jac_inv_r(J, inv);
-            RT w = e < n_here ? det * wq[q] * sc_here : RT(0);
-            // DIAG: a non-positive Jacobian at a real point marks the element (NaN diagonal)
-            if (DIAG && e < n_here && q < nq && !(det > RT(0))) w = (RT)__builtin_nan("");
-            RT S[kH20Slot];
-            if constexpr (DIAG) {
+        for (int j = 0; j < T::P2; j++) {
+            const uint32_t t = lane + 64u * j;
+            const H20At<NG> g(min(t, (uint32_t)EW * PTS - 1u));
+            RT H[3][3];
 #pragma unroll
-                for (int k = 0; k < 3; k++)
+            for (int i = 0; i < 3; i++)
 #pragma unroll
-                    for (int d = 0; d < 3; d++) S[4 * k + d] = inv[d][k];
-            } else {
-                RT g[3][3];  // g[i][k] = du_i/dx_k
+                for (int d = 0; d < 3; d++) H[i][d] = W[g.at[d] + (3 * i + d) * TS];
+            h20_point<RT>(inv[j], w[j], H, k1, k2, k3);
+            if (t < (uint32_t)EW * PTS) {
 #pragma unroll
                 for (int i = 0; i < 3; i++)
 #pragma unroll
-                    for (int k = 0; k < 3; k++)
-                        g[i][k] = H[i][0] * inv[0][k] + H[i][1] * inv[1][k] + H[i][2] * inv[2][k];
-                const RT exx = g[0][0] * w, eyy = g[1][1] * w, ezz = g[2][2] * w;
-                RT sg[3][3];
-                sg[0][0] = k1 * exx + k2 * eyy + k2 * ezz;
-                sg[1][1] = k2 * exx + k1 * eyy + k2 * ezz;
-                sg[2][2] = k2 * exx + k2 * eyy + k1 * ezz;
-                sg[0][1] = sg[1][0] = (k3 * w) * (g[0][1] + g[1][0]);
-                sg[1][2] = sg[2][1] = (k3 * w) * (g[1][2] + g[2][1]);
-                sg[0][2] = sg[2][0] = (k3 * w) * (g[0][2] + g[2][0]);
-#pragma unroll
-                for (int i = 0; i < 3; i++)
-#pragma unroll
-                    for (int d = 0; d < 3; d++)
-                        S[4 * i + d] = inv[d][0] * sg[i][0] + inv[d][1] * sg[i][1] + inv[d][2] * sg[i][2];
+                    for (int d = 0; d < 3; d++) W[g.at[d] + (3 * i + d) * TS] = H[i][d];
             }
-            S[3] = w;
-            S[7] = S[11] = RT(0);
-            lds_sync_wave();  // every lane's reads of the node values precede the slot writes that overlay them
-            RT* slotp = W + lane * kH20Slot;
-#pragma unroll
-            for (int j = 0; j < kH20Slot; j += 2) *reinterpret_cast<RT2*>(slotp + j) = Vec2<RT>::make(S[j], S[j + 1]);
         }
         lds_sync_wave();
         if (next < n_groups) gather();
+        {
+            const uint32_t t = min(lane, 9u * EW - 1u), e = t / 9u, r = t - 9u * e, i = r / 3u, d = r - 3u * i;
+            H20Coef<RT> co;
+            co.template collect<NG>(x, W + t * TS);
+            lds_sync_wave();  // every lane's reads of P precede the contributions that overlay it
+            RT v[20];
+            co.to_nodes(v);
+            char* o = reinterpret_cast<char*>(W + e * T::CS + d * 60u + i);
+            if (lane < 9u * EW) {
+#pragma unroll
+                for (int k = 0; k < 5; k++) {
+                    const uint32_t pk = d == 0 ? kH20Node[0][k] : d == 1 ? kH20Node[1][k] : kH20Node[2][k];
+#pragma unroll
+                    for (int b = 0; b < 4; b++)
+                        *reinterpret_cast<RT*>(o + ((pk >> (8 * b)) & 0xffu) * 3u * sizeof(RT) / 8u) = v[4 * k + b];
+                }
+            }
+        }
+        lds_sync_wave();
+#pragma unroll
+        for (int j = 0; j < NL; j++) {
+            const uint32_t idx = lane + 64u * j, e = idx / 60u, r = idx - e * 60u;
+            if (idx < n_here * 60u) {
+                const RT* c = W + e * T::CS + r;
+                const RT f = c[0] + c[60] + c[120];
+                const uint64_t slot = (uint64_t)slot_begin + first + e;
+                if constexpr (ATOMIC) unsafeAtomicAdd(&out[map[slot * 60u + r] & kMask], f);
+                else out[ve_base + (uint64_t)r * rs + slot * ss] = f;
+            }
+        }
+        lds_sync_wave();  // the contributions are read before the next group's node values
+    }
+}
 
-        // phase 2: f[e] = sum_q dN_q(a) . P_q(:, i) of element e
-        RT f[EW];
-#pragma unroll
-        for (int e = 0; e < EW; e++) f[e] = RT(0);
-        auto point = [&](uint32_t e, uint32_t q, RT d0, RT d1, RT d2) {
-            const RT* S = W + (e * QP + q) * kH20Slot;
-            if constexpr (DIAG) {
-                RT g[3];
-#pragma unroll
-                for (int k = 0; k < 3; k++) g[k] = d0 * S[4 * k] + d1 * S[4 * k + 1] + d2 * S[4 * k + 2];
-                const RT gi = pi == 0 ? g[0] : (pi == 1 ? g[1] : g[2]);
-                const RT gg = g[0] * g[0] + g[1] * g[1] + g[2] * g[2];
-                f[e] += (k1 * gi * gi + k3 * (gg - gi * gi)) * S[3];
-            } else {
-                if constexpr (F32) {
-                    const float4 p4 = *reinterpret_cast<const float4*>(S + 4 * pi);
-                    f[e] += d0 * p4.x + d1 * p4.y + d2 * p4.z;
-                } else {
-                    const RT2 p01 = *reinterpret_cast<const RT2*>(S + 4 * pi);
-                    const RT p2 = S[4 * pi + 2];
-                    f[e] += d0 * p01.x + d1 * p01.y + d2 * p2;
-                }
-            }
-        };
+// diag(s_e K_e) of hex20 elements: lane l = e*QP + q of a wave holds element e at
+// point q and leaves inv and w in LDS, then lane 3a+i sums the points.  qp:
+// [nq][61] (dN_ad at 3a+d, weight).  Set-up only.
+template <int QP>
+__global__ __launch_bounds__(64) void free_hex20_diag_kernel(const double* __restrict__ xe,
+                                                            const double* __restrict__ scale,
+                                                            double* __restrict__ out, uint64_t ve_base, uint32_t rs,
+                                                            uint32_t ss, uint32_t n_slots,
+                                                            const double* __restrict__ qp, uint32_t nq, double c1,
+                                                            double c3)
+{
+    constexpr int EW = 64 / QP;
+    __shared__ double S[64][11];  // inv[d][k] at 3k + d, w at 9 (odd row stride)
+    const uint32_t lane = threadIdx.x, slot0 = blockIdx.x * EW;
+    {
+        const uint32_t e = lane / QP, q = lane % QP, slot = min(slot0 + e, n_slots - 1u);
+        const double* t = qp + (uint64_t)q * 61u;  // padded with rows of weight 0
+        double J[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}}, inv[3][3];
+        for (int a = 0; a < 20; a++)
+            for (int k = 0; k < 3; k++)
+                for (int d = 0; d < 3; d++) J[k][d] += xe[(uint64_t)slot * 60u + 3 * a + k] * t[3 * a + d];
+        const double det = jac_inv_r(J, inv);
+        double w = det * t[60] * scale[slot];
+        // a non-positive Jacobian at a real point marks the element (NaN diagonal)
+        if (q < nq && !(det > 0.0)) w = __builtin_nan("");
+        for (int k = 0; k < 3; k++)
+            for (int d = 0; d < 3; d++) S[lane][3 * k + d] = inv[d][k];
+        S[lane][9] = w;
+    }
+    lds_sync_wave();
+    if (lane >= 60u) return;
+    const uint32_t a = lane / 3u, i = lane - 3u * a;
+    for (uint32_t e = 0; e < EW && slot0 + e < n_slots; e++) {
+        double f = 0.0;
         for (uint32_t q = 0; q < nq; q++) {
-            RT t0, t1, t2;
-            if constexpr (F32) {
-                const float4 t4 = *reinterpret_cast<const float4*>(tab + q * kTabRow + 4 * pa);
-                t0 = t4.x, t1 = t4.y, t2 = t4.z;
-            } else {
-                const RT2 t01 = *reinterpret_cast<const RT2*>(tab + q * kTabRow + 4 * pa);
-                t0 = t01.x, t1 = t01.y, t2 = tab[q * kTabRow + 4 * pa + 2];
-            }
-#pragma unroll
-            for (uint32_t e = 0; e < EW; e++) point(e, q, t0, t1, t2);
+            const double* t = qp + (uint64_t)q * 61u + 3u * a;
+            const double* s = S[e * QP + q];
+            double g[3];
+            for (int k = 0; k < 3; k++) g[k] = t[0] * s[3 * k] + t[1] * s[3 * k + 1] + t[2] * s[3 * k + 2];
+            const double gi = i == 0 ? g[0] : (i == 1 ? g[1] : g[2]);
+            const double gg = g[0] * g[0] + g[1] * g[1] + g[2] * g[2];
+            f += (c1 * gi * gi + c3 * (gg - gi * gi)) * s[9];
         }
-        if (lane < 60) {
-#pragma unroll
-            for (uint32_t e = 0; e < EW; e++) {
-                if (e < n_here) {
-                    const uint64_t slot = slot0 + e;
-                    if constexpr (ATOMIC) unsafeAtomicAdd(&out[map[slot * 60u + lane] & kMask], f[e]);
-                    else out[ve_base + (uint64_t)lane * rs + slot * ss] = f[e];
-                }
-            }
-        }
-        lds_sync_wave();  // phase-2 reads of the slots precede the next group's node writes
+        out[ve_base + (uint64_t)lane * rs + (uint64_t)(slot0 + e) * ss] = f;
     }
 }
 
@@ -419,11 +559,10 @@ template <typename RT> const RT* coords(const FreeArgs& a)
     }
 }
 
-template <int QP, typename RT>
-void launch_hex20(bool masked, bool atomic, bool diag, const FreeArgs& a, hipStream_t s)
+template <int NG, typename RT> void launch_hex20(bool masked, bool atomic, const FreeArgs& a, hipStream_t s)
 {
-    constexpr uint32_t per_block = 4u * (64u / QP);
-    // resident blocks per device: CUs x blocks per CU (the LDS bounds it); a
+    constexpr uint32_t EW = H20<NG>::EW;
+    // resident waves per device: CUs x blocks per CU (the LDS bounds it); a
     // benign race between threads computes the same value
     static std::atomic<int> resident[kMaxDevices];
     int dev = 0;
@@ -433,29 +572,30 @@ void launch_hex20(bool masked, bool atomic, bool diag, const FreeArgs& a, hipStr
     if (res == 0) {
         int cus = 0, per_cu = 0;
         AMX_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-        AMX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, free_hex20_kernel<QP, RT, false, false, false>,
-                                                             256, 0));
+        AMX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, free_hex20_kernel<NG, RT, false, false>, 64, 0));
         res = std::max(1, cus * std::max(per_cu, 1));
         resident[dev].store(res, std::memory_order_relaxed);
     }
-    const uint32_t need = (a.n_slots + per_block - 1) / per_block;
-    const dim3 grid(std::min<uint32_t>(need, (uint32_t)res)), block(256);
+    const uint32_t need = (a.n_slots + EW - 1) / EW;
+    const dim3 grid(std::min<uint32_t>(need, (uint32_t)res)), block(64);
     const RT* x = coords<RT>(a);
     const RT* u = static_cast<const RT*>(a.u);
     RT* out = static_cast<RT*>(a.out);
-#define AMX_H20(M, A, D)                                                                                           \
-    free_hex20_kernel<QP, RT, M, A, D><<<grid, block, 0, s>>>(x, a.scale, a.map, u, out, a.ve_base, a.ve_rs,     \
-                                                              a.ve_ss, a.slot_begin, a.n_slots, a.qp, a.nq, a.c1,   \
-                                                              a.c2, a.c3, a.skip)
-    if constexpr (std::is_same<RT, double>::value) {
-        if (diag) {
-            AMX_H20(false, false, true);
-            return;
-        }
-    }
-    if (masked) { if (atomic) AMX_H20(true, true, false); else AMX_H20(true, false, false); }
-    else { if (atomic) AMX_H20(false, true, false); else AMX_H20(false, false, false); }
+#define AMX_H20(M, A)                                                                                              \
+    free_hex20_kernel<NG, RT, M, A><<<grid, block, 0, s>>>(x, a.scale, a.map, u, out, a.ve_base, a.ve_rs, a.ve_ss,  \
+                                                           a.slot_begin, a.n_slots, a.rule, a.c1, a.c2, a.c3,       \
+                                                           a.skip)
+    if (masked) { if (atomic) AMX_H20(true, true); else AMX_H20(true, false); }
+    else { if (atomic) AMX_H20(false, true); else AMX_H20(false, false); }
 #undef AMX_H20
+}
+
+template <int QP> void launch_hex20_diag(const FreeArgs& a, hipStream_t s)
+{
+    AMX_REQUIRE(a.slot_begin == 0, AMX_INVALID_STATE, "the diagonal covers every slot");
+    constexpr uint32_t EW = 64 / QP;
+    free_hex20_diag_kernel<QP><<<(a.n_slots + EW - 1) / EW, 64, 0, s>>>(
+        a.xe, a.scale, static_cast<double*>(a.out), a.ve_base, a.ve_rs, a.ve_ss, a.n_slots, a.qp, a.nq, a.c1, a.c3);
 }
 
 template <int NN, typename RT>
@@ -488,10 +628,20 @@ void launch_free_t(int kind, bool masked, bool atomic, bool diag, const FreeArgs
     case AMX_ELEM_TET10_LAPLACE: launch_laplace<10, RT>(masked, atomic, diag, a, s); break;
     case AMX_ELEM_HEX20_ELASTIC: {
         AMX_REQUIRE(a.nq <= 64, AMX_NOT_IMPLEMENTED, "hex20: at most 64 quadrature points");
-        const uint32_t qp = free_padded_points(kind, a.nq);
-        if (qp == 8) launch_hex20<8, RT>(masked, atomic, diag, a, s);
-        else if (qp == 32) launch_hex20<32, RT>(masked, atomic, diag, a, s);
-        else launch_hex20<64, RT>(masked, atomic, diag, a, s);
+        if (diag) {
+            const uint32_t qp = free_padded_points(kind, a.nq);
+            if (qp == 8) launch_hex20_diag<8>(a, s);
+            else if (qp == 32) launch_hex20_diag<32>(a, s);
+            else launch_hex20_diag<64>(a, s);
+        } else if (a.nq == 1) {
+            launch_hex20<1, RT>(masked, atomic, a, s);
+        } else if (a.nq == 8) {
+            launch_hex20<2, RT>(masked, atomic, a, s);
+        } else if (a.nq == 27) {
+            launch_hex20<3, RT>(masked, atomic, a, s);
+        } else {
+            launch_hex20<4, RT>(masked, atomic, a, s);
+        }
         break;
     }
     default: fail(AMX_INVALID_ARGUMENT, "unknown element kind " + std::to_string(kind));

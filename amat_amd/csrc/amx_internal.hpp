@@ -91,6 +91,8 @@ struct DevBuf {
 // quadrature table of the FREE element kernels (amx_fem.cpp): nq points of
 // [dN/dxi per node (3 each), weight], padded with zero-weight rows to rows_min
 std::vector<double> free_quadrature(int kind, uint32_t ngt, uint32_t& nq, uint32_t rows_min);
+// the Gauss-Legendre rule of those tables: ngt points, then ngt weights
+std::vector<double> gauss_rule(uint32_t ngt);
 
 }  // namespace amx
 

@@ -89,6 +89,7 @@ FreeArgs free_args(const Op& op, const Group& g, const void* u, void* out, uint3
     a.stride = g.n_slots;
     a.qp = op.qp.as<double>();
     a.nq = op.elem_nq;
+    a.rule = a.qp + op.rule_at;
     a.c1 = op.elem_c[0];
     a.c2 = op.elem_c[1];
     a.c3 = op.elem_c[2];
@@ -187,8 +188,11 @@ void finalize_op(Op& op)
         AMX_REQUIRE(op.elem_kind != 0, AMX_INVALID_STATE, "method 2 (FREE) needs set_element_function before finalize");
         AMX_REQUIRE(!op.has(AMX_PREC_BF16), AMX_NOT_IMPLEMENTED, "method 2 (FREE) has no BF16 form");
         uint32_t nq = 0;
-        const std::vector<double> tab =
+        std::vector<double> tab =
             free_quadrature(op.elem_kind, op.elem_ngt, nq, free_padded_points(op.elem_kind, op.elem_nq));
+        op.rule_at = tab.size();
+        const std::vector<double> rule = gauss_rule(op.elem_ngt);
+        tab.insert(tab.end(), rule.begin(), rule.end());
         upload(op.qp, tab, s, op.device_bytes);
         AMX_HIP(hipStreamSynchronize(s));
     }

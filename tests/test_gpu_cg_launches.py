@@ -5,8 +5,9 @@ On elements that share no DoF the atomic scatter is exact too (one addition
 into a zeroed row), and its CG forms p . q in a pass of its own; so the
 deterministic CG, whose gather forms it, has to return the same bits: sizes at
 the edges of a block's 256 and 1,024 elements, of a group of 32 blocks, of the
-largest grid with four runs per block, and past it (both CGs then make the
-separate pass).
+size up to which a solve alone has the gather form it (65,536 DoFs), and past
+the largest one of served jobs (1,048,576; both CGs then make the separate
+pass).
 """
 import numpy as np
 import pytest
@@ -51,7 +52,7 @@ def solve(torch, op, b, method=None, max_it=10000):
     return dx.cpu().numpy(), st
 
 
-@pytest.mark.parametrize("E", [1, 32, 33, 128, 129, 4096, 4097, 131072, 131073])
+@pytest.mark.parametrize("E", [1, 32, 33, 128, 129, 4096, 4097, 8192, 8193, 131072, 131073])
 def test_gather_forms_the_dot_product(torch_gpu, E):
     N = E * NB
     gmap = np.arange(N).reshape(E, NB)
@@ -64,7 +65,7 @@ def test_gather_forms_the_dot_product(torch_gpu, E):
         np.testing.assert_array_equal(x, y)
 
 
-@pytest.mark.parametrize("E", [33, 4097, 131073])
+@pytest.mark.parametrize("E", [33, 4097, 8193, 131072, 131073])
 def test_served_and_mixed_precision(torch_gpu, E):
     """Reliable updates: the recurrence stops on the device in the launch that
     updates the direction; served and single solves agree bit for bit."""
