@@ -39,6 +39,7 @@ SOURCES = [
     "amx_cong.hip",
     "amx_solver_kernels.hip",
     "amx_mrhs.hip",
+    "amx_mrhs_cong.hip",
     "amx_free.hip",
     "amx_noalloc.hip",
 ]

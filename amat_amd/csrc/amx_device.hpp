@@ -98,4 +98,11 @@ __device__ __forceinline__ void block_totals(const double* part, uint32_t nblk, 
     }
 }
 
+__device__ __forceinline__ void lds_sync_wave()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 }  // namespace amx

@@ -39,13 +39,6 @@ namespace {
 constexpr uint32_t kFlag = 0x80000000u, kMask = 0x7fffffffu;
 constexpr int kMaxDevices = 64;
 
-__device__ __forceinline__ void lds_sync_wave()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // det J and inv[d][k] = cofactor(J)[k][d] / det (cofactors as in the host
 // element routines, amx_fem.cpp jacobian; one division)
 template <typename RT> __device__ __forceinline__ RT jac_inv_r(const RT J[3][3], RT inv[3][3])

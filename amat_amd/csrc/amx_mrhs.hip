@@ -13,6 +13,8 @@
 // per lane.  Smaller elements are packed block-diagonally, G = 32/n elements per
 // 32-row tile (4 hex8), from per-element matrices (FP32 column-major, BF16
 // row-major with 8-aligned rows); the off-diagonal zeros are never stored.
+// Congruent groups of 60 DoFs (K_e = s_e K_ref) take no matrices and have a
+// kernel of their own (amx_mrhs_cong.hip).
 // The element rows reach V either through the deterministic two-pass scatter
 // (rows stored per element, then summed per DoF in ascending element order:
 // bit-reproducible, independent of the launch shape) or FP32 atomics.
@@ -26,6 +28,7 @@
 #include <cstring>
 #include <vector>
 
+#include "amx_mrhs.hpp"
 #include "amx_nsym.hpp"
 #include "amx_op.hpp"
 
@@ -511,69 +514,70 @@ __global__ __launch_bounds__(256) void mrhs_persistent(SegTable tab)
     }
 }
 
-__global__ void zero_f32(float* p, uint64_t n)
+// what the launches over all parts take: out rows of each part
+struct OutSeg {
+    const uint32_t *ids, *off, *pos;  // ids: the DoFs that off and pos list (NULL: all)
+    const float* ve;
+    float* V;
+    uint64_t block0;  // first block of the part
+    uint32_t n_out;   // DoFs
+    uint32_t cols;    // columns per thread: 4, 2 or 1 (nrhs a multiple of it, V and ve aligned)
+};
+struct OutTable {
+    OutSeg s[kMaxSeg];
+    uint32_t n_seg, nrhs;
+};
+__device__ __forceinline__ const OutSeg& out_seg(const OutTable& t, uint64_t& i)
 {
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0.0f;
+    uint32_t k = 0;
+    while (k + 1 < t.n_seg && blockIdx.x >= t.s[k + 1].block0) k++;
+    i = (blockIdx.x - t.s[k].block0) * blockDim.x + threadIdx.x;
+    return t.s[k];
 }
 
-// deterministic scatter, second pass: V[d][c] = sum over d's element rows (fixed
-// order: ascending element, then row) of ve[row][c]
-__global__ __launch_bounds__(256) void mrhs_gather_kernel(const uint32_t* __restrict__ off,
-                                                         const uint32_t* __restrict__ pos, const float* __restrict__ ve,
-                                                         float* __restrict__ V, uint32_t n_total, uint32_t nrhs)
+__global__ __launch_bounds__(256) void mrhs_zero_kernel(OutTable t)
 {
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (uint64_t)n_total * nrhs) return;
-    const uint32_t d = (uint32_t)(i / nrhs), c = (uint32_t)(i - (uint64_t)d * nrhs);
-    const uint32_t b = off[d], cnt = off[d + 1] - b;
-    float s = 0.0f;
-    // chunks of 8 entries: index loads, then row loads, in flight together;
-    // the sum keeps the list order (entries past the end are not added)
+    uint64_t i;
+    const OutSeg& g = out_seg(t, i);
+    if (i < (uint64_t)g.n_out * t.nrhs) g.V[i] = 0.0f;
+}
+
+// one entry of V: the sum over its rows of ve in the order of the list.
+// Chunks of 8 entries: index loads, then row loads, in flight together;
+// entries past the end are not added.
+template <typename T>
+__device__ __forceinline__ void gather_one(const OutSeg& g, uint64_t i, uint32_t row)
+{
+    const T* ve = reinterpret_cast<const T*>(g.ve);
+    const uint32_t d = (uint32_t)(i / row), c = (uint32_t)(i - (uint64_t)d * row);
+    const uint32_t b = g.off[d], cnt = g.off[d + 1] - b;
+    T s = T(0.0f);
     for (uint32_t q0 = 0; q0 < cnt; q0 += 8) {
         uint32_t p[8];
-        float x[8];
+        T x[8];
 #pragma unroll
-        for (uint32_t j = 0; j < 8; j++) p[j] = pos[b + min(q0 + j, cnt - 1)];
+        for (uint32_t j = 0; j < 8; j++) p[j] = g.pos[b + min(q0 + j, cnt - 1)];
 #pragma unroll
-        for (uint32_t j = 0; j < 8; j++) x[j] = ve[(uint64_t)p[j] * nrhs + c];
+        for (uint32_t j = 0; j < 8; j++) x[j] = ve[(uint64_t)p[j] * row + c];
 #pragma unroll
         for (uint32_t j = 0; j < 8; j++)
             if (q0 + j < cnt) s += x[j];
     }
-    V[i] = s;
+    reinterpret_cast<T*>(g.V)[g.ids ? (uint64_t)g.ids[d] * row + c : i] = s;
 }
 
-// the same sums, four columns per thread (nrhs a multiple of 4, 16-byte
-// aligned rows): one 16-byte load per entry; each column's sum keeps the order
-// of mrhs_gather_kernel, so the results are the same bits
-__global__ __launch_bounds__(256) void mrhs_gather4_kernel(const uint32_t* __restrict__ off,
-                                                          const uint32_t* __restrict__ pos,
-                                                          const float4* __restrict__ ve, float4* __restrict__ V,
-                                                          uint32_t n_total, uint32_t nq)
+// second pass of the scatter, all parts: V[d][c] = sum over d's rows of ve
+// (fixed order: ascending element, then row; of a congruent group ascending
+// cluster) of ve[row][c].  Two or four columns per thread where the rows allow it:
+// each column's sum keeps the order, so the results are the same bits.
+__global__ __launch_bounds__(256) void mrhs_gather_kernel(OutTable t)
 {
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (uint64_t)n_total * nq) return;
-    const uint32_t d = (uint32_t)(i / nq), c = (uint32_t)(i - (uint64_t)d * nq);
-    const uint32_t b = off[d], cnt = off[d + 1] - b;
-    float4 s = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    for (uint32_t q0 = 0; q0 < cnt; q0 += 8) {
-        uint32_t p[8];
-        float4 x[8];
-#pragma unroll
-        for (uint32_t j = 0; j < 8; j++) p[j] = pos[b + min(q0 + j, cnt - 1)];
-#pragma unroll
-        for (uint32_t j = 0; j < 8; j++) x[j] = ve[(uint64_t)p[j] * nq + c];
-#pragma unroll
-        for (uint32_t j = 0; j < 8; j++)
-            if (q0 + j < cnt) {
-                s.x += x[j].x;
-                s.y += x[j].y;
-                s.z += x[j].z;
-                s.w += x[j].w;
-            }
-    }
-    V[i] = s;
+    uint64_t i;
+    const OutSeg& g = out_seg(t, i);
+    if (i >= (uint64_t)g.n_out * (t.nrhs / g.cols)) return;
+    if (g.cols == 4) gather_one<f32x4>(g, i, t.nrhs / 4);
+    else if (g.cols == 2) gather_one<f32x2>(g, i, t.nrhs / 2);
+    else gather_one<float>(g, i, t.nrhs);
 }
 
 // element matrices for the MFMA kernels from the tiled FP64 storage:
@@ -637,6 +641,12 @@ struct amx_mrhs {
         uint32_t n, n_elem, n_tiles, n_total;
         uint64_t ve_row0;        // first element row of this part in ve
         DevBuf K, dofs, off, pos;  // off/pos: DoF -> element rows (e*n + r), ascending
+        uint64_t ve_rows;          // rows of this part in ve
+        // congruent 60-DoF groups (amx_mrhs_cong.hip): no K; dofs, off and pos in
+        // the order of the clusters, off and pos of the DoFs ids only
+        bool cong = false;
+        uint32_t n_clusters = 0, max_rows = 0, n_ids = 0;
+        DevBuf kref, scale, slots, clusters, row_dof, direct, ids;
     };
     std::vector<Part> parts;
     hipGraph_t graph = nullptr;
@@ -672,26 +682,98 @@ void launch_persistent(amx_mrhs& m, const SegTable& tab, uint64_t max_slice, hip
     mrhs_persistent<B, T><<<dim3(nbx * kXcd), dim3(64 * m.wpb), 0, s>>>(tab);
 }
 
+template <typename T> void put(DevBuf& b, const std::vector<T>& v)
+{
+    b.alloc(std::max<size_t>(v.size(), 1) * sizeof(T));
+    if (!v.empty()) AMX_HIP(hipMemcpy(b.p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
+}
+
+// the tables of a congruent 60-DoF group, elements in slot order
+void create_cong(const Op& op, const Group& g, const std::vector<uint32_t>& slot_of, bool bf16, amx_mrhs::Part& p)
+{
+    std::vector<uint32_t> em((size_t)p.n_elem * g.n);
+    for (uint32_t j = 0; j < p.n_elem; j++) {
+        const uint32_t* d = &op.local_map[op.eoff[g.elems[g.slot_elem[slot_of[j]]]]];
+        std::copy(d, d + g.n, em.begin() + (size_t)j * g.n);
+    }
+    const MrhsClusters c = mrhs_clusters(em, p.n_elem, p.n_total, bf16);
+    std::vector<double> scale(p.n_elem);
+    for (uint32_t j = 0; j < p.n_elem; j++) scale[j] = op.scale[g.elems[g.slot_elem[slot_of[c.order[j]]]]];
+    p.ve_rows = c.row_dof.size();
+    p.n_clusters = (uint32_t)c.table.size() / 4 - 1;
+    p.max_rows = c.max_rows;
+    p.n_ids = (uint32_t)c.ids.size();
+    put(p.kref, mrhs_kref(op.kref, bf16));
+    std::vector<float> sf;
+    for (double x : scale) {
+        sf.push_back((float)x);
+        if (bf16) sf.push_back((float)(x - (double)(float)x));
+    }
+    put(p.scale, sf);
+    put(p.dofs, c.dofs);
+    put(p.slots, c.slots);
+    put(p.clusters, c.table);
+    put(p.row_dof, c.row_dof);
+    put(p.direct, c.direct);
+    put(p.ids, c.ids);
+    put(p.off, c.off);
+    put(p.pos, c.pos);
+}
+
+uint64_t ve_bytes(const amx_mrhs& m, int nrhs)
+{
+    uint64_t rows = 0;
+    for (auto& p : m.parts) rows += p.ve_rows;
+    return rows * (uint64_t)nrhs * 4;
+}
+
+// The atomic scatter may sum in any order, so it takes the deterministic one's
+// two passes where their buffer is no burden: 24 columns in BF16 on 31^3 hex20 +
+// 80 x 40 x 20 hex8 246 -> 165 us, 64 in FP32 on 24^3 hex20 + 20^3 hex8 189 ->
+// 130 us.  Above, whoever asked for atomics keeps the memory.
+constexpr uint64_t kAtomicVeBytes = 2ull << 30;
+bool two_pass(const amx_mrhs& m, int nrhs)
+{
+    return m.scatter == AMX_SCATTER_DETERMINISTIC || ve_bytes(m, nrhs) <= kAtomicVeBytes;
+}
+
 // element-row buffer of the deterministic scatter (allocated outside launches,
 // so a captured graph never allocates)
 void prepare(amx_mrhs& m, int nrhs)
 {
-    if (m.scatter != AMX_SCATTER_DETERMINISTIC) return;
-    uint64_t rows = 0;
-    for (auto& p : m.parts) rows += (uint64_t)p.n_elem * p.n;
-    const uint64_t bytes = std::max<uint64_t>(rows * (uint64_t)nrhs * 4, 4);
+    if (!two_pass(m, nrhs)) return;
+    const uint64_t bytes = std::max<uint64_t>(ve_bytes(m, nrhs), 4);
     if (m.ve.bytes < bytes) m.ve.alloc(bytes);
 }
+
+// one launch over the parts, or several where their threads pass 32 bits
+struct OutLaunch {
+    void (*kernel)(OutTable);
+    OutTable t{};
+    uint64_t blocks = 0;
+    hipStream_t s;
+    void add(OutSeg g, uint64_t threads)
+    {
+        const uint64_t n = (threads + 255) / 256;
+        if (!n) return;
+        if (blocks + n >= 1u << 24) run();
+        g.block0 = blocks;
+        t.s[t.n_seg++] = g;
+        blocks += n;
+    }
+    void run()
+    {
+        if (blocks) kernel<<<(uint32_t)blocks, 256, 0, s>>>(t);
+        blocks = t.n_seg = 0;
+    }
+    OutLaunch(void (*k)(OutTable), int nrhs, hipStream_t stream) : kernel(k), s(stream) { t.nrhs = (uint32_t)nrhs; }
+};
 
 void launch(amx_mrhs& m, int nrhs, const float* const* U, float* const* V, hipStream_t s)
 {
     SegTable tab{};
-    const bool det = m.scatter == AMX_SCATTER_DETERMINISTIC;
-    if (det) {
-        uint64_t rows = 0;
-        for (auto& p : m.parts) rows += (uint64_t)p.n_elem * p.n;
-        AMX_REQUIRE(m.ve.bytes >= rows * (uint64_t)nrhs * 4, AMX_INVALID_STATE, "element-row buffer not prepared");
-    }
+    const bool det = two_pass(m, nrhs);
+    if (det) AMX_REQUIRE(m.ve.bytes >= ve_bytes(m, nrhs), AMX_INVALID_STATE, "element-row buffer not prepared");
     AMX_REQUIRE(m.parts.size() <= (size_t)kMaxSeg, AMX_NOT_IMPLEMENTED, "too many element groups in one launch");
     const int NT = m.rhs_tile / 32;
     const uint32_t ngroups = (uint32_t)((nrhs + m.rhs_tile - 1) / m.rhs_tile);
@@ -701,7 +783,8 @@ void launch(amx_mrhs& m, int nrhs, const float* const* U, float* const* V, hipSt
     uint64_t max_slice = 0;
     for (size_t i = 0; i < m.parts.size(); i++) {
         auto& p = m.parts[i];
-        Seg& sg = tab.s[i];
+        if (p.cong) continue;
+        Seg& sg = tab.s[tab.n_seg++];
         sg.K = p.K.p;
         sg.dofs = p.dofs.as<uint32_t>();
         sg.U = U[i];
@@ -714,13 +797,31 @@ void launch(amx_mrhs& m, int nrhs, const float* const* U, float* const* V, hipSt
         sg.dstride = (uint32_t)dof_stride((int)p.n, m.bf16);
         sg.ve = det ? m.ve.as<float>() + p.ve_row0 * (uint64_t)nrhs : nullptr;
         max_slice = std::max<uint64_t>(max_slice, ((uint64_t)p.n_tiles * ngroups + kXcd - 1) / kXcd);
-        const uint64_t len = (uint64_t)p.n_total * nrhs;
-        if (len && !det) zero_f32<<<(uint32_t)((len + 255) / 256), 256, 0, s>>>(V[i], len);
     }
-    tab.n_seg = (uint32_t)m.parts.size();
     tab.chunked = (uint32_t)m.chunked;
-    if (max_slice == 0) return;
-    if (m.bf16) {
+    if (!det) {
+        OutLaunch out(mrhs_zero_kernel, nrhs, s);
+        for (size_t i = 0; i < m.parts.size(); i++) {
+            OutSeg g{};
+            g.V = V[i];
+            g.n_out = m.parts[i].n_total;
+            out.add(g, (uint64_t)g.n_out * nrhs);
+        }
+        out.run();
+    }
+    for (size_t i = 0; i < m.parts.size(); i++) {
+        auto& p = m.parts[i];
+        if (!p.cong || !p.n_clusters) continue;
+        launch_mrhs_cong(m.bf16,
+                         {p.kref.p, p.scale.p, p.dofs.as<uint32_t>(), p.slots.as<uint16_t>(),
+                          p.clusters.as<uint32_t>(), p.row_dof.as<uint32_t>(), p.direct.as<uint32_t>(),
+                          U[i], V[i], det ? m.ve.as<float>() + p.ve_row0 * (uint64_t)nrhs : nullptr, p.n_clusters,
+                          (uint32_t)nrhs, p.max_rows, p.n_total, (uint32_t)p.ve_rows},
+                         m.cu_count, s);
+    }
+    if (max_slice == 0) {
+        // no other parts
+    } else if (m.bf16) {
         if (NT == 1) launch_persistent<true, 1>(m, tab, max_slice, s);
         else if (NT == 2) launch_persistent<true, 2>(m, tab, max_slice, s);
         else launch_persistent<true, 4>(m, tab, max_slice, s);
@@ -731,21 +832,21 @@ void launch(amx_mrhs& m, int nrhs, const float* const* U, float* const* V, hipSt
     }
     AMX_HIP(hipGetLastError());
     if (det) {
+        OutLaunch out(mrhs_gather_kernel, nrhs, s);
         for (size_t i = 0; i < m.parts.size(); i++) {
             auto& p = m.parts[i];
-            const uint64_t len = (uint64_t)p.n_total * nrhs;
-            if (!len) continue;
-            const float* ve = m.ve.as<float>() + p.ve_row0 * (uint64_t)nrhs;
-            if (nrhs % 4 == 0 && reinterpret_cast<uintptr_t>(V[i]) % 16 == 0 &&
-                reinterpret_cast<uintptr_t>(ve) % 16 == 0) {
-                mrhs_gather4_kernel<<<(uint32_t)((len / 4 + 255) / 256), 256, 0, s>>>(
-                    p.off.as<uint32_t>(), p.pos.as<uint32_t>(), reinterpret_cast<const float4*>(ve),
-                    reinterpret_cast<float4*>(V[i]), p.n_total, (uint32_t)(nrhs / 4));
-            } else {
-                mrhs_gather_kernel<<<(uint32_t)((len + 255) / 256), 256, 0, s>>>(
-                    p.off.as<uint32_t>(), p.pos.as<uint32_t>(), ve, V[i], p.n_total, (uint32_t)nrhs);
-            }
+            OutSeg g{};
+            g.ids = p.cong ? p.ids.as<uint32_t>() : nullptr;
+            g.off = p.off.as<uint32_t>();
+            g.pos = p.pos.as<uint32_t>();
+            g.ve = m.ve.as<float>() + p.ve_row0 * (uint64_t)nrhs;
+            g.V = V[i];
+            g.n_out = p.cong ? p.n_ids : p.n_total;
+            const uintptr_t odd = reinterpret_cast<uintptr_t>(V[i]) | reinterpret_cast<uintptr_t>(g.ve) | 4u * (uint32_t)nrhs;
+            g.cols = odd % 16 == 0 ? 4 : odd % 8 == 0 ? 2 : 1;
+            out.add(g, (uint64_t)g.n_out * (nrhs / g.cols));
         }
+        out.run();
         AMX_HIP(hipGetLastError());
     }
 }
@@ -785,10 +886,20 @@ int amx_mrhs_create(amx_op* const* ops, int n_ops, int precision, amx_mrhs** out
             for (uint32_t sl = 0; sl < g.n_slots; sl++)
                 if (g.slot_elem[sl] != amx::kPadSlot) slot_of.push_back(sl);
             p.n_elem = (uint32_t)slot_of.size();
+            AMX_REQUIRE(op.n_total < (1u << 24), AMX_NOT_IMPLEMENTED, "multi-RHS products take up to 2^24 - 1 DoFs");
+            AMX_REQUIRE((uint64_t)p.n_elem * g.n < (1ull << 32), AMX_NOT_IMPLEMENTED, "too many element rows");
+            p.ve_row0 = 0;
+            for (auto& q : m->parts) p.ve_row0 += q.ve_rows;
+            p.cong = g.cong && g.n == 60;
+            if (p.cong) {
+                amx::create_cong(op, g, slot_of, m->bf16, p);
+                m->parts.push_back(std::move(p));
+                continue;
+            }
+            p.ve_rows = (uint64_t)p.n_elem * g.n;
             const int G = amx::tile_elems((int)g.n), KD = amx::kdim((int)g.n, m->bf16);
             const int DS = amx::dof_stride((int)g.n, m->bf16);
             p.n_tiles = (p.n_elem + G - 1) / G;
-            AMX_REQUIRE(op.n_total < (1u << 24), AMX_NOT_IMPLEMENTED, "multi-RHS products take up to 2^24 - 1 DoFs");
             std::vector<uint32_t> dofs((size_t)p.n_tiles * DS, amx::kNone);
             for (uint32_t t = 0; t < p.n_tiles; t++) {
                 if (g.n == 60) {
@@ -806,8 +917,6 @@ int amx_mrhs_create(amx_op* const* ops, int n_ops, int precision, amx_mrhs** out
             }
             // DoF -> element rows (e * n + r), ascending: the deterministic scatter's lists
             {
-                p.ve_row0 = 0;
-                for (auto& q : m->parts) p.ve_row0 += (uint64_t)q.n_elem * q.n;
                 std::vector<uint32_t> off(op.n_total + 1, 0), pos((size_t)p.n_elem * g.n);
                 for (uint32_t j = 0; j < p.n_elem; j++) {
                     const uint32_t* em = &op.local_map[op.eoff[g.elems[g.slot_elem[slot_of[j]]]]];
@@ -819,7 +928,6 @@ int amx_mrhs_create(amx_op* const* ops, int n_ops, int precision, amx_mrhs** out
                     const uint32_t* em = &op.local_map[op.eoff[g.elems[g.slot_elem[slot_of[j]]]]];
                     for (uint32_t r = 0; r < g.n; r++) pos[fill[em[r]]++] = j * g.n + r;
                 }
-                AMX_REQUIRE((uint64_t)p.n_elem * g.n < (1ull << 32), AMX_NOT_IMPLEMENTED, "too many element rows");
                 p.off.alloc(off.size() * 4);
                 AMX_HIP(hipMemcpy(p.off.p, off.data(), off.size() * 4, hipMemcpyHostToDevice));
                 p.pos.alloc(std::max<size_t>(pos.size(), 1) * 4);

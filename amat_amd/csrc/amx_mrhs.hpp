@@ -1,0 +1,44 @@
+// amx_mrhs.hpp -- multi-RHS products of congruent 60-DoF groups (amx_mrhs_cong.hip)
+#pragma once
+#include <cstdint>
+#include <vector>
+
+#include "amx_internal.hpp"
+
+namespace amx {
+
+constexpr uint32_t kMrhsNoRow = 0xffffffffu;   // row_dof of a padding row
+constexpr int kMrhsClusterRows = 256;          // rows of a cluster, the dump row included, before padding
+
+// elements in clusters; a cluster's rows are summed in LDS before they leave
+struct MrhsClusters {
+    std::vector<uint32_t> order;          // elements, cluster by cluster
+    std::vector<uint32_t> table;          // [cluster][4]: first element of order, first row of ve, of direct
+                                          // (one more entry at the end)
+    std::vector<uint32_t> dofs;           // [element of order][4][16]: DoFs in B fragment order
+    std::vector<uint16_t> slots;          // [element of order][4][16]: LDS byte offsets of the rows in C fragment order
+    std::vector<uint32_t> row_dof;        // row of ve -> DoF or kMrhsNoRow
+    std::vector<uint32_t> direct;         // DoFs whose rows are final
+    std::vector<uint32_t> ids, off, pos;  // the other DoFs, their rows of ve in ascending order
+    uint32_t max_rows = 0;
+};
+// em: n_elem x 60 DoFs below n_total
+MrhsClusters mrhs_clusters(const std::vector<uint32_t>& em, uint32_t n_elem, uint32_t n_total, bool bf16);
+
+// K_ref (row-major) in A fragment order
+std::vector<uint8_t> mrhs_kref(const std::vector<double>& kref, bool bf16);
+
+struct MrhsCongArgs {
+    const void* kref;        // mrhs_kref
+    const void* scale;       // [element of order], FP32 (BF16 storage: high and low FP32 part)
+    const uint32_t* dofs;
+    const uint16_t* slots;
+    const uint32_t *clusters, *row_dof, *direct;
+    const float* U;
+    float* V;
+    float* ve;               // NULL: atomics into V (zeroed before)
+    uint32_t n_clusters, nrhs, max_rows, n_total, ve_rows;
+};
+void launch_mrhs_cong(bool bf16, const MrhsCongArgs& a, int cu_count, hipStream_t s);
+
+}  // namespace amx

@@ -487,7 +487,9 @@ int amx_mrhs_destroy(amx_mrhs* m);
  * run of element tiles of its XCD's share, 0: the waves interleave over it. */
 int amx_mrhs_set_tiles(amx_mrhs* m, int rhs_tile, int waves_per_block, int work_split);
 int amx_mrhs_get_tiles(const amx_mrhs* m, int* rhs_tile, int* waves_per_block, int* work_split);
-/* AMX_SCATTER_ATOMIC (default) or AMX_SCATTER_DETERMINISTIC. */
+/* AMX_SCATTER_ATOMIC (default; order of the sums not fixed, takes the faster of
+ * the two while the row buffer of the other stays within 2 GiB) or
+ * AMX_SCATTER_DETERMINISTIC. */
 int amx_mrhs_set_scatter(amx_mrhs* m, int scatter);
 /* U[i], V[i]: device arrays of operator i (n_ops of each).  V is overwritten. */
 int amx_mrhs_apply_dev(amx_mrhs* m, int nrhs, const float* const* U, float* const* V, void* stream);
