@@ -26,6 +26,7 @@
 #include <algorithm>
 #include <chrono>
 #include <cstring>
+#include <mutex>
 #include <vector>
 
 #include "amx_mrhs.hpp"
@@ -55,8 +56,8 @@ struct Seg {
     const uint32_t* dofs;   // [tile][dstride] local DoF ids (kNone: padding)
     const float* U;
     float* V;
-    float* ve;              // deterministic scatter: element rows [e*n + r][nrhs]; NULL: atomics into V
-    uint32_t n, n_elem, n_tiles, ngroups, nrhs, dstride;
+    float* ve;              // two passes: element rows [e*n + r][ve_ld]; NULL: atomics into V
+    uint32_t n, n_elem, n_tiles, ngroups, nrhs, dstride, ve_ld;
 };
 
 struct SegTable {
@@ -133,7 +134,7 @@ __device__ __forceinline__ void scatter_rows(const Seg& sg, uint32_t t, uint32_t
                 if (col < sg.nrhs && d != kNone) {
                     if (sg.ve) {
                         const uint64_t row = (uint64_t)t * ROWS + (uint32_t)r0 + 4 * half;
-                        sg.ve[row * sg.nrhs + col] = acc[m][q][i];
+                        sg.ve[row * sg.ve_ld + col] = acc[m][q][i];
                     } else {
                         unsafeAtomicAdd(&sg.V[(uint64_t)d * sg.nrhs + col], acc[m][q][i]);
                     }
@@ -310,7 +311,7 @@ __device__ __forceinline__ void scatter60(const Seg& sg, uint32_t e, const uint3
                     if (col < nrhs && !pad) {
                         if (sg.ve) {
                             const uint64_t row = (uint64_t)e * 60 + 30 * m + 8 * j + 4 * h + r;
-                            sg.ve[row * nrhs + col] = acc[m][q][4 * j + r];
+                            sg.ve[row * sg.ve_ld + col] = acc[m][q][4 * j + r];
                         } else {
                             unsafeAtomicAdd(V + __umul24(d[m][j][r], nrhs) + col, acc[m][q][4 * j + r]);
                         }
@@ -521,11 +522,11 @@ struct OutSeg {
     float* V;
     uint64_t block0;  // first block of the part
     uint32_t n_out;   // DoFs
-    uint32_t cols;    // columns per thread: 4, 2 or 1 (nrhs a multiple of it, V and ve aligned)
+    uint32_t wide;    // rows of V 16-byte aligned
 };
 struct OutTable {
     OutSeg s[kMaxSeg];
-    uint32_t n_seg, nrhs;
+    uint32_t n_seg, nrhs, ve_ld;
 };
 __device__ __forceinline__ const OutSeg& out_seg(const OutTable& t, uint64_t& i)
 {
@@ -542,15 +543,13 @@ __global__ __launch_bounds__(256) void mrhs_zero_kernel(OutTable t)
     if (i < (uint64_t)g.n_out * t.nrhs) g.V[i] = 0.0f;
 }
 
-// one entry of V: the sum over its rows of ve in the order of the list.
-// Chunks of 8 entries: index loads, then row loads, in flight together;
-// entries past the end are not added.
-template <typename T>
-__device__ __forceinline__ void gather_one(const OutSeg& g, uint64_t i, uint32_t row)
+// the sum over list entry k's rows of ve, value c of a row of T.  Chunks of 8
+// entries: index loads, then row loads, in flight together; entries past the
+// end are not added.
+template <typename T> __device__ __forceinline__ T gather_rows(const OutSeg& g, uint32_t k, uint32_t row, uint32_t c)
 {
     const T* ve = reinterpret_cast<const T*>(g.ve);
-    const uint32_t d = (uint32_t)(i / row), c = (uint32_t)(i - (uint64_t)d * row);
-    const uint32_t b = g.off[d], cnt = g.off[d + 1] - b;
+    const uint32_t b = g.off[k], cnt = g.off[k + 1] - b;
     T s = T(0.0f);
     for (uint32_t q0 = 0; q0 < cnt; q0 += 8) {
         uint32_t p[8];
@@ -563,21 +562,33 @@ __device__ __forceinline__ void gather_one(const OutSeg& g, uint64_t i, uint32_t
         for (uint32_t j = 0; j < 8; j++)
             if (q0 + j < cnt) s += x[j];
     }
-    reinterpret_cast<T*>(g.V)[g.ids ? (uint64_t)g.ids[d] * row + c : i] = s;
+    return s;
 }
 
 // second pass of the scatter, all parts: V[d][c] = sum over d's rows of ve
 // (fixed order: ascending element, then row; of a congruent group ascending
-// cluster) of ve[row][c].  Two or four columns per thread where the rows allow it:
-// each column's sum keeps the order, so the results are the same bits.
+// cluster) of ve[row][c], four columns per thread (rows of ve are padded to
+// four; a single column is not).
 __global__ __launch_bounds__(256) void mrhs_gather_kernel(OutTable t)
 {
     uint64_t i;
     const OutSeg& g = out_seg(t, i);
-    if (i >= (uint64_t)g.n_out * (t.nrhs / g.cols)) return;
-    if (g.cols == 4) gather_one<f32x4>(g, i, t.nrhs / 4);
-    else if (g.cols == 2) gather_one<f32x2>(g, i, t.nrhs / 2);
-    else gather_one<float>(g, i, t.nrhs);
+    if (t.ve_ld == 1) {
+        if (i < g.n_out) g.V[g.ids ? g.ids[i] : i] = gather_rows<float>(g, (uint32_t)i, 1, 0);
+        return;
+    }
+    const uint32_t row = t.ve_ld / 4;
+    if (i >= (uint64_t)g.n_out * row) return;
+    const uint32_t k = (uint32_t)(i / row), c = (uint32_t)(i - (uint64_t)k * row);
+    const f32x4 s = gather_rows<f32x4>(g, k, row, c);
+    float* out = g.V + (uint64_t)(g.ids ? g.ids[k] : k) * t.nrhs + 4 * c;
+    if (g.wide) {
+        *reinterpret_cast<f32x4*>(out) = s;
+    } else {
+#pragma unroll
+        for (uint32_t j = 0; j < 4; j++)
+            if (4 * c + j < t.nrhs) out[j] = s[j];
+    }
 }
 
 // element matrices for the MFMA kernels from the tiled FP64 storage:
@@ -637,6 +648,9 @@ struct amx_mrhs {
     int chunked = 1;             // work split inside an XCD slice: 1 contiguous chunk per wave, 0 interleaved
     int scatter = AMX_SCATTER_ATOMIC;
     DevBuf ve;                   // deterministic scatter: element rows of all parts x nrhs
+    DevBuf rows;                 // the same for the atomic scatter where it takes the two passes
+    hipEvent_t rows_free = nullptr;  // recorded after the last use of rows
+    std::mutex rows_mutex;
     struct Part {
         uint32_t n, n_elem, n_tiles, n_total;
         uint64_t ve_row0;        // first element row of this part in ve
@@ -655,6 +669,7 @@ struct amx_mrhs {
     int occupancy[256] = {};  // resident blocks per CU, by kernel variant
     ~amx_mrhs()
     {
+        if (rows_free) (void)hipEventDestroy(rows_free);
         if (exec) (void)hipGraphExecDestroy(exec);
         if (graph) (void)hipGraphDestroy(graph);
     }
@@ -688,6 +703,15 @@ template <typename T> void put(DevBuf& b, const std::vector<T>& v)
     if (!v.empty()) AMX_HIP(hipMemcpy(b.p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
 }
 
+// Congruent 60-DoF groups take amx_mrhs_cong.hip from this many elements on; below,
+// the stored matrices are small and their kernel needs no clusters (two passes,
+// a hex8 mesh beside it, stored -> clusters).  FP32: 12^3 elements 17 columns in
+// atomics 24 -> 27 us, 14^3 33 -> 32 us and 128 columns 80 -> 66 us, 20^3 204 ->
+// 145 us.  BF16, which forms its matrices with every 16 columns: 20^3 17 columns
+// 42 -> 49 us, 26^3 50 columns 175 -> 175 us, 28^3 24 columns 94 -> 96 us, 64
+// columns 215 -> 182 us, 31^3 8 columns 89 -> 64 us.
+constexpr uint32_t kCongElemsF32 = 2048, kCongElemsBf16 = 20000;
+
 // the tables of a congruent 60-DoF group, elements in slot order
 void create_cong(const Op& op, const Group& g, const std::vector<uint32_t>& slot_of, bool bf16, amx_mrhs::Part& p)
 {
@@ -720,28 +744,21 @@ void create_cong(const Op& op, const Group& g, const std::vector<uint32_t>& slot
     put(p.pos, c.pos);
 }
 
+// values per row of ve: 16-byte rows for any number of columns but one
+uint32_t ve_stride(int nrhs) { return nrhs == 1 ? 1u : ((uint32_t)nrhs + 3u) & ~3u; }
+
 uint64_t ve_bytes(const amx_mrhs& m, int nrhs)
 {
     uint64_t rows = 0;
     for (auto& p : m.parts) rows += p.ve_rows;
-    return rows * (uint64_t)nrhs * 4;
-}
-
-// The atomic scatter may sum in any order, so it takes the deterministic one's
-// two passes where their buffer is no burden: 24 columns in BF16 on 31^3 hex20 +
-// 80 x 40 x 20 hex8 246 -> 165 us, 64 in FP32 on 24^3 hex20 + 20^3 hex8 189 ->
-// 130 us.  Above, whoever asked for atomics keeps the memory.
-constexpr uint64_t kAtomicVeBytes = 2ull << 30;
-bool two_pass(const amx_mrhs& m, int nrhs)
-{
-    return m.scatter == AMX_SCATTER_DETERMINISTIC || ve_bytes(m, nrhs) <= kAtomicVeBytes;
+    return rows * (uint64_t)ve_stride(nrhs) * 4;
 }
 
 // element-row buffer of the deterministic scatter (allocated outside launches,
 // so a captured graph never allocates)
 void prepare(amx_mrhs& m, int nrhs)
 {
-    if (!two_pass(m, nrhs)) return;
+    if (m.scatter != AMX_SCATTER_DETERMINISTIC) return;
     const uint64_t bytes = std::max<uint64_t>(ve_bytes(m, nrhs), 4);
     if (m.ve.bytes < bytes) m.ve.alloc(bytes);
 }
@@ -766,14 +783,18 @@ struct OutLaunch {
         if (blocks) kernel<<<(uint32_t)blocks, 256, 0, s>>>(t);
         blocks = t.n_seg = 0;
     }
-    OutLaunch(void (*k)(OutTable), int nrhs, hipStream_t stream) : kernel(k), s(stream) { t.nrhs = (uint32_t)nrhs; }
+    OutLaunch(void (*k)(OutTable), int nrhs, hipStream_t stream) : kernel(k), s(stream)
+    {
+        t.nrhs = (uint32_t)nrhs;
+        t.ve_ld = ve_stride(nrhs);
+    }
 };
 
-void launch(amx_mrhs& m, int nrhs, const float* const* U, float* const* V, hipStream_t s)
+// ve: element rows of all parts (two passes), or NULL (atomics into V)
+void launch(amx_mrhs& m, int nrhs, const float* const* U, float* const* V, float* ve, hipStream_t s)
 {
     SegTable tab{};
-    const bool det = two_pass(m, nrhs);
-    if (det) AMX_REQUIRE(m.ve.bytes >= ve_bytes(m, nrhs), AMX_INVALID_STATE, "element-row buffer not prepared");
+    const uint64_t ve_ld = ve_stride(nrhs);
     AMX_REQUIRE(m.parts.size() <= (size_t)kMaxSeg, AMX_NOT_IMPLEMENTED, "too many element groups in one launch");
     const int NT = m.rhs_tile / 32;
     const uint32_t ngroups = (uint32_t)((nrhs + m.rhs_tile - 1) / m.rhs_tile);
@@ -794,12 +815,13 @@ void launch(amx_mrhs& m, int nrhs, const float* const* U, float* const* V, hipSt
         sg.n_tiles = p.n_tiles;
         sg.ngroups = ngroups;
         sg.nrhs = (uint32_t)nrhs;
+        sg.ve_ld = (uint32_t)ve_ld;
         sg.dstride = (uint32_t)dof_stride((int)p.n, m.bf16);
-        sg.ve = det ? m.ve.as<float>() + p.ve_row0 * (uint64_t)nrhs : nullptr;
+        sg.ve = ve ? ve + p.ve_row0 * ve_ld : nullptr;
         max_slice = std::max<uint64_t>(max_slice, ((uint64_t)p.n_tiles * ngroups + kXcd - 1) / kXcd);
     }
     tab.chunked = (uint32_t)m.chunked;
-    if (!det) {
+    if (!ve) {
         OutLaunch out(mrhs_zero_kernel, nrhs, s);
         for (size_t i = 0; i < m.parts.size(); i++) {
             OutSeg g{};
@@ -815,8 +837,8 @@ void launch(amx_mrhs& m, int nrhs, const float* const* U, float* const* V, hipSt
         launch_mrhs_cong(m.bf16,
                          {p.kref.p, p.scale.p, p.dofs.as<uint32_t>(), p.slots.as<uint16_t>(),
                           p.clusters.as<uint32_t>(), p.row_dof.as<uint32_t>(), p.direct.as<uint32_t>(),
-                          U[i], V[i], det ? m.ve.as<float>() + p.ve_row0 * (uint64_t)nrhs : nullptr, p.n_clusters,
-                          (uint32_t)nrhs, p.max_rows, p.n_total, (uint32_t)p.ve_rows},
+                          U[i], V[i], ve ? ve + p.ve_row0 * ve_ld : nullptr, p.n_clusters,
+                          (uint32_t)nrhs, (uint32_t)ve_ld, p.max_rows, p.n_total, (uint32_t)p.ve_rows},
                          m.cu_count, s);
     }
     if (max_slice == 0) {
@@ -831,7 +853,7 @@ void launch(amx_mrhs& m, int nrhs, const float* const* U, float* const* V, hipSt
         else launch_persistent<false, 4>(m, tab, max_slice, s);
     }
     AMX_HIP(hipGetLastError());
-    if (det) {
+    if (ve) {
         OutLaunch out(mrhs_gather_kernel, nrhs, s);
         for (size_t i = 0; i < m.parts.size(); i++) {
             auto& p = m.parts[i];
@@ -839,16 +861,60 @@ void launch(amx_mrhs& m, int nrhs, const float* const* U, float* const* V, hipSt
             g.ids = p.cong ? p.ids.as<uint32_t>() : nullptr;
             g.off = p.off.as<uint32_t>();
             g.pos = p.pos.as<uint32_t>();
-            g.ve = m.ve.as<float>() + p.ve_row0 * (uint64_t)nrhs;
+            g.ve = ve + p.ve_row0 * ve_ld;
             g.V = V[i];
             g.n_out = p.cong ? p.n_ids : p.n_total;
-            const uintptr_t odd = reinterpret_cast<uintptr_t>(V[i]) | reinterpret_cast<uintptr_t>(g.ve) | 4u * (uint32_t)nrhs;
-            g.cols = odd % 16 == 0 ? 4 : odd % 8 == 0 ? 2 : 1;
-            out.add(g, (uint64_t)g.n_out * (nrhs / g.cols));
+            g.wide = reinterpret_cast<uintptr_t>(V[i]) % 16 == 0 && nrhs % 4 == 0;
+            out.add(g, (uint64_t)g.n_out * ((ve_ld + 3) / 4));
         }
         out.run();
         AMX_HIP(hipGetLastError());
     }
+}
+
+// The atomic scatter may sum in any order, so it takes the two passes of the
+// deterministic one where their buffer is neither small nor a burden: 24 columns
+// in BF16 on 31^3 hex20 + 80 x 40 x 20 hex8 (210 MB) 215 -> 160 us, 64 in FP32 on
+// 24^3 hex20 + 20^3 hex8 (130 MB) 189 -> 133 us.  Below kAtomicVeMin the atomics
+// stay in the cache and the event costs more than they do (10^3 elements, 64
+// columns, 15 MB: 27 -> 32 us) -- but not with clusters, whose rows leave in
+// bursts (18^3, 17 columns: 76 -> 50 us).  Above kAtomicVeMax whoever asked for
+// atomics keeps the memory.
+constexpr uint64_t kAtomicVeMin = 32ull << 20, kAtomicVeMax = 2ull << 30;
+
+void mrhs_apply(amx_mrhs& m, int nrhs, const float* const* U, float* const* V, hipStream_t s)
+{
+    if (m.scatter == AMX_SCATTER_DETERMINISTIC) {
+        prepare(m, nrhs);
+        launch(m, nrhs, U, V, m.ve.as<float>(), s);
+        return;
+    }
+    // calls on other streams and threads may run at the same time: the buffer
+    // passes from one to the next by an event.  A capture (which outlives the
+    // buffer) and a failed allocation leave the call with atomics.
+    const uint64_t bytes = ve_bytes(m, nrhs);
+    bool clusters = false;
+    for (auto& p : m.parts) clusters |= p.cong;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (bytes && (clusters || bytes >= kAtomicVeMin) && bytes <= kAtomicVeMax && hipStreamIsCapturing(s, &st) == hipSuccess &&
+        st == hipStreamCaptureStatusNone) {
+        std::lock_guard<std::mutex> lock(m.rows_mutex);
+        if (!m.rows_free && hipEventCreateWithFlags(&m.rows_free, hipEventDisableTiming) != hipSuccess)
+            m.rows_free = nullptr;
+        if (m.rows_free && m.rows.bytes < bytes) {
+            m.rows.release();
+            if (hipMalloc(&m.rows.p, bytes) == hipSuccess) m.rows.bytes = bytes;
+            else m.rows.p = nullptr;
+        }
+        if (m.rows_free && m.rows.bytes >= bytes) {
+            AMX_HIP(hipStreamWaitEvent(s, m.rows_free, 0));
+            launch(m, nrhs, U, V, m.rows.as<float>(), s);
+            AMX_HIP(hipEventRecord(m.rows_free, s));
+            return;
+        }
+    }
+    (void)hipGetLastError();
+    launch(m, nrhs, U, V, nullptr, s);
 }
 
 }  // namespace
@@ -890,7 +956,7 @@ int amx_mrhs_create(amx_op* const* ops, int n_ops, int precision, amx_mrhs** out
             AMX_REQUIRE((uint64_t)p.n_elem * g.n < (1ull << 32), AMX_NOT_IMPLEMENTED, "too many element rows");
             p.ve_row0 = 0;
             for (auto& q : m->parts) p.ve_row0 += q.ve_rows;
-            p.cong = g.cong && g.n == 60;
+            p.cong = g.cong && g.n == 60 && p.n_elem >= (m->bf16 ? amx::kCongElemsBf16 : amx::kCongElemsF32);
             if (p.cong) {
                 amx::create_cong(op, g, slot_of, m->bf16, p);
                 m->parts.push_back(std::move(p));
@@ -1008,8 +1074,7 @@ int amx_mrhs_apply_dev(amx_mrhs* m, int nrhs, const float* const* U, float* cons
     return guarded(__func__, [&] {
         AMX_REQUIRE(m && U && V && nrhs > 0, AMX_INVALID_ARGUMENT, "bad argument");
         amx::DeviceGuard dg(m->device);
-        amx::prepare(*m, nrhs);
-        amx::launch(*m, nrhs, U, V, static_cast<hipStream_t>(stream));
+        amx::mrhs_apply(*m, nrhs, U, V, static_cast<hipStream_t>(stream));
     });
 }
 
@@ -1020,7 +1085,6 @@ int amx_mrhs_autotune(amx_mrhs* m, int nrhs, const float* const* U, float* const
         AMX_REQUIRE(m && U && V && nrhs > 0 && reps > 0, AMX_INVALID_ARGUMENT, "bad argument");
         amx::DeviceGuard dg(m->device);
         hipStream_t s = static_cast<hipStream_t>(stream);
-        amx::prepare(*m, nrhs);
         hipEvent_t e0, e1;
         AMX_HIP(hipEventCreate(&e0));
         AMX_HIP(hipEventCreate(&e1));
@@ -1034,9 +1098,9 @@ int amx_mrhs_autotune(amx_mrhs* m, int nrhs, const float* const* U, float* const
                         m->rhs_tile = rt;
                         m->wpb = w;
                         m->chunked = c;
-                        amx::launch(*m, nrhs, U, V, s);  // warm-up
+                        amx::mrhs_apply(*m, nrhs, U, V, s);  // warm-up
                         AMX_HIP(hipEventRecord(e0, s));
-                        for (int r = 0; r < reps; r++) amx::launch(*m, nrhs, U, V, s);
+                        for (int r = 0; r < reps; r++) amx::mrhs_apply(*m, nrhs, U, V, s);
                         AMX_HIP(hipEventRecord(e1, s));
                         AMX_HIP(hipEventSynchronize(e1));
                         float f = 0;
@@ -1074,7 +1138,7 @@ int amx_mrhs_graph_capture(amx_mrhs* m, int nrhs, const float* const* U, float* 
         if (m->graph) { (void)hipGraphDestroy(m->graph); m->graph = nullptr; }
         AMX_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
         try {
-            amx::launch(*m, nrhs, U, V, s);
+            amx::launch(*m, nrhs, U, V, m->scatter == AMX_SCATTER_DETERMINISTIC ? m->ve.as<float>() : nullptr, s);
         } catch (...) {
             hipGraph_t g;
             (void)hipStreamEndCapture(s, &g);

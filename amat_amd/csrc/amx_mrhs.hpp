@@ -36,8 +36,8 @@ struct MrhsCongArgs {
     const uint32_t *clusters, *row_dof, *direct;
     const float* U;
     float* V;
-    float* ve;               // NULL: atomics into V (zeroed before)
-    uint32_t n_clusters, nrhs, max_rows, n_total, ve_rows;
+    float* ve;               // rows of ve_ld values (1 or a multiple of 4), 16-byte aligned; NULL: atomics into V (zeroed before)
+    uint32_t n_clusters, nrhs, ve_ld, max_rows, n_total, ve_rows;
 };
 void launch_mrhs_cong(bool bf16, const MrhsCongArgs& a, int cu_count, hipStream_t s);
 

@@ -22,10 +22,9 @@
 //   31^3,  24 columns, BF16   atomics 258 -> 165 us, two passes 176 -> 157 us
 //   28^3, 128 columns, BF16   atomics 560 -> 375 us
 //   24^3,  64 columns, FP32   atomics 213 -> 130 us
-//   31^3,   1 column,  FP32   two passes 136 -> 58 us, atomics 141 -> 59 us
-//   16^3,  50 columns, FP32    73 ->  74 us
-// Below some 1,000 elements the clusters are single elements and the time that
-// of the launches (6^3, 128 columns: 21 us both).
+//   31^3,   1 column,  FP32   two passes 136 -> 63 us, atomics 141 -> 66 us
+//   16^3,  50 columns, FP32    68 ->  59 us
+//   14^3, 128 columns, FP32    80 ->  66 us
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -199,13 +198,16 @@ template <> struct Ref<true> {
 };
 
 // n rows of LDS from row l0 on -> rows row(i) of out, and back to zero.  VW
-// columns per lane, 1 << sh lanes per row; row counts are multiples of 16.
+// columns per lane (cols, and rows aligned to them), 1 << sh lanes per row; row
+// counts are multiples of 16.
 template <int VW, bool ATOMIC, bool WIDE, typename F>
-__device__ __forceinline__ void put_rows(float* W, uint32_t n, float* out, uint32_t nrhs, uint32_t col0, uint32_t sh, F&& row)
+__device__ __forceinline__ void put_rows(float* W, uint32_t n, float* out, uint32_t ld, uint32_t cols, uint32_t col0, F&& row)
 {
     typedef float V __attribute__((ext_vector_type(VW)));
+    uint32_t sh = VW == 4 ? 2 : 4;
+    while (sh && (1u << (sh - 1)) * VW >= cols) sh--;
     const uint32_t r = threadIdx.x >> sh, c = VW * (threadIdx.x & ((1u << sh) - 1u)), per = 64u >> sh;
-    const bool in = col0 + c < nrhs;
+    const bool in = col0 + c < cols;
     for (uint32_t b = 0; b < n; b += 4u * per) {
         V v[4];
         uint32_t to[4];
@@ -221,10 +223,10 @@ __device__ __forceinline__ void put_rows(float* W, uint32_t n, float* out, uint3
         for (uint32_t j = 0; j < 4; j++) {
             if (!in || b + j * per + r >= n) continue;
             if constexpr (ATOMIC) {
-                if (to[j] != kMrhsNoRow) unsafeAtomicAdd(at<WIDE>(out, to[j], nrhs, col0 + c), v[j][0]);
+                if (to[j] != kMrhsNoRow) unsafeAtomicAdd(at<WIDE>(out, to[j], ld, col0 + c), v[j][0]);
             } else {
                 // (not read again before the whole of it is written)
-                __builtin_nontemporal_store(v[j], reinterpret_cast<V*>(at<WIDE>(out, to[j], nrhs, col0 + c)));
+                __builtin_nontemporal_store(v[j], reinterpret_cast<V*>(at<WIDE>(out, to[j], ld, col0 + c)));
             }
         }
     }
@@ -250,10 +252,6 @@ __global__ __launch_bounds__(64, 2) void mrhs_cong_kernel(MrhsCongArgs a)
     cur.open(a, ngroups);
     Cursor nx = cur;
     nx.advance(a, ngroups, hi, step);
-    // lanes per row of the flush
-    constexpr int VW = V4 ? 4 : 1;
-    uint32_t sh = V4 ? 2 : 4;
-    while (sh && (1u << (sh - 1)) * VW >= a.nrhs) sh--;
     // an element's DoFs are loaded two elements ahead, its rows of U, factor and
     // row slots one ahead, into the buffer that the present one does not use
     uint32_t d[2][16];
@@ -317,12 +315,16 @@ __global__ __launch_bounds__(64, 2) void mrhs_cong_kernel(MrhsCongArgs a)
         arrived(1 - p);
         if (cur.e + 1 == cur.end) {
             if constexpr (ATOMIC)
-                put_rows<1, true, WIDE>(W, cur.n_ve, a.V, a.nrhs, cur.col0, sh, [&](uint32_t x) { return a.row_dof[cur.ve0 + x]; });
+                put_rows<1, true, WIDE>(W, cur.n_ve, a.V, a.nrhs, a.nrhs, cur.col0,
+                                        [&](uint32_t x) { return a.row_dof[cur.ve0 + x]; });
+            else if (a.ve_ld == 1)
+                put_rows<1, false, WIDE>(W, cur.n_ve, a.ve, 1, 1, 0, [&](uint32_t x) { return cur.ve0 + x; });
             else
-                put_rows<VW, false, WIDE>(W, cur.n_ve, a.ve, a.nrhs, cur.col0, sh, [&](uint32_t x) { return cur.ve0 + x; });
+                put_rows<4, false, WIDE>(W, cur.n_ve, a.ve, a.ve_ld, a.ve_ld, cur.col0,
+                                         [&](uint32_t x) { return cur.ve0 + x; });
             if (cur.n_dir)
-                put_rows<VW, false, WIDE>(W + cur.n_ve * COLS, cur.n_dir, a.V, a.nrhs, cur.col0, sh,
-                                          [&](uint32_t x) { return a.direct[cur.dir0 + x]; });
+                put_rows<V4 ? 4 : 1, false, WIDE>(W + cur.n_ve * COLS, cur.n_dir, a.V, a.nrhs, a.nrhs, cur.col0,
+                                                  [&](uint32_t x) { return a.direct[cur.dir0 + x]; });
             lds_sync_wave();
             if (cur.item + step >= hi) return true;
         }
@@ -344,9 +346,8 @@ void launch_mrhs_cong(bool bf16, const MrhsCongArgs& a, int cu_count, hipStream_
     const uint32_t lds = a.max_rows * COLS * 4u;
     // two waves per SIMD (VGPRs)
     const uint32_t nbx = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(slice, (uint64_t)cu_count));
-    const bool v4 = a.ve && a.nrhs % 4 == 0 && reinterpret_cast<uintptr_t>(a.V) % 16 == 0 &&
-                    reinterpret_cast<uintptr_t>(a.ve) % 16 == 0;
-    const bool wide = (uint64_t)std::max(a.n_total, a.ve_rows) * a.nrhs >= 1ull << 30 || a.nrhs >= 1u << 22 ||
+    const bool v4 = a.ve && a.nrhs % 4 == 0 && reinterpret_cast<uintptr_t>(a.V) % 16 == 0;
+    const bool wide = (uint64_t)std::max(a.n_total, a.ve_rows) * a.ve_ld >= 1ull << 30 || a.ve_ld >= 1u << 22 ||
                       a.ve_rows >= 1u << 24;
     const dim3 grid(nbx * 8u), block(64);
 #define AMX_MC(B, W)                                                                     \
@@ -388,7 +389,7 @@ std::vector<uint8_t> mrhs_kref(const std::vector<double>& kref, bool bf16)
 // most of its elements, then the lowest), until it has n_max elements or its
 // rows are full; with no neighbour left it goes on from the next free element.
 // On a structured hex20 mesh these are bricks of 2 x 2 x 2: 243 rows leave
-// instead of 480, 21 of them final.  n_max: 8 where that leaves 1,024 clusters
+// instead of 480, 16 of them final.  n_max: 8 where that leaves 1,024 clusters
 // (four per CU), fewer below -- a wave takes the elements of a cluster in turn.
 MrhsClusters mrhs_clusters(const std::vector<uint32_t>& em, uint32_t n_elem, uint32_t n_total, bool bf16)
 {
