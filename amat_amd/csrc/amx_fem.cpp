@@ -315,9 +315,14 @@ std::vector<double> free_quadrature(int kind, uint32_t ngt, uint32_t& nq, uint32
     return t;
 }
 
-std::vector<double> gauss_rule(uint32_t ngt)
+std::vector<double> free_rule(int kind, uint32_t ngt)
 {
     check_ngt(ngt);
+    if (kind == AMX_ELEM_TET10_LAPLACE) {
+        std::vector<double> t;
+        tet_rule(ngt, [&](const double* x, double cm) { t.insert(t.end(), {x[0], x[1], x[2], cm}); });
+        return t;
+    }
     double pw[2 * 16];
     gauss_legendre(ngt, pw);
     std::vector<double> r(2 * ngt);

@@ -139,6 +139,117 @@ __global__ __launch_bounds__(256) void free_laplace_kernel(const RT* __restrict_
     }
 }
 
+// ---- tet10 Laplacian: one lane per element slot --------------------------
+// The derivatives of the quadratic interpolant are linear in xi:
+//   df/dxi_d = A_d + sum_k xi_k D_dk,  D symmetric, with vertices v0 (origin),
+//   v_d, and mid-edge nodes e_d (v0, v_d), e_dk (v_d, v_k):
+//   A_d  = 4 (e_d - v0) - (v_d - v0),  D_dd = 4 ((v_d - e_d) + (v0 - e_d)),
+//   D_dk = 4 ((e_dk - e_k) - (e_d - v0)).
+// A point then costs 9 multiply-adds per field instead of 30, and the output
+// needs the sums M_d = sum p_d, M_dd = sum xi_d p_d, S_dk = sum xi_k p_d + xi_d p_k
+// only.  p = w inv inv^T h is formed from the cofactors, one division per point.
+// Coordinates as in free_laplace_kernel; rule: [point][xi, weight].
+//
+// What bounds it: memory (41^3 cubes of 6, FP64: 153 MB, 28 us at 5.5 TB/s; VGPRs
+// allow 4 waves per SIMD).  Against sums over the 10 nodes at every point, at
+// ngt = 2: element kernel 46 -> 34 us, matvec FP64 65 -> 55 us, FP32 45 -> 35 us;
+// relative L2 error 7.1e-16 -> 4.9e-16 (9^3 cubes), FP32 3.9e-7 -> 2.9e-7.
+template <typename RT> struct Tet10 {
+    RT A[3], D[3], S[3];  // S: D_12, D_23, D_31
+    __device__ __forceinline__ explicit Tet10(const RT (&f)[10])
+    {
+        const RT v0 = f[0], e[3] = {f[4], f[6], f[7]}, c[3] = {f[5], f[9], f[8]};  // c: (1,2) (2,3) (3,1)
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            const RT r = e[d] - v0;
+            A[d] = RT(4) * r - (f[1 + d] - v0);
+            D[d] = RT(4) * ((f[1 + d] - e[d]) - r);
+            S[d] = RT(4) * ((c[d] - e[(d + 1) % 3]) - r);
+        }
+    }
+    __device__ __forceinline__ void at(const RT (&x)[3], RT (&g)[3]) const
+    {
+        g[0] = A[0] + x[0] * D[0] + x[1] * S[0] + x[2] * S[2];
+        g[1] = A[1] + x[1] * D[1] + x[2] * S[1] + x[0] * S[0];
+        g[2] = A[2] + x[2] * D[2] + x[0] * S[2] + x[1] * S[1];
+    }
+};
+
+template <typename RT, bool MASKED, bool ATOMIC>
+__global__ __launch_bounds__(256) void free_tet10_kernel(const RT* __restrict__ xe, const double* __restrict__ scale,
+                                                        const uint32_t* __restrict__ map, const RT* __restrict__ u,
+                                                        RT* __restrict__ out, uint64_t ve_base, uint32_t rs,
+                                                        uint32_t ss, uint32_t slot_begin, uint32_t n_slots,
+                                                        uint32_t stride, const double* __restrict__ rule, uint32_t nq,
+                                                        const uint32_t* __restrict__ skip)
+{
+    if (skip && *skip) return;
+    const uint32_t sl = blockIdx.x * blockDim.x + threadIdx.x;
+    if (sl >= n_slots) return;
+    const uint64_t slot = (uint64_t)slot_begin + sl;
+    uint32_t m[10];
+#pragma unroll
+    for (int a = 0; a < 10; a++) m[a] = map[slot * 10 + a];
+    RT v[3][10];
+#pragma unroll
+    for (int k = 0; k < 3; k++)
+#pragma unroll
+        for (int a = 0; a < 10; a++) v[k][a] = xe[(uint64_t)(3 * a + k) * stride + slot];
+    const RT sc = (RT)scale[slot];
+    RT w[10];
+#pragma unroll
+    for (int a = 0; a < 10; a++) {
+        w[a] = u[m[a] & kMask];
+        if (MASKED && (m[a] & kFlag)) w[a] = RT(0);
+    }
+    const Tet10<RT> X[3] = {Tet10<RT>(v[0]), Tet10<RT>(v[1]), Tet10<RT>(v[2])}, U(w);
+    RT M[3] = {0, 0, 0}, Md[3] = {0, 0, 0}, S[3] = {0, 0, 0};
+    for (uint32_t q = 0; q < nq; q++) {
+        const RT x[3] = {(RT)rule[4 * q], (RT)rule[4 * q + 1], (RT)rule[4 * q + 2]};
+        RT J[3][3], h[3], C[3][3], p[3];
+#pragma unroll
+        for (int k = 0; k < 3; k++) X[k].at(x, J[k]);
+        U.at(x, h);
+        // C[d][k]: cofactor of J[k][d]
+#pragma unroll
+        for (int d = 0; d < 3; d++)
+#pragma unroll
+            for (int k = 0; k < 3; k++)
+                C[d][k] = J[(k + 1) % 3][(d + 1) % 3] * J[(k + 2) % 3][(d + 2) % 3] -
+                          J[(k + 1) % 3][(d + 2) % 3] * J[(k + 2) % 3][(d + 1) % 3];
+        const RT det = J[0][0] * C[0][0] + J[0][1] * C[1][0] + J[0][2] * C[2][0];
+        const RT f = (RT)rule[4 * q + 3] * sc / det;
+        RT g[3];
+#pragma unroll
+        for (int k = 0; k < 3; k++) g[k] = (h[0] * C[0][k] + h[1] * C[1][k] + h[2] * C[2][k]) * f;
+#pragma unroll
+        for (int d = 0; d < 3; d++) p[d] = C[d][0] * g[0] + C[d][1] * g[1] + C[d][2] * g[2];
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            M[d] += p[d];
+            Md[d] += x[d] * p[d];
+            S[d] += x[d] * p[(d + 1) % 3] + x[(d + 1) % 3] * p[d];
+        }
+    }
+    // transposed: r_d is the weight of e_d - v0, S_d of e_(d,d+1) - e_(d+1)
+    RT o[10];
+    constexpr int E[3] = {4, 6, 7}, C2[3] = {5, 9, 8};
+    o[0] = RT(0);
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        const RT r = RT(4) * (M[d] - (Md[d] + S[d]));
+        o[1 + d] = RT(4) * Md[d] - M[d];
+        o[0] += M[d] - r;
+        o[E[d]] = r - RT(4) * (Md[d] + S[(d + 2) % 3]);
+        o[C2[d]] = RT(4) * S[d];
+    }
+#pragma unroll
+    for (int a = 0; a < 10; a++) {
+        if constexpr (ATOMIC) unsafeAtomicAdd(&out[m[a] & kMask], o[a]);
+        else out[ve_base + (uint64_t)a * rs + slot * ss] = o[a];
+    }
+}
+
 // ---- hex20 isotropic elasticity -----------------------------------------
 // The serendipity interpolant is a polynomial with few terms per direction, so
 // its derivatives need not be summed node by node at every point.  With a the
@@ -608,9 +719,25 @@ void launch_laplace(bool masked, bool atomic, bool diag, const FreeArgs& a, hipS
             return;
         }
     }
-    if (masked) { if (atomic) AMX_LAP(true, true, false); else AMX_LAP(true, false, false); }
-    else { if (atomic) AMX_LAP(false, true, false); else AMX_LAP(false, false, false); }
+    if constexpr (NN == 8) {  // (tet10: launch_tet10)
+        if (masked) { if (atomic) AMX_LAP(true, true, false); else AMX_LAP(true, false, false); }
+        else { if (atomic) AMX_LAP(false, true, false); else AMX_LAP(false, false, false); }
+    }
 #undef AMX_LAP
+}
+
+template <typename RT> void launch_tet10(bool masked, bool atomic, const FreeArgs& a, hipStream_t s)
+{
+    const dim3 grid((a.n_slots + 255) / 256), block(256);
+    const RT* x = coords<RT>(a);
+    const RT* u = static_cast<const RT*>(a.u);
+    RT* out = static_cast<RT*>(a.out);
+#define AMX_TET(M, A)                                                                                              \
+    free_tet10_kernel<RT, M, A><<<grid, block, 0, s>>>(x, a.scale, a.map, u, out, a.ve_base, a.ve_rs, a.ve_ss,      \
+                                                       a.slot_begin, a.n_slots, a.stride, a.rule, a.nq, a.skip)
+    if (masked) { if (atomic) AMX_TET(true, true); else AMX_TET(true, false); }
+    else { if (atomic) AMX_TET(false, true); else AMX_TET(false, false); }
+#undef AMX_TET
 }
 
 template <typename RT>
@@ -618,7 +745,10 @@ void launch_free_t(int kind, bool masked, bool atomic, bool diag, const FreeArgs
 {
     switch (kind) {
     case AMX_ELEM_HEX8_LAPLACE: launch_laplace<8, RT>(masked, atomic, diag, a, s); break;
-    case AMX_ELEM_TET10_LAPLACE: launch_laplace<10, RT>(masked, atomic, diag, a, s); break;
+    case AMX_ELEM_TET10_LAPLACE:
+        if (diag) launch_laplace<10, RT>(false, false, true, a, s);
+        else launch_tet10<RT>(masked, atomic, a, s);
+        break;
     case AMX_ELEM_HEX20_ELASTIC: {
         AMX_REQUIRE(a.nq <= 64, AMX_NOT_IMPLEMENTED, "hex20: at most 64 quadrature points");
         if (diag) {

@@ -91,8 +91,9 @@ struct DevBuf {
 // quadrature table of the FREE element kernels (amx_fem.cpp): nq points of
 // [dN/dxi per node (3 each), weight], padded with zero-weight rows to rows_min
 std::vector<double> free_quadrature(int kind, uint32_t ngt, uint32_t& nq, uint32_t rows_min);
-// the Gauss-Legendre rule of those tables: ngt points, then ngt weights
-std::vector<double> gauss_rule(uint32_t ngt);
+// the rule of those tables: the Gauss-Legendre points, then their weights;
+// tet10: [point][x y z weight]
+std::vector<double> free_rule(int kind, uint32_t ngt);
 
 }  // namespace amx
 

@@ -205,7 +205,7 @@ struct FreeArgs {
     uint32_t slot_begin, n_slots, stride;
     const double* qp;        // [points][3*nodes+1]: dN/dxi per node, weight
     uint32_t nq;             // quadrature points (hex20: table padded to free_padded_points rows)
-    const double* rule;      // hex20: points, then weights, of the one-dimensional rule
+    const double* rule;      // hex20, tet10: free_rule
     double c1, c2, c3;       // isotropic constitutive entries (hex20)
     const uint32_t* skip = nullptr;
     bool f32 = false;        // compute and vectors in FP32 (inner solves); FP64 otherwise

@@ -191,7 +191,7 @@ void finalize_op(Op& op)
         std::vector<double> tab =
             free_quadrature(op.elem_kind, op.elem_ngt, nq, free_padded_points(op.elem_kind, op.elem_nq));
         op.rule_at = tab.size();
-        const std::vector<double> rule = gauss_rule(op.elem_ngt);
+        const std::vector<double> rule = free_rule(op.elem_kind, op.elem_ngt);
         tab.insert(tab.end(), rule.begin(), rule.end());
         upload(op.qp, tab, s, op.device_bytes);
         AMX_HIP(hipStreamSynchronize(s));

@@ -95,7 +95,7 @@ struct Op {
     uint32_t elem_ngt = 0, elem_nq = 0;
     double elem_c[3] = {0.0, 0.0, 0.0};
     std::vector<double> elem_xe, elem_scale;
-    DevBuf qp;                           // quadrature table, then (from rule_at) the one-dimensional rule
+    DevBuf qp;                           // quadrature table, then (from rule_at) the rule (free_rule)
     size_t rule_at = 0;
 
     // device tables
