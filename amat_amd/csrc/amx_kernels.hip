@@ -799,30 +799,40 @@ __global__ __launch_bounds__(256) void ebe_generic_kernel(const KT* __restrict__
 // do not displace the element rows, map and vectors that the next element
 // kernel and gather find in the caches (hex8 128^3: element kernel 0.143 ->
 // 0.135 ms, gather 49 -> 46 us).
-constexpr uint32_t kGatherWindow = 2048;
+//   A window with fewer entries leaves out the loads that no thread needs (a
+// uniform test per 256): loads of the last entry by all took their turn in the
+// address units (matvecs of hex20 64^3 160 -> 153 us, tet10 48^3 133 -> 128 us).
+//   Window: 2,048 entries hold 256 DoFs of hex20 (4.6 entries each).  Above a mean
+// of 6 (tet10: 7.2, vertices 24) many blocks need a second one for little:
+// kGatherWide takes them at once (tet10 48^3 128 -> 126 us, 20^3 16.1 -> 13.9, BF16
+// 33^3 23.9 -> 22.7; hex20 64^3 would lose with it, 153 -> 156 us; hex8, at most 8
+// each, does with either: 96^3 37.9 and 37.7 us).
+constexpr uint32_t kGatherWindow = 2048, kGatherWide = 3072;
 
-template <typename VT, int BC>
+template <typename VT, int BC, uint32_t WINDOW = kGatherWindow>
 __device__ __forceinline__ void gather_block(const uint32_t* __restrict__ off, const uint32_t* __restrict__ pos,
                                              const VT* __restrict__ ve, const VT* __restrict__ u,
                                              const uint8_t* __restrict__ flag, const double* __restrict__ coef,
                                              VT* __restrict__ v, uint32_t n, uint32_t d0, VT* __restrict__ buf)
 {
-    constexpr uint32_t PER = kGatherWindow / 256u;
+    constexpr uint32_t PER = WINDOW / 256u;
     const uint32_t tid = threadIdx.x, d = d0 + tid;
     const uint32_t dn = min(256u, n - d0);
     const uint32_t e0 = off[d0], e1 = off[d0 + dn];  // uniform
     uint32_t b = 0, c = 0;
     if (d < n) b = off[d], c = off[d + 1];
     VT sum = VT(0);
-    for (uint32_t w = e0; w < e1; w += kGatherWindow) {
-        const uint32_t cnt = min(kGatherWindow, e1 - w);
+    for (uint32_t w = e0; w < e1; w += WINDOW) {
+        const uint32_t cnt = min(WINDOW, e1 - w);
         uint32_t p[PER];
         VT x[PER];
         // entries past the window's end re-read its last entry and are not kept
 #pragma unroll
-        for (uint32_t j = 0; j < PER; j++) p[j] = __builtin_nontemporal_load(pos + w + min(tid + 256u * j, cnt - 1u));
+        for (uint32_t j = 0; j < PER; j++)
+            if (256u * j < cnt) p[j] = __builtin_nontemporal_load(pos + w + min(tid + 256u * j, cnt - 1u));
 #pragma unroll
-        for (uint32_t j = 0; j < PER; j++) x[j] = ve[p[j]];
+        for (uint32_t j = 0; j < PER; j++)
+            if (256u * j < cnt) x[j] = ve[p[j]];
 #pragma unroll
         for (uint32_t j = 0; j < PER; j++)
             if (tid + 256u * j < cnt) buf[tid + 256u * j] = x[j];
@@ -840,17 +850,17 @@ __device__ __forceinline__ void gather_block(const uint32_t* __restrict__ off, c
     v[d] = sum;
 }
 
-template <typename VT, int BC>
+template <typename VT, int BC, uint32_t WINDOW>
 __global__ __launch_bounds__(256) void gather_kernel(const uint32_t* __restrict__ off, const uint32_t* __restrict__ pos,
                                                     const VT* __restrict__ ve, const VT* __restrict__ u,
                                                     const uint8_t* __restrict__ flag, const double* __restrict__ coef,
                                                     VT* __restrict__ v, uint32_t n, const uint32_t* __restrict__ skip)
 {
-    __shared__ VT buf[kGatherWindow];
+    __shared__ VT buf[WINDOW];
     if (skip && *skip) return;
     const uint32_t d0 = __builtin_amdgcn_readfirstlane(xcd_block(blockIdx.x, gridDim.x)) * 256u;
     if (d0 >= n) return;  // uniform per block
-    gather_block<VT, BC>(off, pos, ve, u, flag, coef, v, n, d0, buf);
+    gather_block<VT, BC, WINDOW>(off, pos, ve, u, flag, coef, v, n, d0, buf);
 }
 
 // many jobs in one launch: block -> 256 DoFs of entry job_of(prefix)
@@ -923,9 +933,10 @@ __device__ __forceinline__ void gather_dot_block(const GatherJob& jb, uint32_t b
             VT x[PER];
 #pragma unroll
             for (uint32_t j = 0; j < PER; j++)
-                p[j] = __builtin_nontemporal_load(pos + w + min(tid + 256u * j, cnt - 1u));
+                if (256u * j < cnt) p[j] = __builtin_nontemporal_load(pos + w + min(tid + 256u * j, cnt - 1u));
 #pragma unroll
-            for (uint32_t j = 0; j < PER; j++) x[j] = ve[p[j]];
+            for (uint32_t j = 0; j < PER; j++)
+                if (256u * j < cnt) x[j] = ve[p[j]];
 #pragma unroll
             for (uint32_t j = 0; j < PER; j++)
                 if (tid + 256u * j < cnt) win[tid + 256u * j] = x[j];
@@ -1615,13 +1626,18 @@ void launch_ebe(const Layout& L, KType kt, bool vt_double, bool masked, bool ato
     AMX_HIP(hipGetLastError());
 }
 
-void launch_gather(bool vt_double, int bc, const uint32_t* off, const uint32_t* pos, const void* ve, const void* u,
-                   const uint8_t* flag, const double* coef, void* v, uint32_t n, hipStream_t s, const uint32_t* skip)
+void launch_gather(bool vt_double, int bc, const uint32_t* off, const uint32_t* pos, uint64_t n_entries, const void* ve,
+                   const void* u, const uint8_t* flag, const double* coef, void* v, uint32_t n, hipStream_t s,
+                   const uint32_t* skip)
 {
     if (n == 0) return;
     const uint32_t nb = blocks_for(n, 256);
-#define AMX_GATHER(VT, BC)                                                                                         \
-    gather_kernel<VT, BC><<<nb, 256, 0, s>>>(off, pos, (const VT*)ve, (const VT*)u, flag, coef, (VT*)v, n, skip)
+    const bool wide = n_entries > 6ull * n;
+#define AMX_GATHER(VT, BC)                                                                                          \
+    (wide ? gather_kernel<VT, BC, kGatherWide><<<nb, 256, 0, s>>>(off, pos, (const VT*)ve, (const VT*)u, flag, coef, \
+                                                                  (VT*)v, n, skip)                                  \
+          : gather_kernel<VT, BC, kGatherWindow><<<nb, 256, 0, s>>>(off, pos, (const VT*)ve, (const VT*)u, flag,     \
+                                                                    coef, (VT*)v, n, skip))
     if (vt_double) {
         if (bc == 0) AMX_GATHER(double, 0);
         else if (bc == 1) AMX_GATHER(double, 1);

@@ -108,7 +108,7 @@ void launch_ebe(const Layout& L, KType kt, bool vt_double, bool masked, bool ato
 // v[d] = sum_{q in [off[d], off[d+1])} ve[pos[q]] (fixed order), then the BC
 // form: bc 0 none; 1 identity (flag[d] -> v[d] = u[d]); 2 penalty
 // (flag[d] -> v[d] += coef[d] * u[d]).
-void launch_gather(bool vt_double, int bc, const uint32_t* off, const uint32_t* pos, const void* ve,
+void launch_gather(bool vt_double, int bc, const uint32_t* off, const uint32_t* pos, uint64_t n_entries, const void* ve,
                    const void* u, const uint8_t* flag, const double* coef, void* v, uint32_t n, hipStream_t s,
                    const uint32_t* skip = nullptr);
 

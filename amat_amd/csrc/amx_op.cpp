@@ -519,8 +519,8 @@ void finalize_op(Op& op)
     // element order as the gather, and the penalty coefficients p - diag
     op.diag.alloc(std::max<uint32_t>(op.n_total, 1) * sizeof(double));
     op.device_bytes += op.diag.bytes;
-    launch_gather(true, 0, op.off.as<uint32_t>(), op.pos.as<uint32_t>(), op.ve.p, nullptr, nullptr, nullptr,
-                  op.diag.p, op.n_total, s);
+    launch_gather(true, 0, op.off.as<uint32_t>(), op.pos.as<uint32_t>(), op.pos.bytes / 4, op.ve.p, nullptr, nullptr,
+                  nullptr, op.diag.p, op.n_total, s);
     op.coef64.alloc(std::max<uint32_t>(op.n_total, 1) * sizeof(double));
     op.device_bytes += op.coef64.bytes;
     launch_fill(op.coef64.p, op.n_total, true, 0.0, s);
@@ -687,7 +687,7 @@ void ebe_launch(Op& op, KType kt, bool vt_double, bool masked, int phase, const 
 void gather_launch(Op& op, bool vt_double, int bc, const void* u, void* v, hipStream_t s, const uint32_t* skip,
                    const void* ve)
 {
-    launch_gather(vt_double, bc, op.off.as<uint32_t>(), op.pos.as<uint32_t>(), ve ? ve : op.ve.p, u,
+    launch_gather(vt_double, bc, op.off.as<uint32_t>(), op.pos.as<uint32_t>(), op.pos.bytes / 4, ve ? ve : op.ve.p, u,
                   op.flag.as<uint8_t>(), op.coef64.as<double>(), v, op.n_total, s, skip);
 }
 
