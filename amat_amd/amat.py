@@ -124,9 +124,21 @@ def _ptr(a) -> int | None:
     raise TypeError(f"unsupported array type {type(a)}")
 
 
+_DTYPE_NAMES: dict = {}  # torch dtype -> "float64", ...
+
+
 def _dev(t, n: int, name: str, device: int, dtype: str = "float64") -> int:
     """Address of a contiguous torch tensor on HIP device `device` with dtype
     `dtype` and at least n entries; raises before anything is launched."""
+    # a usable tensor in five cheap reads (a product of a small mesh is as long as
+    # its host path: 64 to 32,768 hex8 elements 9.7 -> 8.6 us per call); what is wrong
+    # with any other is said below
+    try:
+        if (t.is_cuda and t.get_device() == device and _DTYPE_NAMES.get(t.dtype) == dtype and t.is_contiguous()
+                and t.numel() >= n):
+            return t.data_ptr()
+    except AttributeError:
+        pass
     if t is None or not hasattr(t, "data_ptr"):
         raise TypeError(f"{name} must be a torch tensor on a HIP device")
     if not getattr(t, "is_cuda", False):
@@ -135,6 +147,7 @@ def _dev(t, n: int, name: str, device: int, dtype: str = "float64") -> int:
         raise ValueError(f"{name} is on device {t.device.index}; the operator is on device {device}")
     if str(t.dtype) != "torch." + dtype:
         raise TypeError(f"{name} is {t.dtype}; expected torch.{dtype}")
+    _DTYPE_NAMES[t.dtype] = dtype
     if not t.is_contiguous():
         raise ValueError(f"{name} must be contiguous")
     if t.numel() < n:
@@ -491,7 +504,7 @@ class aMatFree:
     # vectors: float64 (float32 for the FP32 forms) tensors on the operator's
     # device with at least n_total entries; checked before any launch
     def _vec(self, t, name, dtype="float64"):
-        return _dev(t, self._sizes()[0], name, self.device, dtype)
+        return _dev(t, self._size_t[0], name, self.device, dtype)
 
     def matvec_dev(self, v, u, stream=None):
         call("amx_op_matvec_dev", self._h, self._vec(v, "v"), self._vec(u, "u"), _stream_ptr(stream))
