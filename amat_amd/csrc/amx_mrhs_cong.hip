@@ -28,7 +28,9 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstring>
+#include <new>
 #include <type_traits>
 
 #include "amx_device.hpp"
@@ -396,9 +398,11 @@ MrhsClusters mrhs_clusters(const std::vector<uint32_t>& em, uint32_t n_elem, uin
     constexpr uint32_t kShares = 8, kNodes = N / 3, kRows = kMrhsClusterRows - 1;
     const uint32_t n_max = std::min(8u, std::max(1u, n_elem / 1024u));
     struct Share {
-        std::vector<uint32_t> order, count, rows;  // elements; elements and rows per cluster
-        std::vector<uint32_t> row_dof;
-        std::vector<uint16_t> slots;               // [element][60]
+        std::vector<uint32_t> order, count, rows;        // elements; elements and rows per cluster
+        std::vector<uint32_t> row_of;                    // DoFs of the rows, cluster by cluster
+        std::vector<uint16_t> slots;                     // [element][60]
+        std::vector<uint32_t> table, row_dof, direct;    // as in MrhsClusters, counted from the share's start
+        uint32_t max_rows = 0;
     };
     std::vector<Share> sh(kShares);
     // every third DoF stands for its node (a map of another form only makes worse clusters)
@@ -413,8 +417,11 @@ MrhsClusters mrhs_clusters(const std::vector<uint32_t>& em, uint32_t n_elem, uin
     }
     std::vector<uint8_t> taken(n_elem, 0);
     std::vector<uint32_t> shared(n_elem, 0), mult(n_elem, 0);  // of the open cluster; an element belongs to one share
-#pragma omp parallel for schedule(static, 1) num_threads(kShares) if (n_elem > 1024)
-    for (uint32_t p = 0; p < kShares; p++) {
+    MrhsClusters C;
+    C.slots.assign((size_t)n_elem * 64, 0);
+    C.dofs.assign((size_t)n_elem * 64, 0);
+    C.order.assign(n_elem, 0);
+    auto form = [&](uint32_t p) {
         Share& S = sh[p];
         const uint32_t lo = (uint32_t)((uint64_t)n_elem * p / kShares), hi = (uint32_t)((uint64_t)n_elem * (p + 1) / kShares);
         std::vector<uint32_t> seen(n_total, 0), slot_of(n_total, 0), used(n_total, 0);
@@ -446,7 +453,7 @@ MrhsClusters mrhs_clusters(const std::vector<uint32_t>& em, uint32_t n_elem, uin
                     if (seen[d[r]] != row_stamp || used[d[r]] == elem_stamp) {
                         seen[d[r]] = row_stamp;
                         slot_of[d[r]] = rows++;
-                        S.row_dof.push_back(d[r]);
+                        S.row_of.push_back(d[r]);
                     }
                     used[d[r]] = elem_stamp;
                     S.slots.push_back((uint16_t)slot_of[d[r]]);
@@ -508,17 +515,12 @@ MrhsClusters mrhs_clusters(const std::vector<uint32_t>& em, uint32_t n_elem, uin
             cand.clear();
             emit();
         }
-    }
-    MrhsClusters C;
-    C.slots.assign((size_t)n_elem * 64, 0);
-    C.dofs.assign((size_t)n_elem * 64, 0);
-    C.order.reserve(n_elem);
-    std::vector<uint32_t> uses, place;
-    for (const Share& S : sh) {
+        // where the rows lie, and the elements' tables
+        std::vector<uint32_t> uses, place;
         size_t e = 0, r = 0;
         for (size_t i = 0; i < S.count.size(); i++) {
             const uint32_t rows = S.rows[i], n_here = S.count[i];
-            C.table.insert(C.table.end(), {(uint32_t)C.order.size(), (uint32_t)C.row_dof.size(), (uint32_t)C.direct.size(), 0u});
+            S.table.insert(S.table.end(), {(uint32_t)(lo + e), (uint32_t)S.row_dof.size(), (uint32_t)S.direct.size(), 0u});
             uses.assign(rows, 0);
             place.assign(rows, 0);
             for (size_t x = e * N; x < (e + n_here) * N; x++) uses[S.slots[x]]++;
@@ -526,30 +528,30 @@ MrhsClusters mrhs_clusters(const std::vector<uint32_t>& em, uint32_t n_elem, uin
             // after the others, which are padded to sixteens with at least one row,
             // the dump row; what is left of a sixteen goes through ve
             uint32_t n_dir = 0, n_ve = 0, k = 0;
-            for (uint32_t x = 0; x < rows; x++) n_dir += uses[x] == valence[S.row_dof[r + x]];
+            for (uint32_t x = 0; x < rows; x++) n_dir += uses[x] == valence[S.row_of[r + x]];
             n_dir &= ~15u;
             const uint32_t padded = (rows - n_dir + 16) / 16 * 16;
             // rows 4 apart, which a wave's four lane groups reach together, lie in
             // different banks: 4 x 4 transposed within 16
             auto swap4 = [](uint32_t s) { return (s & ~15u) | ((s & 3u) << 2) | ((s >> 2) & 3u); };
-            const uint32_t ve0 = (uint32_t)C.row_dof.size(), dir0 = (uint32_t)C.direct.size();
-            C.row_dof.resize(ve0 + padded, kMrhsNoRow);
-            C.direct.resize(dir0 + n_dir);
+            const uint32_t ve0 = (uint32_t)S.row_dof.size(), dir0 = (uint32_t)S.direct.size();
+            S.row_dof.resize(ve0 + padded, kMrhsNoRow);
+            S.direct.resize(dir0 + n_dir);
             for (uint32_t x = 0; x < rows; x++) {
-                const uint32_t d = S.row_dof[r + x];
+                const uint32_t d = S.row_of[r + x];
                 if (k < n_dir && uses[x] == valence[d]) {
                     const uint32_t at = swap4(k++);
-                    C.direct[dir0 + at] = d;
+                    S.direct[dir0 + at] = d;
                     place[x] = padded + at;
                 } else {
                     place[x] = swap4(n_ve++);
-                    C.row_dof[ve0 + place[x]] = d;
+                    S.row_dof[ve0 + place[x]] = d;
                 }
             }
             const uint32_t dump = swap4(n_ve);
             for (uint32_t j = 0; j < n_here; j++, e++) {
                 const uint32_t el = S.order[e];
-                const uint64_t at = C.order.size();
+                const uint64_t at = lo + e;
                 const uint32_t* d = &em[(size_t)el * N];
                 const uint16_t* sl = &S.slots[e * N];
                 for (uint32_t x = 0; x < 64; x++) {
@@ -559,11 +561,29 @@ MrhsClusters mrhs_clusters(const std::vector<uint32_t>& em, uint32_t n_elem, uin
                     const uint32_t col = bf16 ? 32 * (y / 8) + 8 * q + y % 8 : 4 * y + q;
                     C.dofs[at * 64 + x] = d[col < N ? col : 0];
                 }
-                C.order.push_back(el);
+                C.order[at] = el;
             }
             r += rows;
-            C.max_rows = std::max(C.max_rows, padded + n_dir);
+            S.max_rows = std::max(S.max_rows, padded + n_dir);
         }
+    };
+    std::atomic<bool> failed{false};  // (no exception leaves a parallel region)
+#pragma omp parallel for schedule(static, 1) num_threads(kShares) if (n_elem > 1024)
+    for (uint32_t p = 0; p < kShares; p++) {
+        try {
+            form(p);
+        } catch (...) {
+            failed = true;
+        }
+    }
+    if (failed) throw std::bad_alloc();
+    for (const Share& S : sh) {
+        const uint32_t ve0 = (uint32_t)C.row_dof.size(), dir0 = (uint32_t)C.direct.size();
+        for (size_t i = 0; i < S.table.size(); i += 4)
+            C.table.insert(C.table.end(), {S.table[i], S.table[i + 1] + ve0, S.table[i + 2] + dir0, 0u});
+        C.row_dof.insert(C.row_dof.end(), S.row_dof.begin(), S.row_dof.end());
+        C.direct.insert(C.direct.end(), S.direct.begin(), S.direct.end());
+        C.max_rows = std::max(C.max_rows, S.max_rows);
     }
     C.table.insert(C.table.end(), {(uint32_t)C.order.size(), (uint32_t)C.row_dof.size(), (uint32_t)C.direct.size(), 0u});
     // second pass: the DoFs that are not final, with their rows of ve in

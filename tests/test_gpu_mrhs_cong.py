@@ -15,9 +15,13 @@ from test_gpu_mrhs import TOL_MODEL, bf16_round
 pytestmark = pytest.mark.gpu
 
 
-def build(dims, precision, order=None):
+def build(dims, precision, order=None, twice=False):
     p = problems.elasticity_hex20(*dims)
     g = p.gmap if order is None else p.gmap[order]
+    if twice:   # every seventh element names DoFs twice, one of them three times
+        g = g.copy()
+        g[::7, 5] = g[::7, 2]
+        g[::7, 40] = g[::7, 41] = g[::7, 17]
     E, N = g.shape[0], p.n_dofs
     maps = Maps(0, 1)
     maps.set_map(E, g.astype(np.uint32), np.full(E, 60, np.uint32), N, np.arange(N, dtype=np.uint64), 0, N - 1, N)
@@ -119,3 +123,17 @@ def test_atomic_streams_and_capture(torch_gpu):
         assert torch.equal(v, want)   # the two passes are the deterministic ones
     v0 = V[0].cpu().double().numpy()
     assert rel_l2(W.cpu().double().numpy(), v0) <= TOL_MODEL
+
+
+def test_dofs_named_twice(torch_gpu):
+    torch = torch_gpu
+    op, mr, g, s, k_ref, N = build((16, 16, 17), PREC.FP32, twice=True)
+    nrhs = 6
+    U = mesh.uniform(7, 1, N * nrhs, -1.0, 1.0).astype(np.float32).reshape(N, nrhs)
+    want = model(g, s, k_ref, N, U.astype(np.float64), PREC.FP32)
+    for scatter in (SCATTER.DETERMINISTIC, SCATTER.ATOMIC):
+        mr.set_scatter(scatter)
+        dV = torch.full((N, nrhs), float("nan"), device="cuda")
+        mr.apply_dev(nrhs, [torch.from_numpy(U).cuda()], [dV], torch.cuda.current_stream())
+        V = dV.cpu().numpy().astype(np.float64)
+        assert max(rel_l2(V[:, c], want[:, c]) for c in range(nrhs)) <= TOL_MODEL
