@@ -720,20 +720,20 @@ void create_cong(const Op& op, const Group& g, const std::vector<uint32_t>& slot
         const uint32_t* d = &op.local_map[op.eoff[g.elems[g.slot_elem[slot_of[j]]]]];
         std::copy(d, d + g.n, em.begin() + (size_t)j * g.n);
     }
-    const MrhsClusters c = mrhs_clusters(em, p.n_elem, p.n_total, bf16);
-    std::vector<double> scale(p.n_elem);
-    for (uint32_t j = 0; j < p.n_elem; j++) scale[j] = op.scale[g.elems[g.slot_elem[slot_of[c.order[j]]]]];
+    const std::vector<uint8_t> order = mrhs_order(op.kref);
+    const MrhsClusters c = mrhs_clusters(em, order, p.n_elem, p.n_total, bf16);
+    std::vector<float> scale;
+    for (uint32_t j = 0; j < p.n_elem; j++) {
+        float f[2];
+        mrhs_factor(op.scale[g.elems[g.slot_elem[slot_of[c.order[j]]]]], bf16, f);
+        scale.insert(scale.end(), f, f + 2);
+    }
     p.ve_rows = c.row_dof.size();
     p.n_clusters = (uint32_t)c.table.size() / 4 - 1;
     p.max_rows = c.max_rows;
     p.n_ids = (uint32_t)c.ids.size();
-    put(p.kref, mrhs_kref(op.kref, bf16));
-    std::vector<float> sf;
-    for (double x : scale) {
-        sf.push_back((float)x);
-        if (bf16) sf.push_back((float)(x - (double)(float)x));
-    }
-    put(p.scale, sf);
+    put(p.kref, mrhs_kref(op.kref, order, bf16));
+    put(p.scale, scale);
     put(p.dofs, c.dofs);
     put(p.slots, c.slots);
     put(p.clusters, c.table);

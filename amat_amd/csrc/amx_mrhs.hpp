@@ -22,15 +22,20 @@ struct MrhsClusters {
     std::vector<uint32_t> ids, off, pos;  // the other DoFs, their rows of ve in ascending order
     uint32_t max_rows = 0;
 };
+// the order in which the FP32 product takes the columns of K_ref (row-major)
+std::vector<uint8_t> mrhs_order(const std::vector<double>& kref);
 // em: n_elem x 60 DoFs below n_total
-MrhsClusters mrhs_clusters(const std::vector<uint32_t>& em, uint32_t n_elem, uint32_t n_total, bool bf16);
-
-// K_ref (row-major) in A fragment order
-std::vector<uint8_t> mrhs_kref(const std::vector<double>& kref, bool bf16);
+MrhsClusters mrhs_clusters(const std::vector<uint32_t>& em, const std::vector<uint8_t>& order, uint32_t n_elem,
+                           uint32_t n_total, bool bf16);
+// K_ref in A fragment order
+std::vector<uint8_t> mrhs_kref(const std::vector<double>& kref, const std::vector<uint8_t>& order, bool bf16);
+// a factor as the kernel takes it: s = out[0] + out[1] (FP32: out[0] cut towards
+// zero, out[1] divided by the power of two of out[0])
+void mrhs_factor(double s, bool bf16, float (&out)[2]);
 
 struct MrhsCongArgs {
     const void* kref;        // mrhs_kref
-    const void* scale;       // [element of order], FP32 (BF16 storage: high and low FP32 part)
+    const void* scale;       // [element of order][2], mrhs_factor
     const uint32_t* dofs;
     const uint16_t* slots;
     const uint32_t *clusters, *row_dof, *direct;

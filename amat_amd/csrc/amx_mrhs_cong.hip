@@ -8,7 +8,7 @@
 // (0.49 of the element rows on a structured mesh).
 //   FP32: v_mfma_f32_16x16x4_f32, 60 = 15 steps of 4;
 //   BF16: v_mfma_f32_16x16x32_bf16, two steps, columns 60..63 zero;
-//   A lane l: row 16 m + l % 16, columns 4 ks + l/16 (BF16 32 ks + 8 (l/16) + v);
+//   A lane l: row 16 m + l % 16, columns 4 ks + l/16 of mrhs_order (BF16 32 ks + 8 (l/16) + v);
 //   C lane l, register i: row 16 m + 4 (l/16) + i, column l % 16.
 // Rows 60..63 (tile m = 3) go to a dump row.
 //
@@ -29,6 +29,8 @@
 
 #include <algorithm>
 #include <atomic>
+#include <cfloat>
+#include <cmath>
 #include <cstring>
 #include <new>
 #include <type_traits>
@@ -118,12 +120,17 @@ __device__ __forceinline__ uint32_t bf16_pair(float lo, float hi)
 }
 
 template <bool BF16> struct Ref;
-__device__ __forceinline__ float factor(float s) { return s; }
-__device__ __forceinline__ float factor(f32x2) { return 1.0f; }
+// FP32: K_ref to 32 bits -- 24 in FP32, the 8 below them in BF16, whose product
+// with the leading bits of U takes 8 MFMAs beside 60 -- and the factor 2^k m to
+// 48: U times 2^k is exact, m (high and low part) multiplies the product.  The
+// operands then carry less error than a stored matrix, whose entries s_e K_ref are
+// rounded to FP32.  It costs 3 to 8 % (32^3, 128 columns 558 -> 573 us); K_ref
+// and factor in FP32 alone, the same error in every element, had twice the operand
+// error of a stored matrix.  High parts are cut towards zero and low parts never
+// zero beside them: the products of an infinite U have one sign.
 template <> struct Ref<false> {
-    typedef float S;
-    static constexpr bool kAfter = true;  // the factor is applied to the product
     float k[4][15];
+    u32x4 low[4][2];  // lane's columns 4 (8 t + v) + l/16, v = 0..7 (the order of B.b)
     __device__ __forceinline__ void load(const void* K)
     {
         const f32x4* p = static_cast<const f32x4*>(K) + threadIdx.x;
@@ -133,13 +140,32 @@ template <> struct Ref<false> {
 #pragma unroll
             for (int j = 0; j < 4; j++) k[(4 * i + j) / 15][(4 * i + j) % 15] = v[j];
         }
+#pragma unroll
+        for (int i = 0; i < 8; i++) low[i / 2][i % 2] = __builtin_bit_cast(u32x4, p[64 * (15 + i)]);
     }
     // side(i), i < 15: what is issued in the shadow of four MFMAs.  Two sums of
-    // 8 and 7 steps: with K_ref and the factor rounded by themselves one sum of
-    // 15 had up to 4 % more error than the stored matrices, two have 20 % less.
-    template <typename R, typename F> __device__ __forceinline__ void multiply(S, const R& B, f32x4 (&acc)[4], F&& side) const
+    // 8 and 7 steps: one sum of 15 had more error than the stored matrices' sums.
+    template <typename R, typename F> __device__ __forceinline__ void multiply(f32x2 s, R& B, f32x4 (&acc)[4], F&& side) const
     {
-        f32x4 more[4] = {};
+        const float pow2 = __uint_as_float(__float_as_uint(s[0]) & 0x7f800000u);
+#pragma unroll
+        for (int ks = 0; ks < 15; ks++) B.b[ks] *= pow2;
+        f32x4 more[4];
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            u32x4 b;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int ks = 8 * t + 2 * j;
+                b[j] = __builtin_amdgcn_perm(ks + 1 < 15 ? __float_as_uint(B.b[ks + 1 < 15 ? ks + 1 : 0]) : 0u,
+                                             __float_as_uint(B.b[ks]), 0x07060302u);
+            }
+#pragma unroll
+            for (int m = 0; m < 4; m++)
+                more[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, low[m][t]),
+                                                                  __builtin_bit_cast(bf16x8, b),
+                                                                  t ? more[m] : f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+        }
 #pragma unroll
         for (int ks = 0; ks < 15; ks++) {
 #pragma unroll
@@ -152,14 +178,18 @@ template <> struct Ref<false> {
 #pragma unroll
         for (int m = 0; m < 4; m++) acc[m] += more[m];
     }
+    // the element's value of a row whose product is x
+    static __device__ __forceinline__ float row(f32x2 s, float x)
+    {
+        const float m = __uint_as_float((__float_as_uint(s[0]) & 0x807fffffu) | 0x3f800000u);
+        return fmaf(x, m, x * s[1]);
+    }
 };
 // BF16: the stored matrices are s_e K_ref rounded to FP32, then to BF16.  Factor
 // and K_ref are split in two FP32 values each: h S + (h s + l S) is their product
 // to 48 bits and rounds once, in three instructions (an FP64 product and its
 // conversion take 59 cycles per value, 420 us at 32768 elements x 128 columns).
 template <> struct Ref<true> {
-    typedef f32x2 S;  // high, low
-    static constexpr bool kAfter = false;
     float h[4][2][8], l[4][2][8];
     __device__ __forceinline__ void load(const void* K)
     {
@@ -174,7 +204,7 @@ template <> struct Ref<true> {
             }
         }
     }
-    template <typename R, typename F> __device__ __forceinline__ void multiply(S s, const R& B, f32x4 (&acc)[4], F&& side) const
+    template <typename R, typename F> __device__ __forceinline__ void multiply(f32x2 s, R& B, f32x4 (&acc)[4], F&& side) const
     {
 #pragma unroll
         for (int i = 0; i < 6; i++) side(i);
@@ -197,6 +227,7 @@ template <> struct Ref<true> {
 #pragma unroll
         for (int i = 6; i < 15; i++) side(i);
     }
+    static __device__ __forceinline__ float row(f32x2, float x) { return x; }
 };
 
 // n rows of LDS from row l0 on -> rows row(i) of out, and back to zero.  VW
@@ -259,9 +290,8 @@ __global__ __launch_bounds__(64, 2) void mrhs_cong_kernel(MrhsCongArgs a)
     uint32_t d[2][16];
     u32x4 slots[2][2];
     Rhs<BF16, WIDE> B[2];
-    typedef typename Ref<BF16>::S S;
-    S s[2];
-    const S* scale = static_cast<const S*>(a.scale);
+    f32x2 s[2];
+    const f32x2* scale = static_cast<const f32x2*>(a.scale);
     load_dofs(a, cur.e, q, d[0]);
     load_slots(a, cur.e, q, slots[0]);
     s[0] = scale[cur.e];
@@ -312,7 +342,7 @@ __global__ __launch_bounds__(64, 2) void mrhs_cong_kernel(MrhsCongArgs a)
         });
 #pragma unroll
         for (int i = 0; i < 16; i++)
-            *w[i] = Ref<BF16>::kAfter ? fmaf(factor(s[p]), acc[i / 4][i % 4], o[i]) : o[i] + acc[i / 4][i % 4];
+            *w[i] = o[i] + Ref<BF16>::row(s[p], acc[i / 4][i % 4]);
         lds_sync_wave();
         arrived(1 - p);
         if (cur.e + 1 == cur.end) {
@@ -362,27 +392,80 @@ void launch_mrhs_cong(bool bf16, const MrhsCongArgs& a, int cu_count, hipStream_
     AMX_HIP(hipGetLastError());
 }
 
-// K_ref in the order of Ref::load: value i of lane l in 16-byte pieces, lanes
-// side by side; FP32 i = 15 m + ks; BF16 i = 16 m + 8 ks + v, two
-// FP32 values
-std::vector<uint8_t> mrhs_kref(const std::vector<double>& kref, bool bf16)
+// the FP32 value at or next to x towards zero
+static float cut(double x)
 {
-    const uint32_t n_val = bf16 ? 64 : 60, per = bf16 ? 2 : 4, size = bf16 ? 8 : 4;
-    std::vector<uint8_t> out((size_t)n_val * 64 * size);
+    const float f = (float)x;
+    return std::fabs((double)f) > std::fabs(x) ? std::nextafterf(f, 0.0f) : f;
+}
+
+// A row of a smooth U is a small sum of large terms; what it loses is the rounding
+// of the partial sums on the way.  Column by column the one that keeps the sums
+// of the three translations (every third DoF 1) smallest over all rows.  hex20
+// 20^3, error relative to that of stored matrices: quadratic field 0.32, sine field
+// 0.39, random U 0.82 (in the order of the DoFs 1.6, 1.5 and 0.79).
+std::vector<uint8_t> mrhs_order(const std::vector<double>& kref)
+{
+    std::vector<uint8_t> left(N), order;
+    for (int c = 0; c < N; c++) left[c] = (uint8_t)c;
+    std::vector<double> sum(3 * N, 0.0);
+    while (!left.empty()) {
+        size_t best = 0;
+        double least = 0.0;
+        for (size_t i = 0; i < left.size(); i++) {
+            double change = 0.0;  // of the sum of squares
+            for (int r = 0; r < N; r++) {
+                const double k = kref[(size_t)r * N + left[i]];
+                change += k * (k + 2.0 * sum[r * 3 + left[i] % 3]);
+            }
+            if (i == 0 || change < least) best = i, least = change;
+        }
+        const int c = left[best];
+        for (int r = 0; r < N; r++) sum[r * 3 + c % 3] += kref[(size_t)r * N + c];
+        order.push_back((uint8_t)c);
+        left.erase(left.begin() + best);
+    }
+    return order;
+}
+
+// K_ref in the order of Ref::load, 16-byte pieces of a lane, lanes side by side.
+// BF16: value i = 16 m + 8 ks + v in two FP32 parts; FP32: i = 15 m + ks, then the
+// low parts [m][t][v] in BF16 (ks = 8 t + v).
+std::vector<uint8_t> mrhs_kref(const std::vector<double>& kref, const std::vector<uint8_t>& order, bool bf16)
+{
+    const uint32_t n_val = bf16 ? 64 : 60, per = bf16 ? 2 : 4, size = bf16 ? 8 : 4, n_low = bf16 ? 0 : 64;
+    std::vector<uint8_t> out((size_t)(n_val * size + n_low * 2) * 64, 0);
     for (uint32_t l = 0; l < 64; l++)
         for (uint32_t i = 0; i < n_val; i++) {
-            const uint32_t m = bf16 ? i / 16 : i / 15, row = std::min(16 * m + l % 16, 59u);
-            const uint32_t col = bf16 ? 32 * (i / 8 % 2) + 8 * (l / 16) + i % 8 : 4 * (i % 15) + l / 16;
+            const uint32_t m = bf16 ? i / 16 : i / 15, ks = i % 15, row = std::min(16 * m + l % 16, 59u);
+            const uint32_t col = bf16 ? 32 * (i / 8 % 2) + 8 * (l / 16) + i % 8 : order[4 * ks + l / 16];
             const double x = col < N ? kref[(size_t)row * N + col] : 0.0;
-            const float f = (float)x;
+            const float f = bf16 ? (float)x : cut(x);
             uint8_t* p = out.data() + ((size_t)(i / per * 64 + l) * per + i % per) * size;
             std::memcpy(p, &f, 4);
+            float low = (float)(x - (double)f);
             if (bf16) {
-                const float low = (float)(x - (double)f);
                 std::memcpy(p + 4, &low, 4);
+            } else {
+                if (low == 0.0f && f != 0.0f) low = std::copysign(FLT_MIN, f);
+                uint32_t b;
+                std::memcpy(&b, &low, 4);
+                const uint16_t h = (uint16_t)((b + 0x7fffu + ((b >> 16) & 1u)) >> 16);
+                std::memcpy(out.data() + 60 * 64 * 4 + ((size_t)(2 * m + ks / 8) * 64 + l) * 16 + ks % 8 * 2, &h, 2);
             }
         }
     return out;
+}
+
+void mrhs_factor(double s, bool bf16, float (&out)[2])
+{
+    const float hi = bf16 ? (float)s : cut(s);
+    double lo = s - (double)hi;
+    if (!bf16 && hi != 0.0f) {
+        lo = lo == 0.0 ? std::copysign(0x1p-100, hi) : std::ldexp(lo, -std::ilogb(hi));
+    }
+    out[0] = hi;
+    out[1] = (float)lo;
 }
 
 // Clusters: each of 8 contiguous shares of the elements by itself.  From its
@@ -393,7 +476,8 @@ std::vector<uint8_t> mrhs_kref(const std::vector<double>& kref, bool bf16)
 // On a structured hex20 mesh these are bricks of 2 x 2 x 2: 243 rows leave
 // instead of 480, 16 of them final.  n_max: 8 where that leaves 1,024 clusters
 // (four per CU), fewer below -- a wave takes the elements of a cluster in turn.
-MrhsClusters mrhs_clusters(const std::vector<uint32_t>& em, uint32_t n_elem, uint32_t n_total, bool bf16)
+MrhsClusters mrhs_clusters(const std::vector<uint32_t>& em, const std::vector<uint8_t>& order, uint32_t n_elem,
+                           uint32_t n_total, bool bf16)
 {
     constexpr uint32_t kShares = 8, kNodes = N / 3, kRows = kMrhsClusterRows - 1;
     const uint32_t n_max = std::min(8u, std::max(1u, n_elem / 1024u));
@@ -559,7 +643,7 @@ MrhsClusters mrhs_clusters(const std::vector<uint32_t>& em, uint32_t n_elem, uin
                     const uint32_t row = 16 * (y / 4) + 4 * q + y % 4;
                     C.slots[at * 64 + x] = (uint16_t)((row < N ? place[sl[row]] : dump) * COLS * 4);
                     const uint32_t col = bf16 ? 32 * (y / 8) + 8 * q + y % 8 : 4 * y + q;
-                    C.dofs[at * 64 + x] = d[col < N ? col : 0];
+                    C.dofs[at * 64 + x] = d[col >= N ? 0 : bf16 ? col : order[col]];
                 }
                 C.order[at] = el;
             }
