@@ -712,9 +712,12 @@ template <typename T> void put(DevBuf& b, const std::vector<T>& v)
 // columns 215 -> 182 us, 31^3 8 columns 89 -> 64 us.
 constexpr uint32_t kCongElemsF32 = 2048, kCongElemsBf16 = 20000;
 
-// the tables of a congruent 60-DoF group, elements in slot order
-void create_cong(const Op& op, const Group& g, const std::vector<uint32_t>& slot_of, bool bf16, amx_mrhs::Part& p)
+// the tables of a congruent 60-DoF group, elements in slot order; false (nothing
+// done) where its values ask for stored matrices
+bool create_cong(const Op& op, const Group& g, const std::vector<uint32_t>& slot_of, bool bf16, amx_mrhs::Part& p)
 {
+    int k = 0;
+    if (!mrhs_exponent(op.kref, op.scale, k)) return false;
     std::vector<uint32_t> em((size_t)p.n_elem * g.n);
     for (uint32_t j = 0; j < p.n_elem; j++) {
         const uint32_t* d = &op.local_map[op.eoff[g.elems[g.slot_elem[slot_of[j]]]]];
@@ -725,14 +728,14 @@ void create_cong(const Op& op, const Group& g, const std::vector<uint32_t>& slot
     std::vector<float> scale;
     for (uint32_t j = 0; j < p.n_elem; j++) {
         float f[2];
-        mrhs_factor(op.scale[g.elems[g.slot_elem[slot_of[c.order[j]]]]], bf16, f);
+        mrhs_factor(op.scale[g.elems[g.slot_elem[slot_of[c.order[j]]]]], k, bf16, f);
         scale.insert(scale.end(), f, f + 2);
     }
     p.ve_rows = c.row_dof.size();
     p.n_clusters = (uint32_t)c.table.size() / 4 - 1;
     p.max_rows = c.max_rows;
     p.n_ids = (uint32_t)c.ids.size();
-    put(p.kref, mrhs_kref(op.kref, order, bf16));
+    put(p.kref, mrhs_kref(op.kref, k, order, bf16));
     put(p.scale, scale);
     put(p.dofs, c.dofs);
     put(p.slots, c.slots);
@@ -742,6 +745,8 @@ void create_cong(const Op& op, const Group& g, const std::vector<uint32_t>& slot
     put(p.ids, c.ids);
     put(p.off, c.off);
     put(p.pos, c.pos);
+    p.cong = true;
+    return true;
 }
 
 // values per row of ve: 16-byte rows for any number of columns but one
@@ -956,9 +961,8 @@ int amx_mrhs_create(amx_op* const* ops, int n_ops, int precision, amx_mrhs** out
             AMX_REQUIRE((uint64_t)p.n_elem * g.n < (1ull << 32), AMX_NOT_IMPLEMENTED, "too many element rows");
             p.ve_row0 = 0;
             for (auto& q : m->parts) p.ve_row0 += q.ve_rows;
-            p.cong = g.cong && g.n == 60 && p.n_elem >= (m->bf16 ? amx::kCongElemsBf16 : amx::kCongElemsF32);
-            if (p.cong) {
-                amx::create_cong(op, g, slot_of, m->bf16, p);
+            if (g.cong && g.n == 60 && p.n_elem >= (m->bf16 ? amx::kCongElemsBf16 : amx::kCongElemsF32) &&
+                amx::create_cong(op, g, slot_of, m->bf16, p)) {
                 m->parts.push_back(std::move(p));
                 continue;
             }

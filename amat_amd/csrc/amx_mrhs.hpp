@@ -27,11 +27,14 @@ std::vector<uint8_t> mrhs_order(const std::vector<double>& kref);
 // em: n_elem x 60 DoFs below n_total
 MrhsClusters mrhs_clusters(const std::vector<uint32_t>& em, const std::vector<uint8_t>& order, uint32_t n_elem,
                            uint32_t n_total, bool bf16);
-// K_ref in A fragment order
-std::vector<uint8_t> mrhs_kref(const std::vector<double>& kref, const std::vector<uint8_t>& order, bool bf16);
-// a factor as the kernel takes it: s = out[0] + out[1] (FP32: out[0] cut towards
-// zero, out[1] divided by the power of two of out[0])
-void mrhs_factor(double s, bool bf16, float (&out)[2]);
+// k: the largest entry of K_ref times 2^-k is in [1, 2).  false where an entry or a
+// factor (times 2^k) leaves the range that the kernel takes.
+bool mrhs_exponent(const std::vector<double>& kref, const std::vector<double>& scale, int& k);
+// K_ref times 2^-k in A fragment order
+std::vector<uint8_t> mrhs_kref(const std::vector<double>& kref, int k, const std::vector<uint8_t>& order, bool bf16);
+// a factor as the kernel takes it: 2^k s = out[0] + out[1] (FP32: out[0] cut
+// towards zero, out[1] divided by the power of two of out[0])
+void mrhs_factor(double s, int k, bool bf16, float (&out)[2]);
 
 struct MrhsCongArgs {
     const void* kref;        // mrhs_kref

@@ -119,6 +119,9 @@ __device__ __forceinline__ uint32_t bf16_pair(float lo, float hi)
     return __builtin_amdgcn_perm(b + 0x7fffu + ((b >> 16) & 1u), a + 0x7fffu + ((a >> 16) & 1u), 0x07060302u);
 }
 
+// K_ref is held times a power of two, 2^-k, that brings its largest entry into
+// [1, 2), and the factors times 2^k (mrhs_exponent): both then fit FP32 wherever
+// their products do.
 template <bool BF16> struct Ref;
 // FP32: K_ref to 32 bits -- 24 in FP32, the 8 below them in BF16, whose product
 // with the leading bits of U takes 8 MFMAs beside 60 -- and the factor 2^k m to
@@ -392,6 +395,27 @@ void launch_mrhs_cong(bool bf16, const MrhsCongArgs& a, int cu_count, hipStream_
     AMX_HIP(hipGetLastError());
 }
 
+// Smaller entries and factors would lose their low parts below FP32's range, or
+// their products to it; a stored matrix takes those groups.
+bool mrhs_exponent(const std::vector<double>& kref, const std::vector<double>& scale, int& k)
+{
+    constexpr double kLeast = 0x1p-100, kMost = 0x1p126;
+    double most = 0.0;
+    for (double x : kref) {
+        if (!std::isfinite(x)) return false;
+        most = std::max(most, std::fabs(x));
+    }
+    if (most == 0.0) return false;
+    k = std::ilogb(most);
+    for (double x : kref)
+        if (x != 0.0 && std::fabs(std::ldexp(x, -k)) < kLeast) return false;
+    for (double x : scale) {
+        const double s = std::fabs(std::ldexp(x, k));
+        if (!(s == 0.0 || (s >= kLeast && s <= kMost))) return false;
+    }
+    return true;
+}
+
 // the FP32 value at or next to x towards zero
 static float cut(double x)
 {
@@ -431,7 +455,7 @@ std::vector<uint8_t> mrhs_order(const std::vector<double>& kref)
 // K_ref in the order of Ref::load, 16-byte pieces of a lane, lanes side by side.
 // BF16: value i = 16 m + 8 ks + v in two FP32 parts; FP32: i = 15 m + ks, then the
 // low parts [m][t][v] in BF16 (ks = 8 t + v).
-std::vector<uint8_t> mrhs_kref(const std::vector<double>& kref, const std::vector<uint8_t>& order, bool bf16)
+std::vector<uint8_t> mrhs_kref(const std::vector<double>& kref, int k, const std::vector<uint8_t>& order, bool bf16)
 {
     const uint32_t n_val = bf16 ? 64 : 60, per = bf16 ? 2 : 4, size = bf16 ? 8 : 4, n_low = bf16 ? 0 : 64;
     std::vector<uint8_t> out((size_t)(n_val * size + n_low * 2) * 64, 0);
@@ -439,7 +463,7 @@ std::vector<uint8_t> mrhs_kref(const std::vector<double>& kref, const std::vecto
         for (uint32_t i = 0; i < n_val; i++) {
             const uint32_t m = bf16 ? i / 16 : i / 15, ks = i % 15, row = std::min(16 * m + l % 16, 59u);
             const uint32_t col = bf16 ? 32 * (i / 8 % 2) + 8 * (l / 16) + i % 8 : order[4 * ks + l / 16];
-            const double x = col < N ? kref[(size_t)row * N + col] : 0.0;
+            const double x = col < N ? std::ldexp(kref[(size_t)row * N + col], -k) : 0.0;
             const float f = bf16 ? (float)x : cut(x);
             uint8_t* p = out.data() + ((size_t)(i / per * 64 + l) * per + i % per) * size;
             std::memcpy(p, &f, 4);
@@ -457,8 +481,9 @@ std::vector<uint8_t> mrhs_kref(const std::vector<double>& kref, const std::vecto
     return out;
 }
 
-void mrhs_factor(double s, bool bf16, float (&out)[2])
+void mrhs_factor(double s, int k, bool bf16, float (&out)[2])
 {
+    s = std::ldexp(s, k);
     const float hi = bf16 ? (float)s : cut(s);
     double lo = s - (double)hi;
     if (!bf16 && hi != 0.0f) {

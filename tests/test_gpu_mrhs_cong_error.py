@@ -62,3 +62,48 @@ def test_fp32_error_not_above_stored(torch_gpu, n, kind):
     cong, stored = (rel_l2(product(torch_gpu, mr, U), want) for mr in mrs)
     print(f"{kind} {n}^3: congruent {cong:.2e}, stored {stored:.2e}")
     assert cong <= stored
+
+
+@pytest.mark.parametrize("n,precision", [(14, PREC.FP32), (28, PREC.BF16)])
+@pytest.mark.parametrize("factor", [1e-45, 1e45])
+def test_factors_beyond_fp32(torch_gpu, factor, n, precision):
+    """K_ref or the factors outside FP32's range, their products inside: powers of
+    two (exact) change nothing."""
+    p = problems.elasticity_hex20(n)
+    f = 2.0 ** round(np.log2(factor))
+    q = dataclasses.replace(p, k_ref=p.k_ref * f, scale=p.scale / f)
+    U = fields(p, "random", 5).astype(np.float32)
+    mr, mq = (MultiRHS([r.build_operator(aMatFree, Maps)], precision) for r in (p, q))
+    np.testing.assert_array_equal(product(torch_gpu, mq, U), product(torch_gpu, mr, U))
+
+
+@pytest.mark.parametrize("which", ["entry", "factor"])
+def test_values_too_far_apart_for_parts(torch_gpu, which):
+    """A K_ref entry or a factor 2^-110 of the largest: the group takes stored
+    matrices (FP32 bar of the other multi-RHS products)."""
+    p = problems.elasticity_hex20(14)
+    k, s = p.k_ref.copy(), p.scale.copy()
+    if which == "entry":
+        k[3, 7] = k[7, 3] = 2.0 ** -110 * np.abs(k).max()
+    else:
+        s[5] = 2.0 ** -110
+    p = dataclasses.replace(p, k_ref=k, scale=s)
+    U = fields(p, "random", 3).astype(np.float32)
+    ops, mrs = pair(p, PREC.FP32)
+    cong, stored = (product(torch_gpu, mr, U) for mr in mrs)
+    np.testing.assert_array_equal(cong, stored)
+    assert rel_l2(cong, exact(p, U.astype(np.float64))) <= 2e-7
+
+
+def test_infinities_as_stored(torch_gpu):
+    p = problems.elasticity_hex20(14)
+    ops, mrs = pair(p, PREC.FP32)
+    U = fields(p, "random", 6).astype(np.float32)
+    d = int(p.gmap[1400, 31])
+    U[d, :5] = [np.inf, -np.inf, np.nan, np.inf, 3e38]
+    U[int(p.gmap[1400, 2]), 3] = np.inf
+    cong, stored = (product(torch_gpu, mr, U) for mr in mrs)
+    assert np.isinf(stored).any() and np.isnan(stored).any()
+    np.testing.assert_array_equal(np.isnan(cong), np.isnan(stored))
+    for sign in (np.isposinf, np.isneginf):
+        np.testing.assert_array_equal(sign(cong), sign(stored))
