@@ -42,6 +42,7 @@ namespace amx {
 namespace {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -112,7 +113,7 @@ __device__ __forceinline__ void load_slots(const MrhsCongArgs& a, uint32_t e, ui
 }
 
 // two values rounded to BF16 (nearest even; in integers, half the cost of the
-// conversion instructions)
+// conversion instructions; no NaN, whose largest payloads would carry into zero)
 __device__ __forceinline__ uint32_t bf16_pair(float lo, float hi)
 {
     const uint32_t a = __float_as_uint(lo), b = __float_as_uint(hi);
@@ -216,7 +217,8 @@ template <> struct Ref<true> {
         for (int ks = 0; ks < 2; ks++) {
             u32x4 b;
 #pragma unroll
-            for (int j = 0; j < 4; j++) b[j] = bf16_pair(B.b[8 * ks + 2 * j], B.b[8 * ks + 2 * j + 1]);
+            for (int j = 0; j < 4; j++)
+                b[j] = __builtin_bit_cast(uint32_t, bf16x2{(__bf16)B.b[8 * ks + 2 * j], (__bf16)B.b[8 * ks + 2 * j + 1]});
 #pragma unroll
             for (int m = 0; m < 4; m++) {
                 float x[8];

@@ -107,3 +107,18 @@ def test_infinities_as_stored(torch_gpu):
     np.testing.assert_array_equal(np.isnan(cong), np.isnan(stored))
     for sign in (np.isposinf, np.isneginf):
         np.testing.assert_array_equal(sign(cong), sign(stored))
+
+
+@pytest.mark.parametrize("bits", [0x7FC00000, 0x7FFFFFFF, 0xFFFFFFFF])
+def test_bf16_nan_stays_nan(torch_gpu, bits):
+    """NaN of any payload in U (BF16 rounding in integers carries the largest into
+    a zero) reaches every row of its elements."""
+    p = problems.elasticity_hex20(28)
+    mr = MultiRHS([p.build_operator(aMatFree, Maps)], PREC.BF16)
+    U = fields(p, "random", 3).astype(np.float32)
+    d = int(p.gmap[11000, 31])
+    U.view(np.uint32)[d, 1] = bits
+    V = product(torch_gpu, mr, U)
+    rows = np.unique(p.gmap[(p.gmap == d).any(axis=1)])
+    assert np.isnan(V[rows.astype(np.int64), 1]).all()
+    assert not np.isnan(V[:, [0, 2]]).any()
