@@ -647,8 +647,13 @@ struct amx_mrhs {
     int rhs_tile = 32, wpb = 4;  // NT * 32 columns per wave, waves per block
     int chunked = 1;             // work split inside an XCD slice: 1 contiguous chunk per wave, 0 interleaved
     int scatter = AMX_SCATTER_ATOMIC;
-    DevBuf ve;                   // deterministic scatter: element rows of all parts x nrhs
-    DevBuf rows;                 // the same for the atomic scatter where it takes the two passes
+    // Element rows of all parts x nrhs (two passes).  Calls on other streams and
+    // threads may run at the same time: the buffer passes from one to the next
+    // by an event.  One that a caller's graph was captured with is never freed
+    // before the handle; the handle's own graph has its own.
+    DevBuf rows, graph_rows;
+    std::vector<DevBuf> kept;        // outgrown, but captured
+    bool captured = false;           // rows, in a caller's graph
     hipEvent_t rows_free = nullptr;  // recorded after the last use of rows
     std::mutex rows_mutex;
     struct Part {
@@ -757,15 +762,6 @@ uint64_t ve_bytes(const amx_mrhs& m, int nrhs)
     uint64_t rows = 0;
     for (auto& p : m.parts) rows += p.ve_rows;
     return rows * (uint64_t)ve_stride(nrhs) * 4;
-}
-
-// element-row buffer of the deterministic scatter (allocated outside launches,
-// so a captured graph never allocates)
-void prepare(amx_mrhs& m, int nrhs)
-{
-    if (m.scatter != AMX_SCATTER_DETERMINISTIC) return;
-    const uint64_t bytes = std::max<uint64_t>(ve_bytes(m, nrhs), 4);
-    if (m.ve.bytes < bytes) m.ve.alloc(bytes);
 }
 
 // one launch over the parts, or several where their threads pass 32 bits
@@ -887,38 +883,70 @@ void launch(amx_mrhs& m, int nrhs, const float* const* U, float* const* V, float
 // atomics keeps the memory.
 constexpr uint64_t kAtomicVeMin = 32ull << 20, kAtomicVeMax = 2ull << 30;
 
-void mrhs_apply(amx_mrhs& m, int nrhs, const float* const* U, float* const* V, hipStream_t s)
+bool two_passes(const amx_mrhs& m, uint64_t bytes)
 {
-    if (m.scatter == AMX_SCATTER_DETERMINISTIC) {
-        prepare(m, nrhs);
-        launch(m, nrhs, U, V, m.ve.as<float>(), s);
-        return;
-    }
-    // calls on other streams and threads may run at the same time: the buffer
-    // passes from one to the next by an event.  A capture (which outlives the
-    // buffer) and a failed allocation leave the call with atomics.
-    const uint64_t bytes = ve_bytes(m, nrhs);
+    if (m.scatter == AMX_SCATTER_DETERMINISTIC) return true;
     bool clusters = false;
     for (auto& p : m.parts) clusters |= p.cong;
+    return bytes && (clusters || bytes >= kAtomicVeMin) && bytes <= kAtomicVeMax;
+}
+
+// b with `bytes` at least.  false: the atomic scatter could not have them
+bool ready(amx_mrhs& m, DevBuf& b, uint64_t bytes)
+{
+    bytes = std::max<uint64_t>(bytes, 4);
+    if (b.bytes >= bytes) return true;
+    const bool must = m.scatter == AMX_SCATTER_DETERMINISTIC;
+    if (&b == &m.rows && m.captured) {
+        m.kept.push_back(std::move(b));
+        m.captured = false;
+    }
+    b.release();
+    if (must) {
+        b.alloc(bytes);
+    } else if (hipMalloc(&b.p, bytes) == hipSuccess) {
+        b.bytes = bytes;
+    } else {
+        (void)hipGetLastError();
+        b.p = nullptr;
+        return false;
+    }
+    return true;
+}
+
+void mrhs_apply(amx_mrhs& m, int nrhs, const float* const* U, float* const* V, hipStream_t s)
+{
+    const uint64_t bytes = ve_bytes(m, nrhs);
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (bytes && (clusters || bytes >= kAtomicVeMin) && bytes <= kAtomicVeMax && hipStreamIsCapturing(s, &st) == hipSuccess &&
-        st == hipStreamCaptureStatusNone) {
+    if (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone) {
+        // captured by the caller: the atomic scatter adds into V, the buffer of the
+        // deterministic one has to be there (an application with as many columns
+        // before) unless the caller's kind of capture lets it allocate
+        (void)hipGetLastError();
+        if (m.scatter != AMX_SCATTER_DETERMINISTIC) return launch(m, nrhs, U, V, nullptr, s);
         std::lock_guard<std::mutex> lock(m.rows_mutex);
-        if (!m.rows_free && hipEventCreateWithFlags(&m.rows_free, hipEventDisableTiming) != hipSuccess)
-            m.rows_free = nullptr;
-        if (m.rows_free && m.rows.bytes < bytes) {
-            m.rows.release();
-            if (hipMalloc(&m.rows.p, bytes) == hipSuccess) m.rows.bytes = bytes;
-            else m.rows.p = nullptr;
+        if (m.rows.bytes < std::max<uint64_t>(bytes, 4)) {
+            if (m.captured) m.kept.push_back(std::move(m.rows));
+            m.rows.alloc(std::max<uint64_t>(bytes, 4));
         }
-        if (m.rows_free && m.rows.bytes >= bytes) {
+        m.captured = true;
+        return launch(m, nrhs, U, V, m.rows.as<float>(), s);
+    }
+    if (two_passes(m, bytes)) {
+        std::lock_guard<std::mutex> lock(m.rows_mutex);
+        if (!m.rows_free) AMX_HIP(hipEventCreateWithFlags(&m.rows_free, hipEventDisableTiming));
+        if (ready(m, m.rows, bytes)) {
             AMX_HIP(hipStreamWaitEvent(s, m.rows_free, 0));
-            launch(m, nrhs, U, V, m.rows.as<float>(), s);
+            try {
+                launch(m, nrhs, U, V, m.rows.as<float>(), s);
+            } catch (...) {
+                (void)hipEventRecord(m.rows_free, s);
+                throw;
+            }
             AMX_HIP(hipEventRecord(m.rows_free, s));
             return;
         }
     }
-    (void)hipGetLastError();
     launch(m, nrhs, U, V, nullptr, s);
 }
 
@@ -1137,12 +1165,13 @@ int amx_mrhs_graph_capture(amx_mrhs* m, int nrhs, const float* const* U, float* 
         AMX_REQUIRE(stream != nullptr, AMX_INVALID_ARGUMENT, "capture needs a non-default stream");
         amx::DeviceGuard dg(m->device);
         hipStream_t s = static_cast<hipStream_t>(stream);
-        amx::prepare(*m, nrhs);
         if (m->exec) { (void)hipGraphExecDestroy(m->exec); m->exec = nullptr; }
         if (m->graph) { (void)hipGraphDestroy(m->graph); m->graph = nullptr; }
+        const uint64_t bytes = amx::ve_bytes(*m, nrhs);
+        const bool rows = m->scatter == AMX_SCATTER_DETERMINISTIC && amx::ready(*m, m->graph_rows, bytes);
         AMX_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
         try {
-            amx::launch(*m, nrhs, U, V, m->scatter == AMX_SCATTER_DETERMINISTIC ? m->ve.as<float>() : nullptr, s);
+            amx::launch(*m, nrhs, U, V, rows ? m->graph_rows.as<float>() : nullptr, s);
         } catch (...) {
             hipGraph_t g;
             (void)hipStreamEndCapture(s, &g);

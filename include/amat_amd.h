@@ -488,10 +488,15 @@ int amx_mrhs_destroy(amx_mrhs* m);
 int amx_mrhs_set_tiles(amx_mrhs* m, int rhs_tile, int waves_per_block, int work_split);
 int amx_mrhs_get_tiles(const amx_mrhs* m, int* rhs_tile, int* waves_per_block, int* work_split);
 /* AMX_SCATTER_ATOMIC (default; order of the sums not fixed, takes the faster of
- * the two while the row buffer of the other stays within 2 GiB) or
- * AMX_SCATTER_DETERMINISTIC. */
+ * the two while the row buffer of the other stays within 2 GiB) or AMX_SCATTER_DETERMINISTIC.  A handle keeps the row buffer of
+ * its largest application until it is destroyed; applications that use it run
+ * one after the other, also on several streams. */
 int amx_mrhs_set_scatter(amx_mrhs* m, int scatter);
-/* U[i], V[i]: device arrays of operator i (n_ops of each).  V is overwritten. */
+/* U[i], V[i]: device arrays of operator i (n_ops of each).  V is overwritten.
+ * In a caller's stream capture the atomic scatter adds into V; the deterministic
+ * one uses the handle's row buffer, which an application with as many columns
+ * has to have made before, and the caller orders the replays and the handle's
+ * other applications. */
 int amx_mrhs_apply_dev(amx_mrhs* m, int nrhs, const float* const* U, float* const* V, void* stream);
 /* Times every launch shape (reps launches each) on the given arrays, keeps
  * the fastest; results[18] (may be NULL) receives the mean ms per launch in
@@ -499,8 +504,9 @@ int amx_mrhs_apply_dev(amx_mrhs* m, int nrhs, const float* const* U, float* cons
  * shape was skipped). */
 int amx_mrhs_autotune(amx_mrhs* m, int nrhs, const float* const* U, float* const* V, int reps,
                       double* results, void* stream);
-/* Captures one apply (zero fill + persistent launch) into a HIP graph bound to
- * these arrays; stream must not be the default stream. */
+/* Captures one apply into a HIP graph bound to these arrays (deterministic
+ * scatter: with a row buffer of its own; the atomic scatter adds into V); stream
+ * must not be the default stream. */
 int amx_mrhs_graph_capture(amx_mrhs* m, int nrhs, const float* const* U, float* const* V, void* stream);
 int amx_mrhs_graph_launch(amx_mrhs* m, void* stream);
 

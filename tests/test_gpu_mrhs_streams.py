@@ -1,0 +1,97 @@
+"""The row buffer of the multi-RHS products between streams, graphs and calls
+with more columns: every product equals the one formed alone, bit for bit (the
+two passes sum in a fixed order)."""
+import pytest
+
+from amat_amd import PREC, SCATTER, Maps, MultiRHS, aMatFree, problems
+
+pytestmark = pytest.mark.gpu
+
+
+def make(n, scatter):
+    p = problems.elasticity_hex20(n)
+    mr = MultiRHS([p.build_operator(aMatFree, Maps)], PREC.FP32)
+    mr.set_scatter(scatter)
+    return p, mr
+
+
+def rhs(torch, p, nrhs, seed):
+    return torch.rand(p.n_dofs, nrhs, device="cuda", generator=torch.Generator("cuda").manual_seed(seed)) - 0.5
+
+
+def alone(torch, n, U):
+    """The deterministic product by a handle of its own."""
+    p, mr = make(n, SCATTER.DETERMINISTIC)
+    V = torch.full_like(U, float("nan"))
+    mr.apply_dev(U.shape[1], [U], [V], torch.cuda.current_stream())
+    torch.cuda.synchronize()
+    return V
+
+
+@pytest.mark.parametrize("n", [6, 13])  # stored matrices, clusters
+@pytest.mark.parametrize("scatter", [SCATTER.DETERMINISTIC])
+def test_graph_keeps_its_rows(torch_gpu, n, scatter):
+    """The handle's graph, replayed after applications with more columns (clusters:
+    the atomic scatter's two passes, as in the calls that are not captured)."""
+    torch = torch_gpu
+    p, mr = make(n, scatter)
+    U, st = rhs(torch, p, 5, 1), torch.cuda.Stream()
+    V = torch.full_like(U, float("nan"))
+    want = alone(torch, n, U)
+    torch.cuda.synchronize()
+    mr.graph_capture(5, [U], [V], st)
+    for nrhs in (64, 200):
+        wide = rhs(torch, p, nrhs, 2)
+        out = torch.empty_like(wide)
+        mr.apply_dev(nrhs, [wide], [out], torch.cuda.current_stream())
+        fill = [torch.full((1 << 18,), float("nan"), device="cuda") for _ in range(16)]  # where freed rows would lie
+        V.fill_(float("nan"))
+        torch.cuda.synchronize()
+        mr.graph_launch(st)
+        torch.cuda.synchronize()
+        if scatter == SCATTER.DETERMINISTIC or n == 13:
+            assert torch.equal(V, want)
+        else:  # few rows: FP32 atomics, the bar of the other multi-RHS products
+            assert float(torch.linalg.norm(V - want) / torch.linalg.norm(want)) <= 2e-6
+        assert all(torch.isnan(f).all() for f in fill)
+
+
+@pytest.mark.parametrize("n", [6, 13])
+def test_callers_graph_keeps_its_rows(torch_gpu, n):
+    torch = torch_gpu
+    p, mr = make(n, SCATTER.DETERMINISTIC)
+    U = rhs(torch, p, 5, 1)
+    V = torch.full_like(U, float("nan"))
+    want = alone(torch, n, U)
+    mr.apply_dev(5, [U], [V], torch.cuda.current_stream())  # makes the buffer
+    torch.cuda.synchronize()
+    graph, st = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.graph(graph, stream=st):
+        mr.apply_dev(5, [U], [V], torch.cuda.current_stream())
+    for nrhs in (64, 200):
+        wide = rhs(torch, p, nrhs, 2)
+        out = torch.empty_like(wide)
+        mr.apply_dev(nrhs, [wide], [out], torch.cuda.current_stream())
+        V.fill_(float("nan"))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(V, want)
+
+
+@pytest.mark.parametrize("n", [6, 13])
+def test_deterministic_on_several_streams(torch_gpu, n):
+    torch = torch_gpu
+    p, mr = make(n, SCATTER.DETERMINISTIC)
+    U = [rhs(torch, p, 100, k) for k in range(4)]
+    V = [torch.full_like(u, float("nan")) for u in U]
+    want = [alone(torch, n, u) for u in U]
+    streams = [torch.cuda.Stream() for _ in U]
+    torch.cuda.synchronize()
+    for _ in range(5):
+        for u, v, s in zip(U, V, streams):
+            mr.apply_dev(100, [u], [v], s)
+    torch.cuda.synchronize()
+    for v, w in zip(V, want):
+        assert torch.equal(v, w)
+
