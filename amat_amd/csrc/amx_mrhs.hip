@@ -891,12 +891,20 @@ bool two_passes(const amx_mrhs& m, uint64_t bytes)
     return bytes && (clusters || bytes >= kAtomicVeMin) && bytes <= kAtomicVeMax;
 }
 
+// A capture in another thread does not forbid this one to allocate.
+struct RelaxedCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    RelaxedCapture() { AMX_HIP(hipThreadExchangeStreamCaptureMode(&mode)); }
+    ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
 // b with `bytes` at least.  false: the atomic scatter could not have them
 bool ready(amx_mrhs& m, DevBuf& b, uint64_t bytes)
 {
     bytes = std::max<uint64_t>(bytes, 4);
     if (b.bytes >= bytes) return true;
     const bool must = m.scatter == AMX_SCATTER_DETERMINISTIC;
+    RelaxedCapture relaxed;
     if (&b == &m.rows && m.captured) {
         m.kept.push_back(std::move(b));
         m.captured = false;
@@ -934,7 +942,10 @@ void mrhs_apply(amx_mrhs& m, int nrhs, const float* const* U, float* const* V, h
     }
     if (two_passes(m, bytes)) {
         std::lock_guard<std::mutex> lock(m.rows_mutex);
-        if (!m.rows_free) AMX_HIP(hipEventCreateWithFlags(&m.rows_free, hipEventDisableTiming));
+        if (!m.rows_free) {
+            RelaxedCapture relaxed;
+            AMX_HIP(hipEventCreateWithFlags(&m.rows_free, hipEventDisableTiming));
+        }
         if (ready(m, m.rows, bytes)) {
             AMX_HIP(hipStreamWaitEvent(s, m.rows_free, 0));
             try {

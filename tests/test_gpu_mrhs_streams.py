@@ -1,6 +1,9 @@
 """The row buffer of the multi-RHS products between streams, graphs and calls
 with more columns: every product equals the one formed alone, bit for bit (the
 two passes sum in a fixed order)."""
+import threading
+
+import numpy as np
 import pytest
 
 from amat_amd import PREC, SCATTER, Maps, MultiRHS, aMatFree, problems
@@ -95,3 +98,36 @@ def test_deterministic_on_several_streams(torch_gpu, n):
     for v, w in zip(V, want):
         assert torch.equal(v, w)
 
+
+@pytest.mark.parametrize("scatter", [SCATTER.DETERMINISTIC, SCATTER.ATOMIC])
+def test_first_application_beside_a_capture(torch_gpu, scatter):
+    """The buffer is allocated while another thread captures (global mode): the
+    product is the two-pass one and the capture stays valid."""
+    torch = torch_gpu
+    p, mr = make(13, scatter)
+    U = rhs(torch, p, 32, 1)
+    V = torch.full_like(U, float("nan"))
+    want = alone(torch, 13, U)
+    x = torch.zeros(1000, device="cuda")
+    graph, st, other = torch.cuda.CUDAGraph(), torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    errors = []
+
+    def work():
+        try:
+            mr.apply_dev(32, [U], [V], other)
+        except Exception as e:
+            errors.append(e)
+    with torch.cuda.graph(graph, stream=st):
+        x.add_(1.0)
+        t = threading.Thread(target=work)
+        t.start()
+        t.join()
+        x.add_(1.0)
+    assert not errors
+    torch.cuda.synchronize()
+    assert torch.equal(V, want)
+    for k in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(x.cpu().numpy(), np.full(1000, 2.0 * (k + 1), np.float32))
