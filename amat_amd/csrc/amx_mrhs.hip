@@ -654,6 +654,7 @@ struct amx_mrhs {
     DevBuf rows, graph_rows;
     std::vector<DevBuf> kept;        // outgrown, but captured
     bool captured = false;           // rows, in a caller's graph
+    uint64_t denied = ~0ull;         // bytes that the atomic scatter could not have
     hipEvent_t rows_free = nullptr;  // recorded after the last use of rows
     std::mutex rows_mutex;
     struct Part {
@@ -879,8 +880,8 @@ void launch(amx_mrhs& m, int nrhs, const float* const* U, float* const* V, float
 // 24^3 hex20 + 20^3 hex8 (130 MB) 189 -> 133 us.  Below kAtomicVeMin the atomics
 // stay in the cache and the event costs more than they do (10^3 elements, 64
 // columns, 15 MB: 27 -> 32 us) -- but not with clusters, whose rows leave in
-// bursts (18^3, 17 columns: 76 -> 50 us).  Above kAtomicVeMax whoever asked for
-// atomics keeps the memory.
+// bursts (18^3, 17 columns: 76 -> 50 us).  Above kAtomicVeMax, or 1/16 of the
+// free memory, whoever asked for atomics keeps the memory.
 constexpr uint64_t kAtomicVeMin = 32ull << 20, kAtomicVeMax = 2ull << 30;
 
 bool two_passes(const amx_mrhs& m, uint64_t bytes)
@@ -898,13 +899,23 @@ struct RelaxedCapture {
     ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
 };
 
-// b with `bytes` at least.  false: the atomic scatter could not have them
+// b with `bytes` at least.  false: the atomic scatter is not to have them (a size
+// that was refused once is not asked for again)
 bool ready(amx_mrhs& m, DevBuf& b, uint64_t bytes)
 {
     bytes = std::max<uint64_t>(bytes, 4);
     if (b.bytes >= bytes) return true;
     const bool must = m.scatter == AMX_SCATTER_DETERMINISTIC;
+    if (!must && bytes >= m.denied) return false;
     RelaxedCapture relaxed;
+    if (!must) {
+        size_t free = 0, total = 0;
+        if (hipMemGetInfo(&free, &total) != hipSuccess || bytes > free / 16) {
+            (void)hipGetLastError();
+            m.denied = bytes;
+            return false;
+        }
+    }
     if (&b == &m.rows && m.captured) {
         m.kept.push_back(std::move(b));
         m.captured = false;
@@ -917,6 +928,7 @@ bool ready(amx_mrhs& m, DevBuf& b, uint64_t bytes)
     } else {
         (void)hipGetLastError();
         b.p = nullptr;
+        m.denied = bytes;
         return false;
     }
     return true;

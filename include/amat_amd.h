@@ -488,7 +488,8 @@ int amx_mrhs_destroy(amx_mrhs* m);
 int amx_mrhs_set_tiles(amx_mrhs* m, int rhs_tile, int waves_per_block, int work_split);
 int amx_mrhs_get_tiles(const amx_mrhs* m, int* rhs_tile, int* waves_per_block, int* work_split);
 /* AMX_SCATTER_ATOMIC (default; order of the sums not fixed, takes the faster of
- * the two while the row buffer of the other stays within 2 GiB) or AMX_SCATTER_DETERMINISTIC.  A handle keeps the row buffer of
+ * the two while the row buffer of the other stays within 2 GiB and 1/16 of the
+ * free memory) or AMX_SCATTER_DETERMINISTIC.  A handle keeps the row buffer of
  * its largest application until it is destroyed; applications that use it run
  * one after the other, also on several streams. */
 int amx_mrhs_set_scatter(amx_mrhs* m, int scatter);
