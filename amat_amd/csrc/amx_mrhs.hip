@@ -1191,7 +1191,7 @@ int amx_mrhs_graph_capture(amx_mrhs* m, int nrhs, const float* const* U, float* 
         if (m->exec) { (void)hipGraphExecDestroy(m->exec); m->exec = nullptr; }
         if (m->graph) { (void)hipGraphDestroy(m->graph); m->graph = nullptr; }
         const uint64_t bytes = amx::ve_bytes(*m, nrhs);
-        const bool rows = m->scatter == AMX_SCATTER_DETERMINISTIC && amx::ready(*m, m->graph_rows, bytes);
+        const bool rows = amx::two_passes(*m, bytes) && amx::ready(*m, m->graph_rows, bytes);
         AMX_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
         try {
             amx::launch(*m, nrhs, U, V, rows ? m->graph_rows.as<float>() : nullptr, s);

@@ -505,9 +505,8 @@ int amx_mrhs_apply_dev(amx_mrhs* m, int nrhs, const float* const* U, float* cons
  * shape was skipped). */
 int amx_mrhs_autotune(amx_mrhs* m, int nrhs, const float* const* U, float* const* V, int reps,
                       double* results, void* stream);
-/* Captures one apply into a HIP graph bound to these arrays (deterministic
- * scatter: with a row buffer of its own; the atomic scatter adds into V); stream
- * must not be the default stream. */
+/* Captures one apply into a HIP graph bound to these arrays, with a row buffer of
+ * its own; stream must not be the default stream. */
 int amx_mrhs_graph_capture(amx_mrhs* m, int nrhs, const float* const* U, float* const* V, void* stream);
 int amx_mrhs_graph_launch(amx_mrhs* m, void* stream);
 

@@ -32,7 +32,7 @@ def alone(torch, n, U):
 
 
 @pytest.mark.parametrize("n", [6, 13])  # stored matrices, clusters
-@pytest.mark.parametrize("scatter", [SCATTER.DETERMINISTIC])
+@pytest.mark.parametrize("scatter", [SCATTER.DETERMINISTIC, SCATTER.ATOMIC])
 def test_graph_keeps_its_rows(torch_gpu, n, scatter):
     """The handle's graph, replayed after applications with more columns (clusters:
     the atomic scatter's two passes, as in the calls that are not captured)."""
