@@ -635,8 +635,8 @@ class aMatFree:
 
 class MultiRHS:
     """Multi-RHS element products V_i = sum_e P_e^T K_e P_e U_i of several
-    finalized operators in one persistent MFMA launch (FP32 or BF16 storage,
-    FP32 accumulation).  U_i, V_i: float32 device tensors of n_total x nrhs."""
+    finalized operators in one persistent MFMA launch (congruent hex20 groups: one
+    each; FP32 or BF16 storage, FP32 accumulation).  U_i, V_i: float32 device tensors of n_total x nrhs."""
 
     TILE_SHAPES = [(rt, w, c) for rt in (32, 64, 128) for w in (1, 2, 4) for c in (0, 1)]
 

@@ -1143,13 +1143,18 @@ int amx_mrhs_autotune(amx_mrhs* m, int nrhs, const float* const* U, float* const
         hipEvent_t e0, e1;
         AMX_HIP(hipEventCreate(&e0));
         AMX_HIP(hipEventCreate(&e1));
+        bool tiled = false;  // clusters have no launch shape
+        for (auto& p : m->parts) tiled |= !p.cong && p.n_tiles;
         double best = 1e30;
         int brt = 32, bw = 4, bc = 1, idx = 0;
         for (int rt : {32, 64, 128}) {
             for (int w : {1, 2, 4}) {
                 for (int c : {0, 1}) {
                     double ms = 1e30;
-                    if (rt <= std::max(32, ((nrhs + 31) / 32) * 32)) {
+                    const bool applies = rt <= std::max(32, ((nrhs + 31) / 32) * 32);
+                    if (applies && !tiled && best < 1e30) {
+                        ms = best;  // the same launches
+                    } else if (applies) {
                         m->rhs_tile = rt;
                         m->wpb = w;
                         m->chunked = c;

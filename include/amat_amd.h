@@ -465,7 +465,7 @@ int amx_dev_dot2(const double* x, const double* y, uint64_t n, uint32_t n_blocks
 
 /* ------------------------------------------------ multi-RHS element products
  * V_i = sum_e P_e^T K_e P_e U_i for several operators i in ONE persistent
- * launch, each U_i / V_i a device array of n_total x nrhs floats (DoF-major,
+ * launch (congruent 60-DoF groups: a launch each), each U_i / V_i a device array of n_total x nrhs floats (DoF-major,
  * the nrhs values of a DoF contiguous).  The reference applies one vector at a
  * time (aMatFree::matvec, include/aMatFree.hpp:1681-1775; its GPU methods call
  * a batched GEMV per colour, include/aMatGpu.hpp:21-591); this is the same
@@ -478,7 +478,9 @@ int amx_dev_dot2(const double* x, const double* y, uint64_t n, uint32_t n_blocks
  * Element types: 8, 10, 20 and 60 DoFs per element, one type per operator. */
 typedef struct amx_mrhs amx_mrhs;
 /* Copies the operators' element matrices (from their FP64 storage) into the
- * MFMA layout of precision (AMX_PREC_FP32 or AMX_PREC_BF16).  The operators
+ * MFMA layout of precision (AMX_PREC_FP32 or AMX_PREC_BF16); of 60-DoF groups of
+ * 2,048 elements (BF16 20,000) and more that were given as K_e = scale[e] * k_ref,
+ * k_ref and the factors, unless their values are too far apart.  The operators
  * must be finalized, on one device; at most 8. */
 int amx_mrhs_create(amx_op* const* ops, int n_ops, int precision, amx_mrhs** out);
 int amx_mrhs_destroy(amx_mrhs* m);
@@ -500,7 +502,7 @@ int amx_mrhs_set_scatter(amx_mrhs* m, int scatter);
  * other applications. */
 int amx_mrhs_apply_dev(amx_mrhs* m, int nrhs, const float* const* U, float* const* V, void* stream);
 /* Times every launch shape (reps launches each) on the given arrays, keeps
- * the fastest; results[18] (may be NULL) receives the mean ms per launch in
+ * the fastest (where no operator has tiles, one time stands for all); results[18] (may be NULL) receives the mean ms per launch in
  * the order rhs_tile 32/64/128 x waves 1/2/4 x work_split 0/1 (1e30 where a
  * shape was skipped). */
 int amx_mrhs_autotune(amx_mrhs* m, int nrhs, const float* const* U, float* const* V, int reps,

@@ -131,3 +131,13 @@ def test_first_application_beside_a_capture(torch_gpu, scatter):
         graph.replay()
         torch.cuda.synchronize()
         np.testing.assert_array_equal(x.cpu().numpy(), np.full(1000, 2.0 * (k + 1), np.float32))
+
+
+def test_autotune_of_clusters_times_once(torch_gpu):
+    torch = torch_gpu
+    p, mr = make(13, SCATTER.DETERMINISTIC)
+    U = rhs(torch, p, 40, 1)
+    V = torch.empty_like(U)
+    res = mr.autotune(40, [U], [V], reps=3)
+    assert len(res) == 12 and len(set(res.values())) == 1   # 32 and 64 columns a wave
+    assert mr.tiles() == (32, 1, 0)
