@@ -648,14 +648,22 @@ struct amx_mrhs {
     int chunked = 1;             // work split inside an XCD slice: 1 contiguous chunk per wave, 0 interleaved
     int scatter = AMX_SCATTER_ATOMIC;
     // Element rows of all parts x nrhs (two passes).  Calls on other streams and
-    // threads may run at the same time: the buffer passes from one to the next
-    // by an event.  One that a caller's graph was captured with is never freed
-    // before the handle; the handle's own graph has its own.
-    DevBuf rows, graph_rows;
-    std::vector<DevBuf> kept;        // outgrown, but captured
-    bool captured = false;           // rows, in a caller's graph
+    // threads may run at the same time: a buffer passes from one to the next by an
+    // event.  Buffers that a caller's graph was captured with are its alone (kept);
+    // the handle's own graph has its own.
+    struct Rows {
+        DevBuf buf;
+        hipEvent_t free = nullptr;    // recorded after the last use
+        hipStream_t last = nullptr;   // the stream of that use
+        ~Rows()
+        {
+            if (free) (void)hipEventDestroy(free);
+        }
+    };
+    std::vector<std::unique_ptr<Rows>> rows;
+    DevBuf graph_rows;
+    std::vector<DevBuf> kept;
     uint64_t denied = ~0ull;         // bytes that the atomic scatter could not have
-    hipEvent_t rows_free = nullptr;  // recorded after the last use of rows
     std::mutex rows_mutex;
     struct Part {
         uint32_t n, n_elem, n_tiles, n_total;
@@ -675,7 +683,6 @@ struct amx_mrhs {
     int occupancy[256] = {};  // resident blocks per CU, by kernel variant
     ~amx_mrhs()
     {
-        if (rows_free) (void)hipEventDestroy(rows_free);
         if (exec) (void)hipGraphExecDestroy(exec);
         if (graph) (void)hipGraphDestroy(graph);
     }
@@ -916,10 +923,6 @@ bool ready(amx_mrhs& m, DevBuf& b, uint64_t bytes)
             return false;
         }
     }
-    if (&b == &m.rows && m.captured) {
-        m.kept.push_back(std::move(b));
-        m.captured = false;
-    }
     b.release();
     if (must) {
         b.alloc(bytes);
@@ -934,39 +937,73 @@ bool ready(amx_mrhs& m, DevBuf& b, uint64_t bytes)
     return true;
 }
 
+// A product that leaves the chip room beside it has a buffer for each of up to
+// kRowBuffers streams (13^3 elements, 17 columns, two streams in turn: 18.2 us
+// against 30.7 with one); larger ones share the first.
+constexpr size_t kRowBuffers = 4;
+constexpr uint64_t kSideBySide = 64ull << 20;
+
+// a buffer for a product on stream s, NULL: the atomic scatter is not to have one
+amx_mrhs::Rows* rows_for(amx_mrhs& m, uint64_t bytes, hipStream_t s)
+{
+    amx_mrhs::Rows* r = nullptr;
+    if (bytes <= kSideBySide) {
+        for (auto& x : m.rows)
+            if (x->last == s) r = x.get();
+        for (auto& x : m.rows)
+            if (!r && hipEventQuery(x->free) == hipSuccess) r = x.get();
+        (void)hipGetLastError();  // (not ready)
+    }
+    if (!r && !m.rows.empty() && (bytes > kSideBySide || m.rows.size() == kRowBuffers)) r = m.rows.front().get();
+    if (!r) {
+        RelaxedCapture relaxed;
+        std::unique_ptr<amx_mrhs::Rows> x(new amx_mrhs::Rows());
+        AMX_HIP(hipEventCreateWithFlags(&x->free, hipEventDisableTiming));
+        m.rows.push_back(std::move(x));
+        r = m.rows.back().get();
+    }
+    r->last = s;
+    return ready(m, r->buf, bytes) ? r : nullptr;
+}
+
+// the buffer of a deterministic product that the caller captures: an application
+// with as many columns before has made it, unless the caller's kind of capture
+// allows an allocation
+float* captured_rows(amx_mrhs& m, uint64_t bytes)
+{
+    bytes = std::max<uint64_t>(bytes, 4);
+    for (auto& b : m.kept)
+        if (b.bytes >= bytes) return b.as<float>();
+    DevBuf b;
+    for (auto& x : m.rows)
+        if (!b.p && x->buf.bytes >= bytes) b = std::move(x->buf);
+    if (!b.p) b.alloc(bytes);
+    m.kept.push_back(std::move(b));
+    return m.kept.back().as<float>();
+}
+
 void mrhs_apply(amx_mrhs& m, int nrhs, const float* const* U, float* const* V, hipStream_t s)
 {
     const uint64_t bytes = ve_bytes(m, nrhs);
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone) {
-        // captured by the caller: the atomic scatter adds into V, the buffer of the
-        // deterministic one has to be there (an application with as many columns
-        // before) unless the caller's kind of capture lets it allocate
+        // captured by the caller: the atomic scatter adds into V
         (void)hipGetLastError();
         if (m.scatter != AMX_SCATTER_DETERMINISTIC) return launch(m, nrhs, U, V, nullptr, s);
         std::lock_guard<std::mutex> lock(m.rows_mutex);
-        if (m.rows.bytes < std::max<uint64_t>(bytes, 4)) {
-            if (m.captured) m.kept.push_back(std::move(m.rows));
-            m.rows.alloc(std::max<uint64_t>(bytes, 4));
-        }
-        m.captured = true;
-        return launch(m, nrhs, U, V, m.rows.as<float>(), s);
+        return launch(m, nrhs, U, V, captured_rows(m, bytes), s);
     }
     if (two_passes(m, bytes)) {
         std::lock_guard<std::mutex> lock(m.rows_mutex);
-        if (!m.rows_free) {
-            RelaxedCapture relaxed;
-            AMX_HIP(hipEventCreateWithFlags(&m.rows_free, hipEventDisableTiming));
-        }
-        if (ready(m, m.rows, bytes)) {
-            AMX_HIP(hipStreamWaitEvent(s, m.rows_free, 0));
+        if (amx_mrhs::Rows* r = rows_for(m, bytes, s)) {
+            AMX_HIP(hipStreamWaitEvent(s, r->free, 0));
             try {
-                launch(m, nrhs, U, V, m.rows.as<float>(), s);
+                launch(m, nrhs, U, V, r->buf.as<float>(), s);
             } catch (...) {
-                (void)hipEventRecord(m.rows_free, s);
+                (void)hipEventRecord(r->free, s);
                 throw;
             }
-            AMX_HIP(hipEventRecord(m.rows_free, s));
+            AMX_HIP(hipEventRecord(r->free, s));
             return;
         }
     }

@@ -491,15 +491,14 @@ int amx_mrhs_set_tiles(amx_mrhs* m, int rhs_tile, int waves_per_block, int work_
 int amx_mrhs_get_tiles(const amx_mrhs* m, int* rhs_tile, int* waves_per_block, int* work_split);
 /* AMX_SCATTER_ATOMIC (default; order of the sums not fixed, takes the faster of
  * the two while the row buffer of the other stays within 2 GiB and 1/16 of the
- * free memory) or AMX_SCATTER_DETERMINISTIC.  A handle keeps the row buffer of
- * its largest application until it is destroyed; applications that use it run
- * one after the other, also on several streams. */
+ * free memory) or AMX_SCATTER_DETERMINISTIC.  A handle keeps its row buffers
+ * until it is destroyed: up to four of 64 MiB for products on several streams,
+ * one for larger products, which run one after the other. */
 int amx_mrhs_set_scatter(amx_mrhs* m, int scatter);
 /* U[i], V[i]: device arrays of operator i (n_ops of each).  V is overwritten.
  * In a caller's stream capture the atomic scatter adds into V; the deterministic
- * one uses the handle's row buffer, which an application with as many columns
- * has to have made before, and the caller orders the replays and the handle's
- * other applications. */
+ * one takes over a row buffer, which an application with as many columns has to
+ * have made before, and the caller orders the replays of such graphs. */
 int amx_mrhs_apply_dev(amx_mrhs* m, int nrhs, const float* const* U, float* const* V, void* stream);
 /* Times every launch shape (reps launches each) on the given arrays, keeps
  * the fastest (where no operator has tiles, one time stands for all); results[18] (may be NULL) receives the mean ms per launch in

@@ -141,3 +141,25 @@ def test_autotune_of_clusters_times_once(torch_gpu):
     res = mr.autotune(40, [U], [V], reps=3)
     assert len(res) == 12 and len(set(res.values())) == 1   # 32 and 64 columns a wave
     assert mr.tiles() == (32, 1, 0)
+
+
+@pytest.mark.parametrize("scatter", [SCATTER.DETERMINISTIC, SCATTER.ATOMIC])
+def test_more_streams_than_buffers(torch_gpu, scatter):
+    """Six streams, four buffers of products of few columns, one of a product above
+    64 MiB of rows; sizes in turn on every stream."""
+    torch = torch_gpu
+    p, mr = make(13, scatter)
+    cols = (5, 200, 17)
+    want = [alone(torch, 13, rhs(torch, p, c, c)) for c in cols]
+    U = [rhs(torch, p, c, c) for c in cols]
+    streams = [torch.cuda.Stream() for _ in range(6)]
+    V = [[torch.full_like(u, float("nan")) for u in U] for _ in streams]
+    torch.cuda.synchronize()
+    for k in range(9):
+        for i, st in enumerate(streams):
+            j = (i + k) % 3
+            mr.apply_dev(cols[j], [U[j]], [V[i][j]], st)
+    torch.cuda.synchronize()
+    for i in range(6):
+        for j in range(3):
+            assert torch.equal(V[i][j], want[j])
