@@ -673,6 +673,13 @@ class MultiRHS:
         call("amx_mrhs_get_tiles", self._h, C.byref(a), C.byref(b), C.byref(c))
         return a.value, b.value, c.value
 
+    def matrix_bytes(self) -> list[int]:
+        """Bytes of the element matrices (or K_ref and factors) that a product
+        reads, by operator."""
+        b = (C.c_uint64 * len(self.ops))()
+        call("amx_mrhs_get_matrix_bytes", self._h, b)
+        return list(b)
+
     def apply_dev(self, nrhs: int, U, V, stream=None):
         pu, pv = self._lists(U, V)
         call("amx_mrhs_apply_dev", self._h, int(nrhs), pu, pv, _stream_ptr(stream))

@@ -1161,6 +1161,14 @@ int amx_mrhs_get_tiles(const amx_mrhs* m, int* rhs_tile, int* waves_per_block, i
     });
 }
 
+int amx_mrhs_get_matrix_bytes(const amx_mrhs* m, uint64_t* bytes)
+{
+    return guarded(__func__, [&] {
+        AMX_REQUIRE(m && bytes, AMX_INVALID_ARGUMENT, "NULL argument");
+        for (auto& p : m->parts) *bytes++ = p.cong ? p.kref.bytes + p.scale.bytes : p.K.bytes;
+    });
+}
+
 int amx_mrhs_apply_dev(amx_mrhs* m, int nrhs, const float* const* U, float* const* V, void* stream)
 {
     return guarded(__func__, [&] {

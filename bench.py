@@ -418,11 +418,9 @@ def batch_mode(args) -> dict:
             v0 = torch.empty_like(u0)
             op.matvec_dev(v0, u0, torch.cuda.current_stream())
             errs.append(float(torch.linalg.norm(V[i][:, 0].double() - v0) / torch.linalg.norm(v0)))
-        # congruent 60-DoF groups of this many elements read K_ref and a factor per element, no matrices
-        cong = [p.k_ref is not None and p.dofs_per_elem == 60 and p.n_elem >= (2048 if sk == 4 else 20000)
-                for p in probs]
-        alg = sum(p.n_elem * ((4 if c else p.dofs_per_elem ** 2 * sk) + 4 * p.dofs_per_elem) + p.n_dofs * 8 * nrhs
-                  for p, c in zip(probs, cong))
+        # stored matrices, or K_ref and a factor per element
+        alg = sum(min(b, p.n_elem * p.dofs_per_elem ** 2 * sk) + p.n_elem * 4 * p.dofs_per_elem + p.n_dofs * 8 * nrhs
+                  for p, b in zip(probs, mr.matrix_bytes()))
         flops = sum(2 * p.n_elem * p.dofs_per_elem ** 2 * nrhs for p in probs)
         best = min(ms, ms_graph) if ms_graph == ms_graph else ms
         case = {"precision": prec_name, "scatter": sc_name, "nrhs": nrhs, "tile": list(mr.tiles()), "ms": ms,

@@ -489,6 +489,9 @@ int amx_mrhs_destroy(amx_mrhs* m);
  * run of element tiles of its XCD's share, 0: the waves interleave over it. */
 int amx_mrhs_set_tiles(amx_mrhs* m, int rhs_tile, int waves_per_block, int work_split);
 int amx_mrhs_get_tiles(const amx_mrhs* m, int* rhs_tile, int* waves_per_block, int* work_split);
+/* bytes[n_ops]: the element matrices (or k_ref and factors) that a product reads
+ * of each operator. */
+int amx_mrhs_get_matrix_bytes(const amx_mrhs* m, uint64_t* bytes);
 /* AMX_SCATTER_ATOMIC (default; order of the sums not fixed, takes the faster of
  * the two while the row buffer of the other stays within 2 GiB and 1/16 of the
  * free memory) or AMX_SCATTER_DETERMINISTIC.  A handle keeps its row buffers

@@ -122,3 +122,17 @@ def test_bf16_nan_stays_nan(torch_gpu, bits):
     rows = np.unique(p.gmap[(p.gmap == d).any(axis=1)])
     assert np.isnan(V[rows.astype(np.int64), 1]).all()
     assert not np.isnan(V[:, [0, 2]]).any()
+
+
+def test_matrix_bytes(torch_gpu):
+    """Around the sizes from which congruent groups read no matrices."""
+    ops = {n: problems.elasticity_hex20(*n).build_operator(aMatFree, Maps)
+           for n in ((12, 12, 14), (13, 13, 13), (27, 27, 27), (28, 28, 28))}
+    for (n, op) in ops.items():
+        E = n[0] * n[1] * n[2]
+        for prec, size, least in ((PREC.FP32, 4, 2048), (PREC.BF16, 2, 20000)):
+            b, = MultiRHS([op], prec).matrix_bytes()
+            if E < least:
+                assert b == E * 3600 * size
+            else:   # a factor in two parts per element, one matrix in two parts
+                assert 8 * E < b < 8 * E + 40000
