@@ -648,19 +648,17 @@ struct amx_mrhs {
     int chunked = 1;             // work split inside an XCD slice: 1 contiguous chunk per wave, 0 interleaved
     int scatter = AMX_SCATTER_ATOMIC;
     // Element rows of all parts x nrhs (two passes).  Calls on other streams and
-    // threads may run at the same time: a buffer passes from one to the next by an
-    // event.  Buffers that a caller's graph was captured with are its alone (kept);
-    // the handle's own graph has its own.
+    // threads may run at the same time: a buffer is one stream's, whose order is
+    // enough, or passes from one call to the next by an event (shared; 2 us a
+    // call).  Buffers that a caller's graph was captured with are its alone
+    // (kept); the handle's own graph has its own.
     struct Rows {
+        hipStream_t owner;
         DevBuf buf;
-        hipEvent_t free = nullptr;    // recorded after the last use
-        hipStream_t last = nullptr;   // the stream of that use
-        ~Rows()
-        {
-            if (free) (void)hipEventDestroy(free);
-        }
     };
-    std::vector<std::unique_ptr<Rows>> rows;
+    std::vector<Rows> rows;
+    DevBuf shared;
+    hipEvent_t shared_free = nullptr;  // recorded after the last use of shared
     DevBuf graph_rows;
     std::vector<DevBuf> kept;
     uint64_t denied = ~0ull;         // bytes that the atomic scatter could not have
@@ -683,6 +681,7 @@ struct amx_mrhs {
     int occupancy[256] = {};  // resident blocks per CU, by kernel variant
     ~amx_mrhs()
     {
+        if (shared_free) (void)hipEventDestroy(shared_free);
         if (exec) (void)hipGraphExecDestroy(exec);
         if (graph) (void)hipGraphDestroy(graph);
     }
@@ -937,33 +936,23 @@ bool ready(amx_mrhs& m, DevBuf& b, uint64_t bytes)
     return true;
 }
 
-// A product that leaves the chip room beside it has a buffer for each of up to
-// kRowBuffers streams (13^3 elements, 17 columns, two streams in turn: 18.2 us
-// against 30.7 with one); larger ones share the first.
+// Up to kRowBuffers streams have a buffer of their own (13^3 elements, 17 columns,
+// two streams in turn: 15.9 us against 30.7 with one shared); further streams and
+// products with more rows, beside whose time the event is nothing and beside
+// which little else fits on the chip, share one.
 constexpr size_t kRowBuffers = 4;
-constexpr uint64_t kSideBySide = 64ull << 20;
+constexpr uint64_t kOwnRows = 128ull << 20;
 
-// a buffer for a product on stream s, NULL: the atomic scatter is not to have one
-amx_mrhs::Rows* rows_for(amx_mrhs& m, uint64_t bytes, hipStream_t s)
+// the buffer of a product on stream s.  (hipStreamPerThread, one handle for every
+// thread's stream, says nothing about order.)
+DevBuf& rows_for(amx_mrhs& m, uint64_t bytes, hipStream_t s)
 {
-    amx_mrhs::Rows* r = nullptr;
-    if (bytes <= kSideBySide) {
-        for (auto& x : m.rows)
-            if (x->last == s) r = x.get();
-        for (auto& x : m.rows)
-            if (!r && hipEventQuery(x->free) == hipSuccess) r = x.get();
-        (void)hipGetLastError();  // (not ready)
-    }
-    if (!r && !m.rows.empty() && (bytes > kSideBySide || m.rows.size() == kRowBuffers)) r = m.rows.front().get();
-    if (!r) {
-        RelaxedCapture relaxed;
-        std::unique_ptr<amx_mrhs::Rows> x(new amx_mrhs::Rows());
-        AMX_HIP(hipEventCreateWithFlags(&x->free, hipEventDisableTiming));
-        m.rows.push_back(std::move(x));
-        r = m.rows.back().get();
-    }
-    r->last = s;
-    return ready(m, r->buf, bytes) ? r : nullptr;
+    if (bytes > kOwnRows || s == hipStreamPerThread) return m.shared;
+    for (auto& r : m.rows)
+        if (r.owner == s) return r.buf;
+    if (m.rows.size() == kRowBuffers) return m.shared;
+    m.rows.push_back({s, DevBuf()});
+    return m.rows.back().buf;
 }
 
 // the buffer of a deterministic product that the caller captures: an application
@@ -975,8 +964,9 @@ float* captured_rows(amx_mrhs& m, uint64_t bytes)
     for (auto& b : m.kept)
         if (b.bytes >= bytes) return b.as<float>();
     DevBuf b;
-    for (auto& x : m.rows)
-        if (!b.p && x->buf.bytes >= bytes) b = std::move(x->buf);
+    for (auto& r : m.rows)
+        if (!b.p && r.buf.bytes >= bytes) b = std::move(r.buf);
+    if (!b.p && m.shared.bytes >= bytes) b = std::move(m.shared);
     if (!b.p) b.alloc(bytes);
     m.kept.push_back(std::move(b));
     return m.kept.back().as<float>();
@@ -995,15 +985,22 @@ void mrhs_apply(amx_mrhs& m, int nrhs, const float* const* U, float* const* V, h
     }
     if (two_passes(m, bytes)) {
         std::lock_guard<std::mutex> lock(m.rows_mutex);
-        if (amx_mrhs::Rows* r = rows_for(m, bytes, s)) {
-            AMX_HIP(hipStreamWaitEvent(s, r->free, 0));
+        DevBuf& r = rows_for(m, bytes, s);
+        if (ready(m, r, bytes)) {
+            if (&r != &m.shared) return launch(m, nrhs, U, V, r.as<float>(), s);
+            if (!m.shared_free) {
+                // (for this device's queues alone: no fence for the host and other devices)
+                RelaxedCapture relaxed;
+                AMX_HIP(hipEventCreateWithFlags(&m.shared_free, hipEventDisableTiming | hipEventDisableSystemFence));
+            }
+            AMX_HIP(hipStreamWaitEvent(s, m.shared_free, 0));
             try {
-                launch(m, nrhs, U, V, r->buf.as<float>(), s);
+                launch(m, nrhs, U, V, r.as<float>(), s);
             } catch (...) {
-                (void)hipEventRecord(r->free, s);
+                (void)hipEventRecord(m.shared_free, s);
                 throw;
             }
-            AMX_HIP(hipEventRecord(r->free, s));
+            AMX_HIP(hipEventRecord(m.shared_free, s));
             return;
         }
     }

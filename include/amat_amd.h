@@ -495,8 +495,9 @@ int amx_mrhs_get_matrix_bytes(const amx_mrhs* m, uint64_t* bytes);
 /* AMX_SCATTER_ATOMIC (default; order of the sums not fixed, takes the faster of
  * the two while the row buffer of the other stays within 2 GiB and 1/16 of the
  * free memory) or AMX_SCATTER_DETERMINISTIC.  A handle keeps its row buffers
- * until it is destroyed: up to four of 64 MiB for products on several streams,
- * one for larger products, which run one after the other. */
+ * until it is destroyed: one of up to 128 MiB for each of the first four streams,
+ * one for other streams and larger products, which run one after the other.  A
+ * stream is not to be destroyed while an application on it runs. */
 int amx_mrhs_set_scatter(amx_mrhs* m, int scatter);
 /* U[i], V[i]: device arrays of operator i (n_ops of each).  V is overwritten.
  * In a caller's stream capture the atomic scatter adds into V; the deterministic

@@ -145,11 +145,11 @@ def test_autotune_of_clusters_times_once(torch_gpu):
 
 @pytest.mark.parametrize("scatter", [SCATTER.DETERMINISTIC, SCATTER.ATOMIC])
 def test_more_streams_than_buffers(torch_gpu, scatter):
-    """Six streams, four buffers of products of few columns, one of a product above
-    64 MiB of rows; sizes in turn on every stream."""
+    """Six streams, four with a buffer of their own, one for the others and for the
+    products above 128 MiB of rows; sizes in turn on every stream."""
     torch = torch_gpu
     p, mr = make(13, scatter)
-    cols = (5, 200, 17)
+    cols = (5, 320, 17)
     want = [alone(torch, 13, rhs(torch, p, c, c)) for c in cols]
     U = [rhs(torch, p, c, c) for c in cols]
     streams = [torch.cuda.Stream() for _ in range(6)]
@@ -163,3 +163,39 @@ def test_more_streams_than_buffers(torch_gpu, scatter):
     for i in range(6):
         for j in range(3):
             assert torch.equal(V[i][j], want[j])
+
+
+@pytest.mark.parametrize("scatter", [SCATTER.DETERMINISTIC, SCATTER.ATOMIC])
+def test_second_stream_beside_a_capture(torch_gpu, scatter):
+    """Products above 128 MiB of rows share one buffer: another stream uses it next,
+    while another thread's capture runs."""
+    torch = torch_gpu
+    p, mr = make(13, scatter)
+    U = rhs(torch, p, 320, 1)
+    want = alone(torch, 13, U)
+    V = [torch.full_like(U, float("nan")) for _ in range(2)]
+    x = torch.zeros(1000, device="cuda")
+    graph, streams = torch.cuda.CUDAGraph(), [torch.cuda.Stream() for _ in range(3)]
+    torch.cuda.synchronize()
+    mr.apply_dev(320, [U], [V[0]], streams[0])
+    errors = []
+
+    def work():
+        try:
+            for _ in range(3):
+                mr.apply_dev(320, [U], [V[1]], streams[1])
+                mr.apply_dev(320, [U], [V[0]], streams[0])
+        except Exception as e:
+            errors.append(e)
+    with torch.cuda.graph(graph, stream=streams[2]):
+        x.add_(1.0)
+        t = threading.Thread(target=work)
+        t.start()
+        t.join()
+        x.add_(1.0)
+    assert not errors
+    torch.cuda.synchronize()
+    assert torch.equal(V[0], want) and torch.equal(V[1], want)
+    graph.replay()
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(x.cpu().numpy(), np.full(1000, 2.0, np.float32))
