@@ -10,9 +10,9 @@
 //
 // What bounds it: the FP64 units, three unfused operations per entry (two
 // multiplications, one addition; FP32 / BF16: multiplication, conversion, FMA).
-// hex20 64^3, FP64: element kernel 824 -> 116 us (24 of 39.3 Tops/s), matvec
-// 892 -> 152 us; FP32 matvec 444 -> 142, BF16 377 -> 210 us; hex8 96^3 element
-// kernel 62 -> 20 us, matvec FP64 80 -> 38, FP32 55 -> 30 us.  Where few waves
+// hex20 64^3, FP64: element kernel 830 -> 108 us (26 of 39.3 Tops/s), matvec
+// 881 -> 147 us; FP32 matvec 403 -> 116, BF16 326 -> 182 us; hex8 96^3 element
+// kernel 59 -> 19 us, matvec FP64 77 -> 37, FP32 51 -> 29 us.  Where few waves
 // run (hex20 15^3) the time is latency: FP32 element kernel 9.2 -> 5.5 us.
 #include <hip/hip_runtime.h>
 

@@ -150,9 +150,10 @@ __global__ __launch_bounds__(256) void free_laplace_kernel(const RT* __restrict_
 // only.  p = w inv inv^T h is formed from the cofactors, one division per point.
 // Coordinates as in free_laplace_kernel; rule: [point][xi, weight].
 //
-// What bounds it: memory (41^3 cubes of 6, FP64: 153 MB, 28 us at 5.5 TB/s; VGPRs
-// allow 4 waves per SIMD).  Against sums over the 10 nodes at every point, at
-// ngt = 2: element kernel 46 -> 34 us, matvec FP64 65 -> 55 us, FP32 45 -> 35 us;
+// What bounds it: memory (41^3 cubes of 6, FP64: 153 MB at 5 TB/s; VGPRs allow 4
+// waves per SIMD).  Against sums over the 10 nodes at every point, at ngt = 2:
+// element kernel 38.5 -> 30.9 us, matvec FP64 56.5 -> 44.4 us (4 of it the gather),
+// FP32 41 -> 31 us;
 // relative L2 error 7.1e-16 -> 4.9e-16 (9^3 cubes), FP32 3.9e-7 -> 2.9e-7.
 template <typename RT> struct Tet10 {
     RT A[3], D[3], S[3];  // S: D_12, D_23, D_31
@@ -286,12 +287,14 @@ __global__ __launch_bounds__(256) void free_tet10_kernel(const RT* __restrict__ 
 // in flight (VGPRs; 4 waves per SIMD asked for in FP64 spill, 132 us).  Against
 // node-by-node sums (60 per point and direction, 440 LDS values per lane),
 // element kernel FP64 / matvec FP64 / matvec FP32:
-//   48^3, ngt = 3   176 -> 78 us   217 -> 110 us   147 -> 71 us
-//   48^3, ngt = 2    59 -> 53 us    86 ->  83 us    62 -> 55 us
-//   24^3, ngt = 3                   36 ->  20 us    27 -> 15 us
-//   24^3, ngt = 4                   75 ->  42 us    56 -> 27 us
-// Relative L2 error of the FP64 product (12^3): ngt = 2 2.5e-15 -> 4.5e-16,
-// ngt = 3 and 4 as before (9e-15, 2.1e-14: the digits of the rule).
+//   48^3, ngt = 3   160 -> 68 us   182 -> 87 us   134 -> 59 us
+//   48^3, ngt = 2    48 -> 47 us    71 -> 66 us    56 -> 47 us
+//   24^3, ngt = 3    29 -> 15 us    32 -> 16 us    23 -> 13 us
+//   24^3, ngt = 4    64 -> 36 us    67 -> 38 us    49 -> 23 us
+// Relative L2 error of the FP64 product against 64 bits with the same rule (12^3,
+// ngt = 2, 3, 4): 3.2e-15, 1.8e-15, 2.5e-15 -> 1.7e-16, 1.5e-16, 1.5e-16.  The
+// digits of the rule's weights put the product 5.7e-16, 1.06e-14 and 2.5e-14 off that
+// of an exact rule, whatever kernel forms it.
 constexpr uint32_t kH20Node[3][5] = {  // byte j: 8 * node of entry j (per line f-, f+, f0; then the edge pairs)
     {0x18400800u, 0x28205010u, 0x70303860u, 0x68784858u, 0x90988880u},
     {0x20581800u, 0x10087838u, 0x68302848u, 0x90889880u, 0x70605040u},

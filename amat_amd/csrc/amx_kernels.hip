@@ -801,12 +801,13 @@ __global__ __launch_bounds__(256) void ebe_generic_kernel(const KT* __restrict__
 // 0.135 ms, gather 49 -> 46 us).
 //   A window with fewer entries leaves out the loads that no thread needs (a
 // uniform test per 256): loads of the last entry by all took their turn in the
-// address units (matvecs of hex20 64^3 160 -> 153 us, tet10 48^3 133 -> 128 us).
+// address units (gathers of hex20 64^3 52 -> 43 us, tet10 48^3 32 -> 28 us; matvecs
+// 155 -> 145 and 92 -> 88 us).
 //   Window: 2,048 entries hold 256 DoFs of hex20 (4.6 entries each).  Above a mean
 // of 6 (tet10: 7.2, vertices 24) many blocks need a second one for little:
-// kGatherWide takes them at once (tet10 48^3 128 -> 126 us, 20^3 16.1 -> 13.9, BF16
-// 33^3 23.9 -> 22.7; hex20 64^3 would lose with it, 153 -> 156 us; hex8, at most 8
-// each, does with either: 96^3 37.9 and 37.7 us).
+// kGatherWide takes them at once (matvecs of tet10 48^3 88 -> 86 us, 20^3 13.9 -> 11.8,
+// BF16 33^3 24.3 -> 23.2; the gather of hex20 64^3 would lose with it, 43.3 -> 44.4
+// us; hex8, at most 8 each, does with either: 96^3 22.4 us).
 constexpr uint32_t kGatherWindow = 2048, kGatherWide = 3072;
 
 template <typename VT, int BC, uint32_t WINDOW = kGatherWindow>

@@ -16,8 +16,9 @@
 // Congruent groups of 60 DoFs (K_e = s_e K_ref) take no matrices and have a
 // kernel of their own (amx_mrhs_cong.hip).
 // The element rows reach V either through the deterministic two-pass scatter
-// (rows stored per element, then summed per DoF in ascending element order:
-// bit-reproducible, independent of the launch shape) or FP32 atomics.
+// (rows stored per element, then summed per DoF in ascending element order -- of
+// congruent groups per cluster, in ascending cluster order: bit-reproducible,
+// independent of the launch shape) or FP32 atomics.
 // Work split: every segment (operator) is cut into 8 contiguous slices, one per
 // XCD (workgroups are dispatched round-robin over the 8 XCDs), so elements that
 // share nodes run on the same L2.
@@ -716,12 +717,13 @@ template <typename T> void put(DevBuf& b, const std::vector<T>& v)
 }
 
 // Congruent 60-DoF groups take amx_mrhs_cong.hip from this many elements on; below,
-// the stored matrices are small and their kernel needs no clusters (two passes,
-// a hex8 mesh beside it, stored -> clusters).  FP32: 12^3 elements 17 columns in
-// atomics 24 -> 27 us, 14^3 33 -> 32 us and 128 columns 80 -> 66 us, 20^3 204 ->
-// 145 us.  BF16, which forms its matrices with every 16 columns: 20^3 17 columns
-// 42 -> 49 us, 26^3 50 columns 175 -> 175 us, 28^3 24 columns 94 -> 96 us, 64
-// columns 215 -> 182 us, 31^3 8 columns 89 -> 64 us.
+// the stored matrices are small and their kernel needs no clusters (a hex8 mesh
+// beside it, atomic scatter, stored -> clusters).  FP32: 10^3 elements 17 columns
+// 16.5 -> 19.9 us, 12^3 21.2 -> 23.3 us (128 columns 51 -> 46 us), 13^3 27.8 -> 26.7
+// us, 14^3 29.6 -> 27.9 us, 128 columns 72 -> 62 us.  BF16, which forms its matrices
+// with every 16 columns: 20^3 17 columns 40 -> 46 us, 26^3 50 columns 165 -> 174 us,
+// 27^3 24 columns 82 -> 84 us, 28^3 90 -> 88 us, 64 columns 210 -> 173 us, 31^3 8
+// columns 85 -> 60 us.
 constexpr uint32_t kCongElemsF32 = 2048, kCongElemsBf16 = 20000;
 
 // the tables of a congruent 60-DoF group, elements in slot order; false (nothing
@@ -882,11 +884,11 @@ void launch(amx_mrhs& m, int nrhs, const float* const* U, float* const* V, float
 
 // The atomic scatter may sum in any order, so it takes the two passes of the
 // deterministic one where their buffer is neither small nor a burden: 24 columns
-// in BF16 on 31^3 hex20 + 80 x 40 x 20 hex8 (210 MB) 215 -> 160 us, 64 in FP32 on
-// 24^3 hex20 + 20^3 hex8 (130 MB) 189 -> 133 us.  Below kAtomicVeMin the atomics
-// stay in the cache and the event costs more than they do (10^3 elements, 64
-// columns, 15 MB: 27 -> 32 us) -- but not with clusters, whose rows leave in
-// bursts (18^3, 17 columns: 76 -> 50 us).  Above kAtomicVeMax, or 1/16 of the
+// in BF16 on 31^3 hex20 + 80 x 40 x 20 hex8 (210 MB) 220 -> 151 us, 64 in FP32 on
+// 24^3 hex20 + 20^3 hex8 (130 MB) 195 -> 134 us.  Below kAtomicVeMin the atomics
+// stay in the cache and the second pass costs more than they do (10^3 elements, 64
+// columns, 15 MB: 24 -> 27 us) -- but not with clusters, whose rows leave in
+// bursts (18^3, 17 columns: 76 -> 47 us).  Above kAtomicVeMax, or 1/16 of the
 // free memory, whoever asked for atomics keeps the memory.
 constexpr uint64_t kAtomicVeMin = 32ull << 20, kAtomicVeMax = 2ull << 30;
 

@@ -12,19 +12,19 @@
 //   C lane l, register i: row 16 m + 4 (l/16) + i, column l % 16.
 // Rows 60..63 (tile m = 3) go to a dump row.
 //
-// What bounds it: FP32 the matrix cores -- 205 us of MFMA at 32768 elements x
+// What bounds it: FP32 the matrix cores -- 219 us of MFMA at 32768 elements x
 // 128 columns, at two waves per SIMD (VGPRs) that the loads, the sums in LDS and
 // the rows' way out only partly hide under it; BF16 forming the matrices (three
 // instructions per value and its rounding) and the rows.  Against a kernel that
 // reads the stored matrices and writes every element row (both passes of the
 // scatter, one hex8 mesh beside it):
-//   32^3, 128 columns, FP32   785 -> 592 us (of it 537 -> 430 and 254 -> 132)
-//   31^3,  24 columns, BF16   atomics 258 -> 165 us, two passes 176 -> 157 us
-//   28^3, 128 columns, BF16   atomics 560 -> 375 us
-//   24^3,  64 columns, FP32   atomics 213 -> 130 us
-//   31^3,   1 column,  FP32   two passes 136 -> 63 us, atomics 141 -> 66 us
-//   16^3,  50 columns, FP32    68 ->  59 us
-//   14^3, 128 columns, FP32    80 ->  66 us
+//   32^3, 128 columns, FP32   790 -> 607 us (of it 538 -> 454 and 254 -> 132)
+//   31^3,  24 columns, BF16   atomics 258 -> 150 us, two passes 172 -> 150 us
+//   28^3, 128 columns, BF16   atomics 559 -> 372 us
+//   24^3,  64 columns, FP32   atomics 208 -> 134 us
+//   31^3,   1 column,  FP32   two passes 127 -> 60 us, atomics 126 -> 59 us
+//   16^3,  50 columns, FP32    58 ->  57 us
+//   14^3, 128 columns, FP32    73 ->  62 us
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
