@@ -892,11 +892,16 @@ void launch(amx_mrhs& m, int nrhs, const float* const* U, float* const* V, float
 // free memory, whoever asked for atomics keeps the memory.
 constexpr uint64_t kAtomicVeMin = 32ull << 20, kAtomicVeMax = 2ull << 30;
 
-bool two_passes(const amx_mrhs& m, uint64_t bytes)
+bool two_passes(const amx_mrhs& m, uint64_t bytes, int nrhs, float* const* V)
 {
     if (m.scatter == AMX_SCATTER_DETERMINISTIC) return true;
     bool clusters = false;
     for (auto& p : m.parts) clusters |= p.cong;
+    // operators that share an output add up in it, which only atomics do
+    for (size_t i = 0; i < m.parts.size(); i++)
+        for (size_t j = 0; j < i; j++)
+            if (V[i] < V[j] + (uint64_t)m.parts[j].n_total * nrhs && V[j] < V[i] + (uint64_t)m.parts[i].n_total * nrhs)
+                return false;
     return bytes && (clusters || bytes >= kAtomicVeMin) && bytes <= kAtomicVeMax;
 }
 
@@ -985,7 +990,7 @@ void mrhs_apply(amx_mrhs& m, int nrhs, const float* const* U, float* const* V, h
         std::lock_guard<std::mutex> lock(m.rows_mutex);
         return launch(m, nrhs, U, V, captured_rows(m, bytes), s);
     }
-    if (two_passes(m, bytes)) {
+    if (two_passes(m, bytes, nrhs, V)) {
         std::lock_guard<std::mutex> lock(m.rows_mutex);
         DevBuf& r = rows_for(m, bytes, s);
         if (ready(m, r, bytes)) {
@@ -1240,7 +1245,7 @@ int amx_mrhs_graph_capture(amx_mrhs* m, int nrhs, const float* const* U, float* 
         if (m->exec) { (void)hipGraphExecDestroy(m->exec); m->exec = nullptr; }
         if (m->graph) { (void)hipGraphDestroy(m->graph); m->graph = nullptr; }
         const uint64_t bytes = amx::ve_bytes(*m, nrhs);
-        const bool rows = amx::two_passes(*m, bytes) && amx::ready(*m, m->graph_rows, bytes);
+        const bool rows = amx::two_passes(*m, bytes, nrhs, V) && amx::ready(*m, m->graph_rows, bytes);
         AMX_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
         try {
             amx::launch(*m, nrhs, U, V, rows ? m->graph_rows.as<float>() : nullptr, s);

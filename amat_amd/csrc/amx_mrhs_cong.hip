@@ -359,8 +359,9 @@ __global__ __launch_bounds__(64, 2) void mrhs_cong_kernel(MrhsCongArgs a)
             else
                 put_rows<4, false, WIDE>(W, cur.n_ve, a.ve, a.ve_ld, a.ve_ld, cur.col0,
                                          [&](uint32_t x) { return cur.ve0 + x; });
+            // (atomics: another operator may add into the same V)
             if (cur.n_dir)
-                put_rows<V4 ? 4 : 1, false, WIDE>(W + cur.n_ve * COLS, cur.n_dir, a.V, a.nrhs, a.nrhs, cur.col0,
+                put_rows<V4 ? 4 : 1, ATOMIC, WIDE>(W + cur.n_ve * COLS, cur.n_dir, a.V, a.nrhs, a.nrhs, cur.col0,
                                                   [&](uint32_t x) { return a.direct[cur.dir0 + x]; });
             lds_sync_wave();
             if (cur.item + step >= hi) return true;

@@ -499,7 +499,8 @@ int amx_mrhs_get_matrix_bytes(const amx_mrhs* m, uint64_t* bytes);
  * one for other streams and larger products, which run one after the other.  A
  * stream is not to be destroyed while an application on it runs. */
 int amx_mrhs_set_scatter(amx_mrhs* m, int scatter);
-/* U[i], V[i]: device arrays of operator i (n_ops of each).  V is overwritten.
+/* U[i], V[i]: device arrays of operator i (n_ops of each).  V is overwritten;
+ * with the atomic scatter, operators that share an array add up in it.
  * In a caller's stream capture the atomic scatter adds into V; the deterministic
  * one takes over a row buffer, which an application with as many columns has to
  * have made before, and the caller orders the replays of such graphs. */

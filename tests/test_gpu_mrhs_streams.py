@@ -199,3 +199,31 @@ def test_second_stream_beside_a_capture(torch_gpu, scatter):
     graph.replay()
     torch.cuda.synchronize()
     np.testing.assert_array_equal(x.cpu().numpy(), np.full(1000, 2.0, np.float32))
+
+
+@pytest.mark.parametrize("dims", [(6, 7), (13, 14)])   # stored matrices, clusters (and more than 32 MiB of rows)
+def test_atomic_operators_add_up_in_a_shared_output(torch_gpu, dims):
+    torch = torch_gpu
+    ops = [problems.elasticity_hex20(n).build_operator(aMatFree, Maps) for n in dims]
+    N = [problems.elasticity_hex20(n).n_dofs for n in dims]
+    mr, nrhs = MultiRHS(ops, PREC.FP32), 100
+    gen = torch.Generator("cuda").manual_seed(4)
+    U = [torch.rand(n, nrhs, device="cuda", generator=gen) - 0.5 for n in N]
+    V = [torch.empty_like(u) for u in U]
+    mr.set_scatter(SCATTER.DETERMINISTIC)
+    mr.apply_dev(nrhs, U, V, torch.cuda.current_stream())
+    want = V[1].clone()
+    want[:N[0]] += V[0]
+    mr.set_scatter(SCATTER.ATOMIC)
+    out = torch.full_like(U[1], float("nan"))
+    for graph in (False, True):
+        out.fill_(float("nan"))
+        if graph:
+            st = torch.cuda.Stream()
+            torch.cuda.synchronize()
+            mr.graph_capture(nrhs, U, [out, out], st)
+            mr.graph_launch(st)
+        else:
+            mr.apply_dev(nrhs, U, [out, out], torch.cuda.current_stream())
+        torch.cuda.synchronize()
+        assert float(torch.linalg.norm(out - want) / torch.linalg.norm(want)) <= 2e-6
