@@ -151,13 +151,20 @@ inline uint32_t free_nodes(int kind)
 {
     return kind == AMX_ELEM_HEX8_LAPLACE ? 8u : (kind == AMX_ELEM_HEX20_ELASTIC ? 20u : 10u);
 }
-// algorithmic FP64 flops of one FREE element application (amx_free.hip):
-// Laplace per point 30 n + 85 (Jacobian 18 n, h 6 n, output 6 n, inverse and
-// transforms 85); hex20 per point 1260 (Jacobian 360, H 360, output 360,
-// inverse, strain, stress and P 180)
+// flops of one FREE element application as the kernels of amx_free.hip do it:
+// hex8 per point 30 n + 85 (Jacobian 18 n, h 6 n, output 6 n, inverse and
+// transforms 85); tet10 per element 153 (coefficients of four fields, output) and
+// per point 160; hex20, n1 points per direction: per point 161 (inverse 42,
+// weight 2, strain, stress and P 117), for each of 9 (field, direction) twice 58
+// + 14 n1 + 6 n1^2 + 2 n1^3 (coefficients, derivatives of coordinates and u) and
+// once 58 + 19 n1 + 8 n1^2 + 3 n1^3 (output), and 120 sums over directions
 inline uint64_t free_flops_per_elem(int kind, uint32_t nq)
 {
-    return (uint64_t)nq * (kind == AMX_ELEM_HEX20_ELASTIC ? 1260u : 30u * free_nodes(kind) + 85u);
+    if (kind == AMX_ELEM_HEX8_LAPLACE) return (uint64_t)nq * (30u * free_nodes(kind) + 85u);
+    if (kind == AMX_ELEM_TET10_LAPLACE) return 153u + 160u * (uint64_t)nq;
+    uint64_t n1 = 1;
+    while (n1 * n1 * n1 < nq) n1++;
+    return 9u * (174u + 47u * n1 + 20u * n1 * n1 + 7u * nq) + 120u + 161u * (uint64_t)nq;
 }
 
 // RAII: make the handle's device current, restore the previous one on exit.

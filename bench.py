@@ -295,8 +295,8 @@ def free_mode(args) -> dict:
                 r["fp64_peak_frac"] = inf.flops / (ms_e * 1e-3) / FP64_PEAK
                 r["rel_l2_vs_stored"] = rel
             else:
-                elem_bytes = E * (60 * 60 * 8 + 4 * 60) + N * 8
-                r["element_kernel_hbm_frac"] = elem_bytes / (ms_e * 1e-3) / HBM_PEAK
+                # factors, map and u (K_e = E_e K_ref: no matrices are read)
+                r["element_kernel_hbm_frac"] = (inf.alg_bytes_fp64 - 8 * N) / (ms_e * 1e-3) / HBM_PEAK
             res[f"ngt{ngt}_{name}"] = r
             log(f"[free] ngt {ngt} {name}: {ms:.4f} ms/matvec ({N / ms / 1e6:.2f} GDoF/s), element kernel "
                 f"{ms_e:.4f} ms, gather {ms_g:.4f} ms, device {inf.device_bytes / 1e9:.2f} GB"

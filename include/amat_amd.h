@@ -210,7 +210,7 @@ typedef struct amx_op_info {
     uint64_t alg_bytes_fp64;    /* E(b + 4n) + 16 N, b = FP64 bytes read per element (8 n^2, 8 n(n+1)/2
                                    packed, the record size of near-symmetric records, 8 for a factor): one
                                    FP64 matvec's algorithmic HBM bytes */
-    uint64_t flops;             /* 2 sum_e n_e^2 per matvec */
+    uint64_t flops;             /* 2 sum_e n_e^2 per matvec (method 2: what its kernels do) */
     uint32_t packed_symmetric;  /* element groups stored as packed symmetric tiles */
     uint32_t near_symmetric;    /* element groups stored as near-symmetric records (FP64) */
 } amx_op_info;
