@@ -503,7 +503,8 @@ int amx_mrhs_set_scatter(amx_mrhs* m, int scatter);
  * with the atomic scatter, operators that share an array add up in it.
  * In a caller's stream capture the atomic scatter adds into V; the deterministic
  * one takes over a row buffer, which an application with as many columns has to
- * have made before, and the caller orders the replays of such graphs. */
+ * have made before; the caller orders the replays of such graphs, after that
+ * application too. */
 int amx_mrhs_apply_dev(amx_mrhs* m, int nrhs, const float* const* U, float* const* V, void* stream);
 /* Times every launch shape (reps launches each) on the given arrays, keeps
  * the fastest (where no operator has tiles, one time stands for all); results[18] (may be NULL) receives the mean ms per launch in

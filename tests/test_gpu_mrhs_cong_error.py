@@ -136,3 +136,15 @@ def test_matrix_bytes(torch_gpu):
                 assert b == E * 3600 * size
             else:   # a factor in two parts per element, one matrix in two parts
                 assert 8 * E < b < 8 * E + 40000
+
+
+@pytest.mark.parametrize("n,precision,bar", [(14, PREC.FP32, 1e-6), (28, PREC.BF16, 1e-2)])
+def test_unsymmetric_reference_matrix(torch_gpu, n, precision, bar):
+    """Columns are taken in an order of K_ref's own; the bars of the other multi-RHS
+    products against the FP64 operator."""
+    p = problems.elasticity_hex20(n)
+    p = dataclasses.replace(p, k_ref=np.random.default_rng(9).normal(size=(60, 60)))
+    U = fields(p, "random", 4).astype(np.float32)
+    mr = MultiRHS([p.build_operator(aMatFree, Maps)], precision)
+    for scatter in (SCATTER.DETERMINISTIC, SCATTER.ATOMIC):
+        assert rel_l2(product(torch_gpu, mr, U, scatter), exact(p, U.astype(np.float64))) <= bar
