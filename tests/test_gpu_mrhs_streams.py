@@ -227,3 +227,38 @@ def test_atomic_operators_add_up_in_a_shared_output(torch_gpu, dims):
             mr.apply_dev(nrhs, U, [out, out], torch.cuda.current_stream())
         torch.cuda.synchronize()
         assert float(torch.linalg.norm(out - want) / torch.linalg.norm(want)) <= 2e-6
+
+
+@pytest.mark.parametrize("cols", [(5, 64, 200), (320, 400)])   # a stream's buffer, the shared one
+@pytest.mark.parametrize("scatter", [SCATTER.DETERMINISTIC, SCATTER.ATOMIC])
+def test_buffers_grow_beside_a_capture(torch_gpu, scatter, cols):
+    torch = torch_gpu
+    p, mr = make(13, scatter)
+    U = [rhs(torch, p, c, c) for c in cols]
+    want = [alone(torch, 13, u) for u in U]
+    V = [torch.full_like(u, float("nan")) for u in U]
+    x = torch.zeros(1000, device="cuda")
+    graph, st, other = torch.cuda.CUDAGraph(), torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    mr.apply_dev(cols[0], [U[0]], [V[0]], other)
+    errors = []
+
+    def work():
+        try:
+            for c, u, v in list(zip(cols, U, V))[1:]:
+                mr.apply_dev(c, [u], [v], other)
+        except Exception as e:
+            errors.append(e)
+    with torch.cuda.graph(graph, stream=st):
+        x.add_(1.0)
+        t = threading.Thread(target=work)
+        t.start()
+        t.join()
+        x.add_(1.0)
+    assert not errors
+    torch.cuda.synchronize()
+    for v, w in zip(V, want):
+        assert torch.equal(v, w)
+    graph.replay()
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(x.cpu().numpy(), np.full(1000, 2.0, np.float32))
